@@ -1,0 +1,93 @@
+// Device helpers shared by the matrix-core kernels: the three-term bf16 form of an fp32 value,
+// and the codec's Snake activation.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace q3t {
+
+typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+
+// x = hi + mid + lo, each bf16: hi = bf16(x) (round to nearest even, v_cvt_pk_bf16_f32 on two
+// lanes at a time); x - hi is exact in fp32 and holds the remaining 16 bits, split the same way
+// into mid and lo.  Not contracted: the residual is taken from the rounded x even where x is a
+// product computed just before (otherwise the compiler may fuse that product into x - hi).
+template <int N, typename V>
+__device__ __forceinline__ void split_bf16_nc(const float *x, V &hi, V &mid, V &lo) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int e = 0; e < N; e += 2) {
+    const f32x2_t v = {x[e], x[e + 1]};
+    const bf16x2_t h = __builtin_convertvector(v, bf16x2_t);
+    const f32x2_t r1 = v - __builtin_convertvector(h, f32x2_t);
+    const bf16x2_t m = __builtin_convertvector(r1, bf16x2_t);
+    const f32x2_t r2 = r1 - __builtin_convertvector(m, f32x2_t);
+    const bf16x2_t l = __builtin_convertvector(r2, bf16x2_t);
+    hi[e] = h[0]; hi[e + 1] = h[1];
+    mid[e] = m[0]; mid[e + 1] = m[1];
+    lo[e] = l[0]; lo[e + 1] = l[1];
+  }
+}
+__device__ __forceinline__ void split_bf16x8_nc(const float *x, bf16x8_t &hi, bf16x8_t &mid, bf16x8_t &lo) {
+  split_bf16_nc<8>(x, hi, mid, lo);
+}
+
+// Snake: v + sin(v ea)^2 ib, with the per-channel tables ea = exp(alpha), ib = 1 / (exp(beta) +
+// 1e-9) (codec_snake_beta_f32, kernels.rs:692-710).
+//
+// sin^2 has period pi, so y = v ea is reduced by n = rint(y / pi) to r = y - n pi in
+// [-pi/2, pi/2] (pi in two fp32 parts, each step one fma) and the sign of sin(r) does not
+// matter; sin(r) is an odd polynomial of degree 11 (least-squares minimax fit of the relative
+// error over |r| <= 1.62, 3.5e-11 before rounding).  Straight-line code of 14 operations: the
+// library's sinf takes data-dependent branches for its range reduction, which a matrix-core
+// kernel's prologue or epilogue cannot hide.  Against fp64 over N(0, 1) and N(0, 100) arguments
+// sin(r) is within 1.2e-7 absolute, 2e-8 rms (a correctly rounded sine: 6e-8, 1.5e-8).  The
+// reduction holds while n is an exact small integer; past kSnakeFast the caller takes snake_any.
+constexpr float kSnakeFast = 65536.0f;
+
+__device__ __forceinline__ float snake_fast(float v, float y, float ib) {
+  const float n = __builtin_rintf(y * 3.183098733e-01f);
+  float r = __builtin_fmaf(n, -3.141592741e+00f, y);
+  r = __builtin_fmaf(n, 8.742277657e-08f, r);
+  const float z = r * r;
+  float p = __builtin_fmaf(z, -2.381510633e-08f, 2.752115961e-06f);
+  p = __builtin_fmaf(z, p, -1.984078554e-04f);
+  p = __builtin_fmaf(z, p, 8.333330043e-03f);
+  p = __builtin_fmaf(z, p, -1.666666716e-01f);
+  const float s = __builtin_fmaf(r * z, p, r);
+  return __builtin_fmaf(s * s, ib, v);
+}
+
+__device__ __forceinline__ float snake_any(float v, float y, float ib) {
+  const float s = sinf(y);
+  return __builtin_fmaf(s * s, ib, v);
+}
+
+// Snake of N values in place (any magnitude): the library sine only where some |y| is past the
+// fast form's range (or not a number).
+template <int N>
+__device__ __forceinline__ void snake_n(float *v, const float *ea, const float *ib) {
+  float big = 0.f;
+  bool bad = false;
+  float x[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const float y = v[i] * ea[i];
+    big = fmaxf(big, fabsf(y));
+    x[i] = snake_fast(v[i], y, ib[i]);
+  }
+  bad = !(big < kSnakeFast);
+  if (__builtin_expect(bad, 0)) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) x[i] = snake_any(v[i], v[i] * ea[i], ib[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = x[i];
+}
+
+}  // namespace q3t

@@ -3,12 +3,16 @@
 //
 // Layout: activations are time-major [T][C] fp32.  Every convolution is one GEMM over
 // (overlapping) rows of its input:
-//   * a causal convolution with K taps and dilation d reads, for output row t, the K input rows
-//     t - (K-1)d, .., t as one GEMM row of K segments (GemmArgs::xseg_*), from a buffer that
-//     starts with zero rows; its weight [O][C][K] is stored as [O][K][C] to match;
+//   * a decoder convolution with 7 taps and dilation d is one launch_codec_conv, which applies the
+//     Snake before it (a residual unit's first) to the rows it stages and the Snake after it to
+//     the rows it stores;
 //   * a transposed convolution with stride s and kernel 2s (right-trimmed) computes output rows
-//     t*s + p from input rows t-1 and t: one GEMM row [x(t-1), x(t)] (2C wide) against s*O
-//     weight rows (phase p, channel o), so its output is directly time-major [s*T][O];
+//     t*s + p from input rows t-1 and t: a 2-tap launch_codec_conv against s*O columns (phase p,
+//     channel o), so its output is directly time-major [s*T][O];
+//   * a Snake whose input nothing else reads (before the transposed convolutions and the last
+//     convolution) is applied by the GEMM or convolution that produces that input;
+//   * the pre-conv's 3 taps are one GEMM over overlapping rows of a buffer that starts with zero
+//     rows, its weight [O][C][K] stored as [O][K][C];
 //   * pointwise convolutions and linears are plain GEMMs.
 // Weights are bf16 (the synthetic checkpoint's own values; an F32 checkpoint is rounded on
 // load); activations enter the matrix cores as three exact bf16 terms with fp32 accumulation.
@@ -56,16 +60,17 @@ struct Codec {
     float *dw_w, *dw_b, *ln_g, *ln_b, *pw1_b, *pw2_b, *gamma;
     uint16_t *pw1, *pw2;
   } up[2];
-  uint16_t *init_w = nullptr;  // [1536][7][1024]
+  uint16_t *init_w = nullptr;  // codec_conv_pack layout, as Block::tw and Unit::w1
   float *init_b = nullptr;
-  // Snake tables (a*: exp(alpha), b*: exp(beta) + 1e-9, per channel; launch_codec_snake).
+  // Snake tables (a*: exp(alpha), b*: 1 / (exp(beta) + 1e-9), per channel).
   struct Unit {
     float *a1a, *a1b, *a2a, *a2b, *b1, *b2;
-    uint16_t *w1, *w2;  // [co][7][co], [co][co]
+    uint16_t *w1;       // 7 taps co -> co
+    uint16_t *w2;       // [co][co], or as w1 with one tap where codec_unit_ok(co)
   };
   struct Block {
     float *snake_a, *snake_b;
-    uint16_t *tw;  // [s x co][previous ci | current ci]
+    uint16_t *tw;  // 2 taps (input rows t-1, t), ci -> s x co
     float *tb;     // [s x co]
     Unit u[3];
   } blocks[4];
@@ -104,7 +109,7 @@ Codec *codec_load(const std::string &model_dir, int64_t *device_bytes) {
     auto f32 = [&](const std::string &n, int64_t len) { return st.f32(n, {len}); };
     auto up_f32 = [&](const std::string &n, int64_t len) { return c->upload(f32(n, len)); };
     // A Snake's alpha / beta (prefix + "alpha" / "beta"), turned into the per-channel tables
-    // launch_codec_snake reads (exp(alpha), exp(beta) + 1e-9) on the device.
+    // Snakes read (exp(alpha), 1 / (exp(beta) + 1e-9)) on the device.
     auto up_snake = [&](const std::string &prefix, int64_t len, float *&a, float *&b) {
       a = up_f32(prefix + "alpha", len);
       b = up_f32(prefix + "beta", len);
@@ -208,8 +213,10 @@ Codec *codec_load(const std::string &model_dir, int64_t *device_bytes) {
     }
 
     // decoder (codec_hip.rs:802-1072, 1253-1394)
-    c->init_w = c->upload(taps_last_to_first(bf16("decoder.decoder.0.conv.weight", {kInit, kPreConv, 7}), kInit,
-                                             kPreConv, 7));
+    // [O][C][K] (the checkpoint's) -> matrix-core order
+    auto conv_at = [](int n, int ci, int j, int, int C, int taps) { return ((size_t)n * C + ci) * taps + j; };
+    c->init_w = c->upload(codec_conv_pack(bf16("decoder.decoder.0.conv.weight", {kInit, kPreConv, 7}), kInit, kPreConv,
+                                          7, conv_at));
     c->init_b = up_f32("decoder.decoder.0.conv.bias", kInit);
     for (int b = 0; b < 4; ++b) {
       const auto [ci, co, s] = kBlocks[b];
@@ -217,15 +224,16 @@ Codec *codec_load(const std::string &model_dir, int64_t *device_bytes) {
       Codec::Block &B = c->blocks[b];
       up_snake(p + ".0.", ci, B.snake_a, B.snake_b);
       const auto tw = bf16(p + ".1.conv.weight", {ci, co, 2 * s});  // [in][out][2s]
+      // column n = phase * co + o; tap 0 = input row t-1 (kernel index phase + s), tap 1 = row t
       std::vector<uint16_t> w((size_t)s * co * 2 * ci);
-      for (int ph = 0; ph < s; ++ph)
+      for (int k = 0; k < ci; ++k)
         for (int o = 0; o < co; ++o)
-          for (int k = 0; k < ci; ++k) {
-            uint16_t *row = &w[((size_t)ph * co + o) * 2 * ci];
-            row[k] = tw[((size_t)k * co + o) * 2 * s + ph + s];  // input row t-1
-            row[ci + k] = tw[((size_t)k * co + o) * 2 * s + ph];  // input row t
-          }
-      B.tw = c->upload(w);
+          for (int ph = 0; ph < s; ++ph)
+            for (int j = 0; j < 2; ++j)
+              w[(((size_t)ph * co + o) * 2 + j) * ci + k] = tw[((size_t)k * co + o) * 2 * s + ph + (j == 0 ? s : 0)];
+      B.tw = c->upload(codec_conv_pack(w, s * co, ci, 2, [](int n, int ch, int j, int, int C, int) {
+        return ((size_t)n * 2 + j) * C + ch;
+      }));
       const std::vector<float> b1 = f32(p + ".1.conv.bias", co);
       std::vector<float> tb;
       for (int ph = 0; ph < s; ++ph) tb.insert(tb.end(), b1.begin(), b1.end());
@@ -235,9 +243,10 @@ Codec *codec_load(const std::string &model_dir, int64_t *device_bytes) {
         Codec::Unit &Un = B.u[u];
         up_snake(r + ".act1.", co, Un.a1a, Un.a1b);
         up_snake(r + ".act2.", co, Un.a2a, Un.a2b);
-        Un.w1 = c->upload(taps_last_to_first(bf16(r + ".conv1.conv.weight", {co, co, 7}), co, co, 7));
+        Un.w1 = c->upload(codec_conv_pack(bf16(r + ".conv1.conv.weight", {co, co, 7}), co, co, 7, conv_at));
         Un.b1 = up_f32(r + ".conv1.conv.bias", co);
-        Un.w2 = c->upload(bf16(r + ".conv2.conv.weight", {co, co, 1}));
+        const auto w2 = bf16(r + ".conv2.conv.weight", {co, co, 1});
+        Un.w2 = c->upload(codec_unit_ok(co) ? codec_conv_pack(w2, co, co, 1, conv_at) : w2);
         Un.b2 = up_f32(r + ".conv2.conv.bias", co);
       }
     }
@@ -296,11 +305,10 @@ namespace {
 
 // Floats of the decode workspace for F frames (buffer list of codec_decode, in order).
 size_t workspace_floats(size_t F) {
-  const size_t pad_max = (size_t)kPad * kInit;
   const size_t big = (size_t)kCodecSamplesPerFrame * kFinal * F;  // largest T x C of the decoder blocks
   return 256 * 24 + F * 2 * kCodebookDim + (kPad + F) * kProjected + F * kPreConv + F * kHidden + F * 3 * kQ +
          F * kQ + F * kInter + F + F * kPreConv + 2 * ((kPad + 4 * F) * kUp) + 4 * F * kUp + 4 * F * kConvNext +
-         big + (pad_max + (size_t)640 * 192 * F) + (pad_max + big) + 2 * big;
+         (kPad * kFinal + big) + 2 * big;
 }
 
 }  // namespace
@@ -326,12 +334,10 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
   auto zero_pad = [&](float *buf, int C) { HIPC(hipMemsetAsync(buf, 0, (size_t)kPad * C * sizeof(float), s)); };
   auto gemm = [&](int epi, const float *X, int ldx, int M, const uint16_t *W, int N, int K, float *Y, int ldy,
                   const float *bias, const float *res = nullptr, int ldr = 0, const float *scale = nullptr,
-                  const float *row_scale = nullptr, const float *gamma = nullptr, int seg_len = 0,
-                  int seg_stride = 0) {
+                  const float *row_scale = nullptr, const float *gamma = nullptr) {
     GemmArgs g{};
     g.X = X; g.ldx = ldx; g.W = W; g.Y = Y; g.ldy = ldy; g.M = M; g.N = N; g.K = K;
     g.bias = bias; g.res = res; g.ldr = ldr; g.scale = scale; g.row_scale = row_scale; g.gamma = gamma;
-    g.xseg_len = seg_len; g.xseg_stride = seg_stride;
     g.split_ws = c.split_ws; g.split_cap = Codec::kSplitFloats;
     hip_check(launch_gemm(epi, g, s), "launch_gemm(codec)");
   };
@@ -385,7 +391,6 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
     hip_check(launch_codec_dwconv(Up + (size_t)(kPad - 6) * kUp, U.dw_w, U.dw_b, T, kUp, 7, D, s), "dwconv");
     hip_check(launch_codec_layernorm(D, U.ln_g, U.ln_b, T, kUp, kLnEps, D, s), "layernorm");
     gemm(EPI_BIAS_GELU, D, kUp, T, U.pw1, kConvNext, kUp, G, kConvNext, U.pw1_b);
-    zero_pad(Uo, kUp);
     float *O = Uo + (size_t)kPad * kUp;
     gemm(EPI_AFFINE_RES, G, kConvNext, T, U.pw2, kUp, kConvNext, O, kUp, U.pw2_b, Y, kUp, U.gamma);
     xin = O;
@@ -393,36 +398,47 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
 
   // 5. decoder: causal conv kernel 7, four blocks, Snake, last conv, clamp
   const size_t big = (size_t)kCodecSamplesPerFrame * kFinal * F;
-  float *R = take(big);
-  float *S = take((size_t)kPad * kInit + (size_t)640 * 192 * F);
-  float *A = take((size_t)kPad * kInit + big);
-  float *C1 = take(big);
-  float *A2 = take(big);
-  gemm(EPI_BIAS, Uo + (size_t)(kPad - 6) * kUp, kUp, T, c.init_w, kInit, 7 * kUp, R, kInit, c.init_b, nullptr, 0,
-       nullptr, nullptr, nullptr, kUp, kUp);
+  float *R = take(big), *A2 = take(big);
+  float *Sp = take((size_t)kPad * kFinal + big);  // starts with the zero rows the last conv reads
+  float *S = Sp + (size_t)kPad * kFinal;          // Snaked input of the next transposed (or last) convolution
+  auto conv = [&](int taps, const float *X, int rows, int C, int d, const float *sa, const float *sb, const uint16_t *W,
+                  const float *bias, const float *oa, const float *ob, float *Y, int N) {
+    const CodecConvArgs a{X, rows, C, d, sa, sb, W, bias, oa, ob, Y, N, c.split_ws, Codec::kSplitFloats,
+                          nullptr, nullptr, nullptr, nullptr};
+    hip_check(launch_codec_conv(taps, a, s), "launch_codec_conv");
+  };
+  // the initial convolution's output is only read through block 0's Snake
+  conv(7, xin, T, kUp, 1, nullptr, nullptr, c.init_w, c.init_b, c.blocks[0].snake_a, c.blocks[0].snake_b, S, kInit);
   for (int b = 0; b < 4; ++b) {
     const auto [ci, co, st] = kBlocks[b];
     const Codec::Block &B = c.blocks[b];
-    zero_pad(S, ci);
-    hip_check(launch_codec_snake(R, B.snake_a, B.snake_b, ci, (size_t)T * ci, S + (size_t)kPad * ci, s), "snake");
-    gemm(EPI_BIAS, S + (size_t)(kPad - 1) * ci, ci, T, B.tw, st * co, 2 * ci, R, st * co, B.tb, nullptr, 0, nullptr,
-         nullptr, nullptr, ci, ci);
+    conv(2, S, T, ci, 1, nullptr, nullptr, B.tw, B.tb, nullptr, nullptr, R, st * co);
     T *= st;
+    // a block's output is only read through the next block's (or the last convolution's) Snake
+    const float *na = b < 3 ? c.blocks[b + 1].snake_a : c.fin_a, *nb = b < 3 ? c.blocks[b + 1].snake_b : c.fin_b;
+    float *cur = R, *other = A2;
     for (int u = 0; u < 3; ++u) {
       const Codec::Unit &Un = B.u[u];
-      const int d = kDilations[u];
-      zero_pad(A, co);
-      hip_check(launch_codec_snake(R, Un.a1a, Un.a1b, co, (size_t)T * co, A + (size_t)kPad * co, s), "snake");
-      gemm(EPI_BIAS, A + (size_t)(kPad - 6 * d) * co, co, T, Un.w1, co, 7 * co, C1, co, Un.b1, nullptr, 0, nullptr,
-           nullptr, nullptr, co, d * co);
-      hip_check(launch_codec_snake(C1, Un.a2a, Un.a2b, co, (size_t)T * co, A2, s), "snake");
-      gemm(EPI_AFFINE_RES, A2, co, T, Un.w2, co, co, R, co, Un.b2, R, co, nullptr);
+      const bool end = u == 2;
+      if (codec_unit_ok(co)) {
+        float *out = end ? S : other;
+        const CodecConvArgs a{cur, T, co, kDilations[u], Un.a1a, Un.a1b, Un.w1, Un.b1, Un.a2a, Un.a2b, out, co,
+                              nullptr, 0, Un.w2, Un.b2, end ? na : nullptr, end ? nb : nullptr};
+        hip_check(launch_codec_conv(7, a, s), "launch_codec_conv(unit)");
+        std::swap(cur, other);
+        continue;
+      }
+      conv(7, R, T, co, kDilations[u], Un.a1a, Un.a1b, Un.w1, Un.b1, Un.a2a, Un.a2b, A2, co);
+      GemmArgs g{};
+      g.X = A2; g.ldx = co; g.W = Un.w2; g.Y = end ? S : R; g.ldy = co; g.M = T; g.N = co; g.K = co;
+      g.bias = Un.b2; g.res = R; g.ldr = co;
+      g.snake_a = na; g.snake_b = nb;
+      g.split_ws = c.split_ws; g.split_cap = Codec::kSplitFloats;
+      hip_check(launch_gemm(end ? EPI_RES_SNAKE : EPI_AFFINE_RES, g, s), "launch_gemm(1x1)");
     }
   }
-  zero_pad(A, kFinal);
-  hip_check(launch_codec_snake(R, c.fin_a, c.fin_b, kFinal, (size_t)T * kFinal, A + (size_t)kPad * kFinal, s), "snake");
-  hip_check(launch_codec_final(A + (size_t)(kPad - 6) * kFinal, c.fin_w, c.fin_bias, T, kFinal, 7, samples, s),
-            "codec_final");
+  HIPC(hipMemsetAsync(Sp, 0, (size_t)kPad * kFinal * sizeof(float), s));
+  hip_check(launch_codec_final(S - (size_t)6 * kFinal, c.fin_w, c.fin_bias, T, kFinal, 7, samples, s), "codec_final");
   HIPC(hipStreamSynchronize(s));
 }
 

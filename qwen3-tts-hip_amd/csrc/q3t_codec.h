@@ -3,6 +3,7 @@
 #pragma once
 
 #include <string>
+#include <vector>
 
 #include "q3t_device.h"
 
@@ -28,12 +29,37 @@ float *codec_samples_buffer(Codec &c, size_t n);
 // Kernels (q3t_codec.hip).
 hipError_t launch_codec_rvq(const int32_t *codes, int frames, int groups, const float *first, const float *rest,
                             int V, int D, float *E, hipStream_t s);
-// Snake over [n / C][C]: out = x + sin(x * ea[c])^2 / eb[c], with the per-channel tables
-// ea = exp(alpha), eb = exp(beta) + 1e-9 that launch_codec_snake_prep makes in place from the
-// checkpoint's alpha / beta (snake_beta_f32, kernels.rs).
-hipError_t launch_codec_snake(const float *x, const float *ea, const float *eb, int C, size_t n, float *out,
-                              hipStream_t s);
+// The Snake tables of a checkpoint's alpha / beta, in place: alpha := exp(alpha), beta := 1 /
+// (exp(beta) + 1e-9) (snake_beta_f32, kernels.rs).
 hipError_t launch_codec_snake_prep(float *alpha, float *beta, int C, hipStream_t s);
+
+// A causal convolution of `taps` taps (7, or 2 at d = 1: the transposed convolutions, whose
+// stride phases are columns) over time-major rows, with the Snakes around it (q3t_codec_conv.hip).
+// Kinds: 7 taps with an output Snake and with or without an input one; 2 taps with neither.
+struct CodecConvArgs {
+  const float *X;         // [T][C]; rows before 0 count as zeros
+  int32_t T, C, d;        // C a multiple of 32; d = dilation, at most 9
+  const float *sa, *sb;   // input Snake tables [C], or null
+  const uint16_t *W;      // codec_conv_pack layout
+  const float *bias;      // [N]
+  const float *oa, *ob;   // output Snake tables [N], or null
+  float *Y;               // [T][N], not X
+  int32_t N;              // a multiple of 96
+  float *split_ws;        // channel splits of short inputs: [split][T][N] raw sums, or null
+  int64_t split_cap;      // floats in split_ws
+  // A whole residual unit (7 taps, both Snakes, C = N, codec_unit_ok): the Snaked output goes on
+  // through a 1x1 convolution in the same launch, Y = S(X + (b2 + w2 . out)), S the Snake of
+  // ra / rb or, with null tables, the identity.
+  const uint16_t *w2;     // codec_conv_pack layout, one tap; null: no second half
+  const float *b2, *ra, *rb;
+};
+bool codec_unit_ok(int C);
+hipError_t launch_codec_conv(int taps, const CodecConvArgs &a, hipStream_t s);
+// Weights in matrix-core order, [N / 16][C / 32][taps][64 lanes][8]: lane i + 16 k of (tile, chunk,
+// tap) holds column 16 tile + i, channels 32 chunk + 8 k .. + 7.  at(n, c, j, N, C, taps) is the
+// source index of column n, channel c, tap j.
+std::vector<uint16_t> codec_conv_pack(const std::vector<uint16_t> &w, int N, int C, int taps,
+                                      size_t (*at)(int n, int c, int j, int N, int C, int taps));
 hipError_t launch_codec_dwconv(const float *xin, const float *w, const float *b, int T, int C, int K, float *out,
                                hipStream_t s);
 hipError_t launch_codec_layernorm(const float *x, const float *g, const float *b, int T, int C, float eps, float *out,

@@ -58,6 +58,7 @@ enum Epilogue : int32_t {
   // matrix-core GEMMs only (the codec decoder):
   EPI_AFFINE_RES = 4,  // out[n] = res[n] + (acc + bias[n]) * scale[n] (bias, scale optional)
   EPI_BIAS_GELU = 5,   // out[n] = gelu(acc + bias[n]), erf form
+  EPI_RES_SNAKE = 6,   // out[n] = snake(res[n] + (acc + bias[n])), tables snake_a / snake_b
 };
 
 // Greedy token hand-off into a CodePredictor group (one stream): the group's input token is
@@ -202,6 +203,7 @@ struct GemmArgs {
   const float *res;        // EPI_RESIDUAL: [M][ldr]
   const float *bias;       // EPI_BIAS: [N]
   const float *scale;      // EPI_AFFINE_RES: [N] or null
+  const float *snake_a, *snake_b;  // EPI_RES_SNAKE: [N] exp(alpha), 1 / (exp(beta) + 1e-9)
   int32_t M, N, K, ldx, ldy, ldr;
   // Segmented X rows (matrix-core GEMMs; a dilated convolution's taps): with xseg_len > 0,
   // element k of row m is X[m * ldx + (k / xseg_len) * xseg_stride + k % xseg_len].

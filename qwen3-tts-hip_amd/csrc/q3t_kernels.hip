@@ -5,6 +5,8 @@
 // fixed cross-wave order), so results are bit-reproducible run to run.
 #include "q3t_kernels.h"
 
+#include "q3t_bf16x3.h"
+
 #include <float.h>
 #include <math.h>
 
@@ -1389,35 +1391,11 @@ __global__ __launch_bounds__(128) void k_attn_merge(AttnMergeArgs a) {
 // B[k][j] in lane j + 16 (k / 8), element k % 8; C[i][j] in lane j + 16 (i / 4), element i % 4.
 // SwiGLU: the first NB/2 column tiles are gate rows, the last NB/2 the matching up rows.
 // ---------------------------------------------------------------------------------------
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-typedef float f32x2_t __attribute__((ext_vector_type(2)));
-
 // x = hi + mid + lo, each a bf16: 24 significant bits, so every product with a bf16 weight
 // is exact and the GEMM matches an fp32 GEMV up to the order of the fp32 additions.
 // hi = bf16(x) (round to nearest even, v_cvt_pk_bf16_f32 on two lanes at a time); x - hi is
 // exact in fp32 and holds the remaining 16 bits, split the same way into mid and lo.
 __device__ __forceinline__ void split_bf16x8(const float *x, bf16x8_t &hi, bf16x8_t &mid, bf16x8_t &lo) {
-#pragma unroll
-  for (int e = 0; e < 8; e += 2) {
-    const f32x2_t v = {x[e], x[e + 1]};
-    const bf16x2_t h = __builtin_convertvector(v, bf16x2_t);
-    const f32x2_t r1 = v - __builtin_convertvector(h, f32x2_t);
-    const bf16x2_t m = __builtin_convertvector(r1, bf16x2_t);
-    const f32x2_t r2 = r1 - __builtin_convertvector(m, f32x2_t);
-    const bf16x2_t l = __builtin_convertvector(r2, bf16x2_t);
-    hi[e] = h[0]; hi[e + 1] = h[1];
-    mid[e] = m[0]; mid[e + 1] = m[1];
-    lo[e] = l[0]; lo[e + 1] = l[1];
-  }
-}
-
-// split_bf16x8 without contraction: the residual is taken from the rounded x even where x is
-// a product computed just before (otherwise the compiler may fuse that product into x - hi).
-__device__ __forceinline__ void split_bf16x8_nc(const float *x, bf16x8_t &hi, bf16x8_t &mid, bf16x8_t &lo) {
-#pragma clang fp contract(off)
 #pragma unroll
   for (int e = 0; e < 8; e += 2) {
     const f32x2_t v = {x[e], x[e + 1]};
@@ -1455,13 +1433,19 @@ __device__ __forceinline__ float gemm_epilogue(const GemmArgs &a, int m, int n, 
     v = v + a.bias[n];
     v = 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
   }
+  if constexpr (EPI == EPI_RES_SNAKE) {
+    v = a.res[(size_t)m * a.ldr + n] + (v + a.bias[n]);
+    const float ea = a.snake_a[n], ib = a.snake_b[n];
+    snake_n<1>(&v, &ea, &ib);
+  }
   return v;
 }
 
 // gemm_epilogue with its operands loaded beforehand: r = res[m][n], b = bias[n] (when
-// given), c = scale[n] (when given); the same arithmetic in the same order.
+// given), c = scale[n] (when given; the Snake form: c = snake_a[n], c2 = snake_b[n]); the same
+// arithmetic in the same order.
 template <int EPI>
-__device__ __forceinline__ float gemm_epilogue_ops(const GemmArgs &a, float v, float r, float b, float c) {
+__device__ __forceinline__ float gemm_epilogue_ops(const GemmArgs &a, float v, float r, float b, float c, float c2) {
   if constexpr (EPI == EPI_RESIDUAL) v = r + v;
   if constexpr (EPI == EPI_BIAS) v = v + b;
   if constexpr (EPI == EPI_AFFINE_RES) {
@@ -1472,6 +1456,10 @@ __device__ __forceinline__ float gemm_epilogue_ops(const GemmArgs &a, float v, f
   if constexpr (EPI == EPI_BIAS_GELU) {
     v = v + b;
     v = 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
+  }
+  if constexpr (EPI == EPI_RES_SNAKE) {
+    v = r + (v + b);
+    snake_n<1>(&v, &c, &c2);
   }
   return v;
 }
@@ -1569,17 +1557,18 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(GemmArgs a) {
   // epilogue: lane holds C[4 * kb + e][li] of every tile
   // The epilogue's operands are loaded before the first store (Y may be the residual itself:
   // a load after a store that may alias it would wait for that store).
-  constexpr bool RES = EPI == EPI_RESIDUAL || EPI == EPI_AFFINE_RES;
-  constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU;
+  constexpr bool RES = EPI == EPI_RESIDUAL || EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE;
+  constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU || EPI == EPI_RES_SNAKE;
   constexpr bool OPS = RES || BIAS;
-  float rv[OPS ? MB : 1][OPS ? NTILE : 1][4], bv[OPS ? NTILE : 1], cv[OPS ? NTILE : 1];
+  float rv[OPS ? MB : 1][OPS ? NTILE : 1][4], bv[OPS ? NTILE : 1], cv[OPS ? NTILE : 1], c2v[OPS ? NTILE : 1];
   if constexpr (OPS) {
     if (nsplit == 1) {
 #pragma unroll
       for (int j = 0; j < NTILE; ++j) {
         const int nc = min(n0 + 16 * j + li, a.N - 1);
         bv[j] = (BIAS && (EPI != EPI_AFFINE_RES || a.bias)) ? a.bias[nc] : 0.f;
-        cv[j] = (EPI == EPI_AFFINE_RES && a.scale) ? a.scale[nc] : 1.f;
+        cv[j] = (EPI == EPI_AFFINE_RES && a.scale) ? a.scale[nc] : (EPI == EPI_RES_SNAKE ? a.snake_a[nc] : 1.f);
+        c2v[j] = EPI == EPI_RES_SNAKE ? a.snake_b[nc] : 1.f;
 #pragma unroll
         for (int i = 0; i < MB; ++i)
 #pragma unroll
@@ -1612,7 +1601,7 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(GemmArgs a) {
             a.split_ws[((size_t)z * a.M + m) * a.N + n] = v;
             continue;
           }
-          if constexpr (OPS) v = gemm_epilogue_ops<EPI>(a, v, rv[i][j][e], bv[j], cv[j]);
+          if constexpr (OPS) v = gemm_epilogue_ops<EPI>(a, v, rv[i][j][e], bv[j], cv[j], c2v[j]);
         }
         a.Y[(size_t)m * a.ldy + n] = v;
       }
@@ -1831,14 +1820,19 @@ __global__ __launch_bounds__(256, 2) void k_gemm_lds(GemmArgs a) {
     // Every epilogue operand is loaded before the first store: Y may be the residual itself
     // (each element read and written by this lane only), and a load after a store that may
     // alias it would wait for that store, one memory round trip per element.
-    constexpr bool RES = EPI == EPI_RESIDUAL || EPI == EPI_AFFINE_RES;
-    constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU;
-    float rv[2][4][RES ? NU : 1], bv[BIAS ? NU : 1], cv[EPI == EPI_AFFINE_RES ? NU : 1];
+    constexpr bool RES = EPI == EPI_RESIDUAL || EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE;
+    constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU || EPI == EPI_RES_SNAKE;
+    constexpr bool SCALE = EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE;
+    float rv[2][4][RES ? NU : 1], bv[BIAS ? NU : 1], cv[SCALE ? NU : 1], c2v[EPI == EPI_RES_SNAKE ? NU : 1];
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       const int nc = min(nb * BW + u * 16 + li, a.N - 1);
       if constexpr (BIAS) bv[u] = (EPI != EPI_AFFINE_RES || a.bias) ? a.bias[nc] : 0.f;
       if constexpr (EPI == EPI_AFFINE_RES) cv[u] = a.scale ? a.scale[nc] : 1.f;
+      if constexpr (EPI == EPI_RES_SNAKE) {
+        cv[u] = a.snake_a[nc];
+        c2v[u] = a.snake_b[nc];
+      }
     }
     if constexpr (RES) {
 #pragma unroll
@@ -1857,13 +1851,26 @@ __global__ __launch_bounds__(256, 2) void k_gemm_lds(GemmArgs a) {
       for (int e = 0; e < 4; ++e) {
         const int m = m0 + t * 16 + 4 * kb + e;
         if (m >= a.M) continue;
+        if constexpr (EPI == EPI_RES_SNAKE) {  // one row's column tiles through the Snake together
+          float v[NU];
+#pragma unroll
+          for (int u = 0; u < NU; ++u) v[u] = rv[t][e][u] + (acc[t][u][e] + bv[u]);
+          snake_n<NU>(v, cv, c2v);
+#pragma unroll
+          for (int u = 0; u < NU; ++u) {
+            const int n = nb * BW + u * 16 + li;
+            if (n < a.N) a.Y[(size_t)m * a.ldy + n] = v[u];
+          }
+          continue;
+        }
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
           const int n = nb * BW + u * 16 + li;
           if (n >= a.N) continue;
           a.Y[(size_t)m * a.ldy + n] = gemm_epilogue_ops<EPI>(a, acc[t][u][e], RES ? rv[t][e][RES ? u : 0] : 0.f,
                                                               BIAS ? bv[BIAS ? u : 0] : 0.f,
-                                                              EPI == EPI_AFFINE_RES ? cv[EPI == EPI_AFFINE_RES ? u : 0] : 1.f);
+                                                              SCALE ? cv[SCALE ? u : 0] : 1.f,
+                                                              EPI == EPI_RES_SNAKE ? c2v[EPI == EPI_RES_SNAKE ? u : 0] : 1.f);
         }
       }
   }
@@ -3569,6 +3576,8 @@ hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
     case EPI_SWIGLU: return gemm_epi<EPI_SWIGLU>(a, s);
     case EPI_BIAS: return gemm_epi<EPI_BIAS>(a, s);
     case EPI_AFFINE_RES: return a.res ? gemm_epi<EPI_AFFINE_RES>(a, s) : hipErrorInvalidValue;
+    case EPI_RES_SNAKE:
+      return a.res && a.bias && a.snake_a && a.snake_b ? gemm_epi<EPI_RES_SNAKE>(a, s) : hipErrorInvalidValue;
     case EPI_BIAS_GELU: return a.bias ? gemm_epi<EPI_BIAS_GELU>(a, s) : hipErrorInvalidValue;
   }
   return hipErrorInvalidValue;

@@ -39,6 +39,46 @@ def test_decode_matches_oracle(codec_case, frames):
     assert err <= WAVE_TOL
 
 
+@pytest.mark.parametrize("frames", [1, 2, 5])
+def test_decode_at_block_edges(codec_case, frames):
+    """The decoder convolutions' 64-row blocks at half, exactly one and a remainder of a block
+    (32 rows a frame after the first transposed convolution), split over channels, with rows
+    before time 0 in every block.  ~45 layers of fp32 sums of exact products end within 3.4e-6 of
+    float64 (2-norm) on inputs of 6 to 240 frames; four times that is allowed."""
+    eng, oracle = codec_case
+    codes = np.random.default_rng(100 + frames).integers(0, 2048, (frames, 16)).astype(np.int32)
+    print(f"[gpu] decode_codes frames={frames}", flush=True)
+    got, ref = eng.decode_codes(codes), oracle.decode(codes)
+    err = float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+    print(f"decode {frames} frames: rel err {err:.2e}")
+    assert err <= 1.4e-5
+
+
+def test_snake_of_large_arguments(models, tmp_path):
+    """Snakes whose arguments pass the fast sine's range (alpha = e^12: |x e^12| above 65536)
+    in input, output and residual position, beside ones that do not: finite and near float64.
+    The argument's own fp32 rounding, |y| 2^-24 ~ 0.02 at |y| = 3e5, passes at most 2 e^-beta = 2 e^-7
+    of itself on, 4e-5 a Snake."""
+    tensors = dict(synth.codec_tensors(0))
+    for name in ("decoder.decoder.1.block.2.act1", "decoder.decoder.3.block.3.act1", "decoder.decoder.3.block.3.act2",
+                 "decoder.decoder.4.block.4.act1", "decoder.decoder.4.block.0", "decoder.decoder.5"):
+        for part, value in (("alpha", 12.0), ("beta", 7.0)):
+            t = tensors[f"{name}.{part}"].copy()
+            t[::3] = synth.f32_to_bf16_bits(np.float32([value]))[0]
+            tensors[f"{name}.{part}"] = t
+    model, _ = models.get("tiny")
+    model.write(str(tmp_path))
+    synth.write_codec(str(tmp_path), 0, tensors)
+    codes = np.random.default_rng(9).integers(0, 2048, (3, 16)).astype(np.int32)
+    with E.HipTtsEngine(str(tmp_path), E.EngineOptions(max_cache_steps=64)) as eng:
+        got = eng.decode_codes(codes)
+    ref = C.CodecOracle(tensors).decode(codes)
+    assert np.isfinite(got).all()
+    err = float(np.abs(got - ref).max())
+    print(f"large Snake arguments: max err {err:.2e}")
+    assert err <= WAVE_TOL
+
+
 def test_decode_is_causal_and_wraps_codes(codec_case):
     eng, _ = codec_case
     codes = np.random.default_rng(7).integers(0, 2048, (8, 16)).astype(np.int32)
