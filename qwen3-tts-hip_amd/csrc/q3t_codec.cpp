@@ -364,8 +364,7 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
     const Codec::Layer &L = c.layers[i];
     hip_check(launch_row_rms(H, kHidden, F, kHidden, kRmsEps, INV, s), "row_rms");
     gemm(EPI_STORE, H, kHidden, F, L.qkv, 3 * kQ, kHidden, QKV, 3 * kQ, nullptr, nullptr, 0, nullptr, INV, L.g_in);
-    hip_check(launch_codec_rope(QKV, F, 3 * kQ, kHeads, c.rope, s), "codec_rope");
-    hip_check(launch_codec_attention(QKV, F, 3 * kQ, kHeads, 0.125f, ATT, kQ, s), "codec_attention");
+    hip_check(launch_codec_attention(QKV, F, 3 * kQ, kHeads, c.rope, 0.125f, ATT, kQ, s), "codec_attention");
     gemm(EPI_AFFINE_RES, ATT, kQ, F, L.o, kHidden, kQ, H, kHidden, nullptr, H, kHidden, L.attn_scale);
     hip_check(launch_row_rms(H, kHidden, F, kHidden, kRmsEps, INV, s), "row_rms");
     gemm(EPI_SWIGLU, H, kHidden, F, L.gu, kInter, kHidden, ACT, kInter, nullptr, nullptr, 0, nullptr, INV, L.g_post);

@@ -64,9 +64,9 @@ hipError_t launch_codec_dwconv(const float *xin, const float *w, const float *b,
                                hipStream_t s);
 hipError_t launch_codec_layernorm(const float *x, const float *g, const float *b, int T, int C, float eps, float *out,
                                   hipStream_t s);
-hipError_t launch_codec_rope(float *qkv, int T, int ld, int heads, const float2 *table, hipStream_t s);
-hipError_t launch_codec_attention(const float *qkv, int T, int ld, int heads, float scale, float *out, int ldo,
-                                  hipStream_t s);
+// Causal attention with RoPE over raw qkv rows (64 dims a head; table [T][32] (cos, sin)).
+hipError_t launch_codec_attention(const float *qkv, int T, int ld, int heads, const float2 *table, float scale,
+                                  float *out, int ldo, hipStream_t s);
 hipError_t launch_codec_final(const float *xin, const float *w, const float *b, int T, int C, int K, float *out,
                               hipStream_t s);
 

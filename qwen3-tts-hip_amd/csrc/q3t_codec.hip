@@ -1,8 +1,9 @@
 // gfx950 kernels of the codec decoder (codec frames -> 24 kHz audio) besides its matrix-core
-// GEMMs (launch_gemm): RVQ gather, Snake, depthwise causal conv, LayerNorm, RoPE, causal
-// attention, and the last convolution.  Activations are time-major [T][C] fp32; a "padded"
+// GEMMs (launch_gemm) and convolutions: RVQ gather, depthwise causal conv, LayerNorm, causal
+// attention with RoPE, and the last convolution.  Activations are time-major [T][C] fp32; a "padded"
 // buffer starts with zero rows so that causal convolutions read rows before time 0 as zeros.
 #include "q3t_codec.h"
+#include "q3t_bf16x3.h"
 
 #include <float.h>
 #include <math.h>
@@ -77,77 +78,125 @@ __global__ void k_codec_layernorm(const float *x, const float *g, const float *b
   for (int c = threadIdx.x; c < C; c += 256) o[c] = (r[c] - mean) * inv * g[c] + b[c];
 }
 
-// Rotate-half RoPE in place on the q and k heads of each row of qkv ([T][ld]: q heads, then k
-// heads, 64 dims each), position = row (rope_bhsd_f32, kernels.rs:40-77); cos/sin table [T][32].
-__global__ void k_codec_rope(float *qkv, int T, int ld, int heads, const float2 *table) {
-  const int t = blockIdx.x;
-  const int h = blockIdx.y;  // 0 .. 2 * heads - 1: q heads then k heads
-  const int i = threadIdx.x;  // pair 0 .. 31
-  float *v = qkv + (size_t)t * ld + h * 64;
-  const float2 cs = table[(size_t)t * 32 + i];
-  const float a = v[i], b = v[i + 32];
-  v[i] = a * cs.x - b * cs.y;
-  v[i + 32] = b * cs.x + a * cs.y;
-}
+// Causal attention over rows 0..t for query row t and head h: rotate-half RoPE on q and k
+// (position = row, cos/sin table [T][32]; rope_bhsd_f32, kernels.rs:40-77), scores scaled by
+// `scale`, softmax, weighted sum of V (attention_scores_causal_f32 + masked softmax + apply_value,
+// kernels.rs:980-1040).  qkv rows: [q heads | k heads | v heads] x 64 dims, not rotated.
+//
+// One workgroup per (head, 16 query rows), longest first, on v_mfma_f32_16x16x4_f32 (fp32 products
+// and sums); its four waves take every fourth 16-key tile with an online softmax each, the next
+// tile in flight, and merge through LDS in wave order (k_attn_prefill's scheme at 64 dims).  Lane
+// (li, kk) holds dims 8 kk .. + 7 and 32 + 8 kk .. + 7 of key and query row li, the two halves of
+// 8 rotation pairs, so RoPE needs no exchange and no pass of its own; scores of keys 4 kk + e for
+// query li; and dims 16 kk .. + 15 of the output of query li (value rows are read 4 dims a lane).
+// Bound: the latency of a tile's chain, T / 64 tiles a wave.  One workgroup per query row on the
+// vector units, with a RoPE launch before it, took 69 + 4 us at T = 240.
+__global__ __launch_bounds__(256, 2) void k_codec_attention(const float *qkv, int T, int ld, int heads,
+                                                            const float2 *table, float scale, float *out, int ldo) {
+  constexpr int W = 4;
+  __shared__ float mo[W][16][64];
+  __shared__ float mm[W][16], ml[W][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kk = lane >> 4;
+  const int h = blockIdx.x, q0 = 16 * ((int)gridDim.y - 1 - (int)blockIdx.y), Q = heads * 64;
+  const int nkt = (min(q0 + 16, T) + 15) / 16;
 
-// Causal attention over rows 0..t for query row t and head h: scores scaled by `scale`,
-// softmax, weighted sum of V (attention_scores_causal_f32 + masked softmax + apply_value,
-// kernels.rs:980-1040).  qkv rows: [q heads | k heads | v heads] x 64 dims.  The four waves
-// score interleaved batches of 8 keys (each score one wave sum, the same in every lane and
-// whichever wave computes it); wave 0 then forms the probabilities with the scores' maximum
-// and sums V in key order.
-__global__ __launch_bounds__(256) void k_codec_attention(const float *qkv, int T, int ld, int heads, float scale,
-                                                         float *out, int ldo) {
-  extern __shared__ float sc[];  // [T]
-  __shared__ float mw[4];
-  const int h = blockIdx.x, t = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int Q = heads * 64;
-  const float q = qkv[(size_t)t * ld + h * 64 + lane];
-  float m = -FLT_MAX;
-  // Key rows in batches of 8, every load of a batch issued before its reductions.
-  constexpr int KB = 8;
-  for (int u0 = wave * KB; u0 <= t; u0 += 4 * KB) {
-    float kv[KB];
+  struct Rows {  // a row's 16 dims, their 8 rotations, and (keys) 4 value rows of 4 dims
+    f32x4_t x[4], cs[4], v[4];
+  };
+  auto load_row = [&](int r, int col, Rows &o) {
+    const f32x4_t *p = reinterpret_cast<const f32x4_t *>(qkv + (size_t)r * ld + col + 8 * kk);
+    o.x[0] = p[0]; o.x[1] = p[1]; o.x[2] = p[8]; o.x[3] = p[9];
+    const f32x4_t *c = reinterpret_cast<const f32x4_t *>(table + (size_t)r * 32 + 8 * kk);
 #pragma unroll
-    for (int j = 0; j < KB; ++j) kv[j] = qkv[(size_t)min(u0 + j, t) * ld + Q + h * 64 + lane];
+    for (int i = 0; i < 4; ++i) o.cs[i] = c[i];
+  };
+  auto rotate = [](const Rows &o, float *y) {  // y[i], y[8 + i]: pair i
 #pragma unroll
-    for (int j = 0; j < KB; ++j) {
-      // A rounded product, not contracted into the butterfly's first add (which would add
-      // each lane's own exact product to its partner's rounded one): every lane then holds
-      // the same score.
-#pragma clang fp contract(off)
-      if (u0 + j > t) break;
-      const float s = wave_sum64(q * kv[j]) * scale;
-      if (lane == 0) sc[u0 + j] = s;
-      m = fmaxf(m, s);
+    for (int i = 0; i < 8; ++i) {
+      const float p = o.x[i >> 2][i & 3], q = o.x[2 + (i >> 2)][i & 3];
+      const float cos = o.cs[i >> 1][2 * (i & 1)], sin = o.cs[i >> 1][2 * (i & 1) + 1];
+      y[i] = p * cos - q * sin;
+      y[8 + i] = q * cos + p * sin;
     }
+  };
+  auto load_tile = [&](int kt, Rows &o) {
+    load_row(min(16 * kt + li, T - 1), Q + h * 64, o);
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+      o.v[s] = *reinterpret_cast<const f32x4_t *>(qkv + (size_t)min(16 * kt + 4 * kk + s, T - 1) * ld + 2 * Q + h * 64 +
+                                                  4 * li);
+  };
+  Rows cur, nxt;
+  if (wave < nkt) load_tile(wave, cur);
+  float q[16];
+  {
+    Rows r;
+    load_row(min(q0 + li, T - 1), h * 64, r);
+    rotate(r, q);
   }
-  if (lane == 0) mw[wave] = m;
+  f32x4_t o[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  float m_run = -FLT_MAX, l = 0.f;
+  const int qrow = q0 + li;
+  for (int kt = wave; kt < nkt; kt += W) {
+    if (kt + W < nkt) load_tile(kt + W, nxt);
+    float k[16];
+    rotate(cur, k);
+    f32x4_t st = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 16; ++s) st = __builtin_amdgcn_mfma_f32_16x16x4f32(k[s], q[s], st, 0, 0, 0);
+    float p[4], mt = -FLT_MAX;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      p[e] = 16 * kt + 4 * kk + e <= qrow ? st[e] * scale : -FLT_MAX;
+      mt = fmaxf(mt, p[e]);
+    }
+    mt = fmaxf(mt, __shfl_xor(mt, 16, 64));
+    mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
+    const float m_new = fmaxf(m_run, mt), corr = expf(m_run - m_new);
+    float ps = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      p[e] = p[e] == -FLT_MAX ? 0.f : expf(p[e] - m_new);
+      ps += p[e];
+    }
+    l = l * corr + ps;
+    m_run = m_new;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) o[t] *= corr;
+#pragma unroll
+    for (int s = 0; s < 4; ++s)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(cur.v[s][t], p[s], o[t], 0, 0, 0);
+    cur = nxt;
+  }
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (kk == 0) {
+    mm[wave][li] = m_run;
+    ml[wave][li] = l;
+  }
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mo[wave][4 * e + t][lane] = o[t][e];
   __syncthreads();
-  m = fmaxf(fmaxf(mw[0], mw[1]), fmaxf(mw[2], mw[3]));
-  float l = 0.f;
-  if (wave == 0) {
-    for (int u = lane; u <= t; u += 64) {
-      const float p = expf(sc[u] - m);
-      sc[u] = p;
-      l += p;
-    }
-    l = wave_sum64(l);
-  }
-  __syncthreads();
-  if (wave != 0) return;
-  float acc = 0.f;
-  for (int u0 = 0; u0 <= t; u0 += KB) {
-    float vv[KB];
+  if (qrow >= T) return;
+  float m = mm[0][li];
 #pragma unroll
-    for (int j = 0; j < KB; ++j) vv[j] = qkv[(size_t)min(u0 + j, t) * ld + 2 * Q + h * 64 + lane];
+  for (int w = 1; w < W; ++w) m = fmaxf(m, mm[w][li]);
+  float lsum = 0.f, r[4] = {};
 #pragma unroll
-    for (int j = 0; j < KB; ++j) {
-      if (u0 + j > t) break;
-      acc = fmaf(sc[u0 + j], vv[j], acc);
-    }
+  for (int w = 0; w < W; ++w) {  // a wave without a tile has m = -FLT_MAX, l = 0: weight 0
+    const float f = expf(mm[w][li] - m);
+    lsum += ml[w][li] * f;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) r[t] += mo[w][4 * wave + t][lane] * f;
   }
-  out[(size_t)t * ldo + h * 64 + lane] = acc / l;
+  const float inv = 1.0f / lsum;
+  *reinterpret_cast<float4 *>(out + (size_t)qrow * ldo + h * 64 + 16 * kk + 4 * wave) =
+      make_float4(r[0] * inv, r[1] * inv, r[2] * inv, r[3] * inv);
 }
 
 // Last convolution to one channel + clamp to [-1, 1]: out[t] = clamp(b + sum_{j, c}
@@ -248,18 +297,12 @@ hipError_t launch_codec_layernorm(const float *x, const float *g, const float *b
   return hipGetLastError();
 }
 
-hipError_t launch_codec_rope(float *qkv, int T, int ld, int heads, const float2 *table, hipStream_t s) {
-  if (T <= 0 || heads <= 0 || ld < 2 * heads * 64) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_codec_rope, dim3(T, 2 * heads), dim3(32), 0, s, qkv, T, ld, heads, table);
-  return hipGetLastError();
-}
-
-hipError_t launch_codec_attention(const float *qkv, int T, int ld, int heads, float scale, float *out, int ldo,
-                                  hipStream_t s) {
-  if (T <= 0 || T > kCodecMaxAttnRows || heads <= 0 || ld < 3 * heads * 64 || ldo < heads * 64)
+hipError_t launch_codec_attention(const float *qkv, int T, int ld, int heads, const float2 *table, float scale,
+                                  float *out, int ldo, hipStream_t s) {
+  if (T <= 0 || T > kCodecMaxAttnRows || heads <= 0 || ld < 3 * heads * 64 || ld % 4 || ldo < heads * 64 || ldo % 4)
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_codec_attention, dim3(heads, T), dim3(256), (size_t)T * sizeof(float), s, qkv, T, ld, heads,
-                     scale, out, ldo);
+  hipLaunchKernelGGL(k_codec_attention, dim3(heads, (T + 15) / 16), dim3(256), 0, s, qkv, T, ld, heads, table, scale,
+                     out, ldo);
   return hipGetLastError();
 }
 

@@ -2082,7 +2082,7 @@ __global__ __launch_bounds__(256) void k_row_rms(const float *X, int ldx, int M,
 //     (q written back in place), K and V stored into the row's stream cache.  One wave per
 //     vector.
 //   k_attn_prefill: per (stream, query head, 16-row query block): causal attention over
-//     the stream's cache rows on the fp32 matrix cores, one wave per unit.
+//     the stream's cache rows on the fp32 matrix cores, one workgroup per unit.
 // ---------------------------------------------------------------------------------------
 __device__ __forceinline__ int prefill_segment(const PrefillBatchArgs &a, int row) {
   int s = 0;
@@ -2266,23 +2266,50 @@ __global__ __launch_bounds__(256) void k_attn_prefix(PrefillAttnArgs a) {
   }
 }
 
-// One wave per unit (stream s, query head hq, query rows q0 .. q0 + 15), units in
+// 8 consecutive cache elements as loaded, converted where they are used: a load can be in flight
+// across other work.
+template <typename KVT>
+struct KvRaw8;
+template <>
+struct KvRaw8<float> {
+  f32x4_t a, b;
+  __device__ __forceinline__ void load(const float *p) {
+    a = reinterpret_cast<const f32x4_t *>(p)[0];
+    b = reinterpret_cast<const f32x4_t *>(p)[1];
+  }
+  __device__ __forceinline__ float operator[](int i) const { return i < 4 ? a[i] : b[i - 4]; }
+};
+template <>
+struct KvRaw8<uint16_t> {
+  u32x4 w;
+  __device__ __forceinline__ void load(const uint16_t *p) { w = *reinterpret_cast<const u32x4 *>(p); }
+  __device__ __forceinline__ float operator[](int i) const { return (i & 1) ? bf_hi(w[i >> 1]) : bf_lo(w[i >> 1]); }
+};
+
+// One workgroup per unit (stream s, query head hq, query rows q0 .. q0 + 15), units in
 // PrefillBatchArgs::unit0 order: per stream, the last query block first (the longest causal
-// range).  v_mfma_f32_16x16x4_f32 (fp32 products and sums):
+// range).  The four waves take every fourth 16-key tile and merge at the end: a unit is a serial
+// chain of tiles (load, 32 dependent matrix-core steps, softmax, 32 more), and a prompt has few
+// units against 1,024 SIMDs, so the longest chain sets the time (521 rows, 16 heads, bf16 cache:
+// 79 us as one wave per unit, ~25 us so).  Each wave's next tile is in flight while it works on
+// this one.  v_mfma_f32_16x16x4_f32 (fp32 products and sums):
 //   S^T = K Q^T per 16-key tile: lane (li, kk) supplies key row li and query row li, dims
 //     32 kk + s at step s (32 steps: the four lane groups cover the 128 dims in quarters), and
 //     holds scores of keys 4 kk + e (e = 0..3) for query li.
 //   O^T += V^T P^T: step s' takes keys 4 kk + s' (lane group kk), so each lane's own score
 //     e = s' is its B operand; A row i of output tile t is dim 8 i + t, so a lane reads 8
-//     consecutive floats of a value row and ends up holding dims 32 kk .. 32 kk + 31 of query li.
-//   Online softmax per query over 16-key tiles: the tile max over the four lane groups by lane
+//     consecutive elements of a value row and ends up holding dims 32 kk .. 32 kk + 31 of query li.
+//   Online softmax per query over the wave's tiles: the tile max over the four lane groups by lane
 //     exchanges, per-lane partial sums of p (added across the groups at the end).
+//   Merge: (m, l, O) of the four waves through LDS in wave order; wave w stores dims
+//     32 kk + 8 w .. + 7 of each query.
 template <typename KVT>
-__global__ __launch_bounds__(256) void k_attn_prefill(PrefillBatchArgs a) {
-  constexpr int D = 128;
-  const int lane = threadIdx.x & 63, li = lane & 15, kk = lane >> 4;
-  const int u = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (u >= a.unit0[a.nseg]) return;
+__global__ __launch_bounds__(256, 2) void k_attn_prefill(PrefillBatchArgs a) {
+  constexpr int D = 128, W = 4;
+  __shared__ float mo[W][32][64];  // [wave][8 e' + t]: element (tile t, e') of each lane
+  __shared__ float mm[W][16], ml[W][16];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kk = lane >> 4;
+  const int u = blockIdx.x;
   int sg = 0;
   while (sg + 1 < a.nseg && u >= a.unit0[sg + 1]) ++sg;
   const int P = a.P[sg], local = u - a.unit0[sg];
@@ -2292,37 +2319,36 @@ __global__ __launch_bounds__(256) void k_attn_prefill(PrefillBatchArgs a) {
   const float *qkv = a.qkv + (size_t)a.row0[sg] * a.ldq;
   const KVT *kb = reinterpret_cast<const KVT *>(a.kcache[sg]) + (size_t)kvh * a.cap * D;
   const KVT *vb = reinterpret_cast<const KVT *>(a.vcache[sg]) + (size_t)kvh * a.cap * D;
+  const int nkt = (min(q0 + 16, P) + 15) / 16;  // key tiles up to the block's last row
 
+  KvRaw8<KVT> kv[4], vv[4], kn[4], vn[4];
+  auto load = [&](int kt, KvRaw8<KVT> *k, KvRaw8<KVT> *v) {
+    const KVT *kp = kb + (size_t)min(16 * kt + li, P - 1) * D + 32 * kk;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) k[c].load(kp + 8 * c);
+#pragma unroll
+    for (int s2 = 0; s2 < 4; ++s2) v[s2].load(vb + (size_t)min(16 * kt + 4 * kk + s2, P - 1) * D + 8 * li);
+  };
   float q[32];
   {
     const float *qp = qkv + (size_t)min(q0 + li, P - 1) * a.ldq + hq * D + 32 * kk;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const float4 x0 = reinterpret_cast<const float4 *>(qp + 8 * c)[0];
-      const float4 x1 = reinterpret_cast<const float4 *>(qp + 8 * c)[1];
-      q[8 * c] = x0.x; q[8 * c + 1] = x0.y; q[8 * c + 2] = x0.z; q[8 * c + 3] = x0.w;
-      q[8 * c + 4] = x1.x; q[8 * c + 5] = x1.y; q[8 * c + 6] = x1.z; q[8 * c + 7] = x1.w;
+    for (int c = 0; c < 8; ++c) {
+      const float4 x = reinterpret_cast<const float4 *>(qp)[c];
+      q[4 * c] = x.x; q[4 * c + 1] = x.y; q[4 * c + 2] = x.z; q[4 * c + 3] = x.w;
     }
   }
   f32x4_t o[8];
 #pragma unroll
   for (int t = 0; t < 8; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float m_run = -FLT_MAX, l_part = 0.f;
-  const int qrow = q0 + li;                      // this lane's query (rows >= P are not stored)
-  const int nkt = (min(q0 + 16, P) + 15) / 16;   // key tiles up to the block's last row
-  for (int kt = 0; kt < nkt; ++kt) {
-    float kv[32];
-    {
-      const KVT *kp = kb + (size_t)min(16 * kt + li, P - 1) * D + 32 * kk;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) KvIo<KVT>::load8(kp + 8 * c, kv + 8 * c);
-    }
-    float vv[4][8];
-#pragma unroll
-    for (int s2 = 0; s2 < 4; ++s2) KvIo<KVT>::load8(vb + (size_t)min(16 * kt + 4 * kk + s2, P - 1) * D + 8 * li, vv[s2]);
+  float m_run = -FLT_MAX, l = 0.f;
+  const int qrow = q0 + li;  // this lane's query (rows >= P are not stored)
+  if (wave < nkt) load(wave, kv, vv);
+  for (int kt = wave; kt < nkt; kt += W) {
+    if (kt + W < nkt) load(kt + W, kn, vn);
     f32x4_t st = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int s1 = 0; s1 < 32; ++s1) st = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[s1], q[s1], st, 0, 0, 0);
+    for (int s1 = 0; s1 < 32; ++s1) st = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[s1 >> 3][s1 & 7], q[s1], st, 0, 0, 0);
     float p[4], mt = -FLT_MAX;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -2340,7 +2366,7 @@ __global__ __launch_bounds__(256) void k_attn_prefill(PrefillBatchArgs a) {
       p[e] = p[e] == -FLT_MAX ? 0.f : expf(p[e] - m_new);
       ps += p[e];
     }
-    l_part = l_part * corr + ps;
+    l = l * corr + ps;
     m_run = m_new;
 #pragma unroll
     for (int t = 0; t < 8; ++t) o[t] *= corr;
@@ -2348,18 +2374,38 @@ __global__ __launch_bounds__(256) void k_attn_prefill(PrefillBatchArgs a) {
     for (int s2 = 0; s2 < 4; ++s2)
 #pragma unroll
       for (int t = 0; t < 8; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[s2][t], p[s2], o[t], 0, 0, 0);
-  }
-  float l = l_part;
-  l += __builtin_bit_cast(float, lane_xor_u32<16>(__builtin_bit_cast(uint32_t, l)));
-  l += __builtin_bit_cast(float, lane_xor_u32<32>(__builtin_bit_cast(uint32_t, l)));
-  if (qrow >= P) return;
-  const float inv = 1.0f / l;
-  float *op = a.out + (size_t)(a.row0[sg] + qrow) * a.ldo + hq * D + 32 * kk;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    reinterpret_cast<float4 *>(op + 8 * e)[0] = make_float4(o[0][e] * inv, o[1][e] * inv, o[2][e] * inv, o[3][e] * inv);
-    reinterpret_cast<float4 *>(op + 8 * e)[1] = make_float4(o[4][e] * inv, o[5][e] * inv, o[6][e] * inv, o[7][e] * inv);
+    for (int c = 0; c < 4; ++c) {
+      kv[c] = kn[c];
+      vv[c] = vn[c];
+    }
   }
+  l = pair32_sum(pair16_sum(l));
+  if (kk == 0) {
+    mm[wave][li] = m_run;
+    ml[wave][li] = l;
+  }
+#pragma unroll
+  for (int t = 0; t < 8; ++t)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) mo[wave][8 * e + t][lane] = o[t][e];
+  __syncthreads();
+  if (qrow >= P) return;
+  float m = mm[0][li];
+#pragma unroll
+  for (int w = 1; w < W; ++w) m = fmaxf(m, mm[w][li]);
+  float lsum = 0.f, r[8] = {};
+#pragma unroll
+  for (int w = 0; w < W; ++w) {  // a wave without a tile has m = -FLT_MAX, l = 0: weight 0
+    const float f = expf(mm[w][li] - m);
+    lsum += ml[w][li] * f;
+#pragma unroll
+    for (int t = 0; t < 8; ++t) r[t] += mo[w][8 * wave + t][lane] * f;
+  }
+  const float inv = 1.0f / lsum;
+  float4 *op = reinterpret_cast<float4 *>(a.out + (size_t)(a.row0[sg] + qrow) * a.ldo + hq * D + 32 * kk + 8 * wave);
+  op[0] = make_float4(r[0] * inv, r[1] * inv, r[2] * inv, r[3] * inv);
+  op[1] = make_float4(r[4] * inv, r[5] * inv, r[6] * inv, r[7] * inv);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -3674,7 +3720,7 @@ hipError_t launch_prefill_attention(const PrefillBatchArgs &a, hipStream_t s) {
     rows += a.P[i];
   }
   if (rows != a.M) return hipErrorInvalidValue;
-  const dim3 g1((a.q_heads + 2 * a.kv_heads + 3) / 4, a.M), g2((a.unit0[a.nseg] + 3) / 4), block(256);
+  const dim3 g1((a.q_heads + 2 * a.kv_heads + 3) / 4, a.M), g2(a.unit0[a.nseg]), block(256);
   if (a.kv_bf16) {
     hipLaunchKernelGGL(k_prefill_qkv<uint16_t>, g1, block, 0, s, a);
     hipLaunchKernelGGL(k_attn_prefill<uint16_t>, g2, block, 0, s, a);

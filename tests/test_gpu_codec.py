@@ -39,11 +39,11 @@ def test_decode_matches_oracle(codec_case, frames):
     assert err <= WAVE_TOL
 
 
-@pytest.mark.parametrize("frames", [1, 2, 5])
+@pytest.mark.parametrize("frames", [1, 2, 5, 16, 17])
 def test_decode_at_block_edges(codec_case, frames):
     """The decoder convolutions' 64-row blocks at half, exactly one and a remainder of a block
     (32 rows a frame after the first transposed convolution), split over channels, with rows
-    before time 0 in every block.  ~45 layers of fp32 sums of exact products end within 3.4e-6 of
+    before time 0 in every block, and the attention's 16-row tiles (16, 17).  ~45 layers of fp32 sums of exact products end within 3.4e-6 of
     float64 (2-norm) on inputs of 6 to 240 frames; four times that is allowed."""
     eng, oracle = codec_case
     codes = np.random.default_rng(100 + frames).integers(0, 2048, (frames, 16)).astype(np.int32)

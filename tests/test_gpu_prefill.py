@@ -40,3 +40,22 @@ def test_prefill_lengths_match_oracle(models, spec, kv_bf16):
             tol = (2e-3, 2e-4) if kv_bf16 else (1e-5, 1e-6)
             _close(hidden, o.hidden, *tol, f"P={P} hidden")
             _close(logits, want, *tol, f"P={P} logits")
+
+
+@pytest.mark.parametrize("kv_bf16", [False, True])
+def test_prefill_tiles_per_wave(models, kv_bf16):
+    """Lengths at which the attention's four waves (every fourth 16-key tile each) gain a tile, or
+    one of them does: 48 / 49 and 63 .. 65 rows (three, four and five tiles), 80 / 81 and 128 / 129."""
+    model, d = models.get("tiny", 0)
+    rng = np.random.default_rng(12)
+    print(f"[gpu] prefill tiles per wave kv_bf16={kv_bf16}", flush=True)
+    with E.HipTtsEngine(d, E.EngineOptions(max_cache_steps=CAP, kv_bf16=kv_bf16)) as eng:
+        for P in (48, 49, 63, 64, 65, 80, 81, 128, 129):
+            x = (rng.standard_normal((P, model.spec.talker.hidden)) * 0.5).astype(np.float32)
+            hidden, logits, _ = eng.debug_talker_prefill(x)
+            o = Oracle(model.tensors, model.config(), max_cache_steps=CAP, kv_bf16=kv_bf16)
+            want = o.prefill(x.astype(np.float64))
+            # the bounds of test_prefill_lengths_match_oracle
+            tol = (2e-3, 2e-4) if kv_bf16 else (1e-5, 1e-6)
+            _close(hidden, o.hidden, *tol, f"P={P} hidden")
+            _close(logits, want, *tol, f"P={P} logits")
