@@ -44,6 +44,7 @@ struct Codec {
   std::vector<void *> allocs;
   int64_t bytes = 0;
   float *cb_first = nullptr, *cb_rest = nullptr;  // normalized codebooks [V][D], [15][V][D]
+  // Matrices are packed (launch_pack_weights; convolutions: codec_conv_pack).
   uint16_t *w_rvq = nullptr;                      // [512][first 256 | rest 256]
   uint16_t *pre_w = nullptr;                      // [1024][3][512]
   float *pre_b = nullptr;
@@ -66,7 +67,7 @@ struct Codec {
   struct Unit {
     float *a1a, *a1b, *a2a, *a2b, *b1, *b2;
     uint16_t *w1;       // 7 taps co -> co
-    uint16_t *w2;       // [co][co], or as w1 with one tap where codec_unit_ok(co)
+    uint16_t *w2;       // [co][co]
   };
   struct Block {
     float *snake_a, *snake_b;
@@ -77,8 +78,8 @@ struct Codec {
   float *fin_a = nullptr, *fin_b = nullptr, *fin_w = nullptr, *fin_bias = nullptr;  // fin_w [7][96]
   float *ws = nullptr;  // decode workspace, grown to the largest frame count seen
   size_t ws_floats = 0;
-  // K-split partial sums of the GEMMs that would otherwise run as few workgroups (short
-  // windows: a streaming chunk decodes ~31 frames)
+  // Channel-split partial sums of the convolutions of short windows (a streaming chunk decodes
+  // ~31 frames)
   float *split_ws = nullptr;
   static constexpr int64_t kSplitFloats = (int64_t)4 << 20;
   int32_t *codes_ws = nullptr;  // staging for host codes
@@ -115,6 +116,23 @@ Codec *codec_load(const std::string &model_dir, int64_t *device_bytes) {
       b = up_f32(prefix + "beta", len);
       hip_check(launch_codec_snake_prep(a, b, (int)len, nullptr), "launch_codec_snake_prep");
     };
+    // An N x K matrix in matrix-core order (launch_pack_weights).
+    auto up_packed = [&](const std::vector<uint16_t> &v, int N, int K) {
+      int64_t scratch = 0;
+      uint16_t *rows = dev_alloc<uint16_t>(v.size(), scratch), *d = nullptr;
+      try {
+        HIPC(hipMemcpy(rows, v.data(), v.size() * 2, hipMemcpyHostToDevice));
+        d = dev_alloc<uint16_t>(v.size(), c->bytes);
+        c->allocs.push_back(d);
+        hip_check(launch_pack_weights(rows, d, N, K, nullptr), "launch_pack_weights");
+        HIPC(hipStreamSynchronize(nullptr));
+      } catch (...) {
+        (void)hipFree(rows);
+        throw;
+      }
+      (void)hipFree(rows);
+      return d;
+    };
     // [O][C][K] -> [O][K][C]
     auto taps_last_to_first = [](const std::vector<uint16_t> &w, int O, int C, int K) {
       std::vector<uint16_t> r((size_t)O * C * K);
@@ -148,17 +166,18 @@ Codec *codec_load(const std::string &model_dir, int64_t *device_bytes) {
           w[(size_t)o * 2 * kCodebookDim + d] = w1[(size_t)o * kCodebookDim + d];
           w[(size_t)o * 2 * kCodebookDim + kCodebookDim + d] = w2[(size_t)o * kCodebookDim + d];
         }
-      c->w_rvq = c->upload(w);
+      c->w_rvq = up_packed(w, kProjected, 2 * kCodebookDim);
     }
-    c->pre_w = c->upload(taps_last_to_first(bf16("decoder.pre_conv.conv.weight", {kPreConv, kProjected, 3}),
-                                            kPreConv, kProjected, 3));
+    c->pre_w = up_packed(taps_last_to_first(bf16("decoder.pre_conv.conv.weight", {kPreConv, kProjected, 3}), kPreConv,
+                                            kProjected, 3),
+                         kPreConv, 3 * kProjected);
     c->pre_b = up_f32("decoder.pre_conv.conv.bias", kPreConv);
 
     // pre-transformer (codec_hip.rs:380-654, 1139-1188)
     const std::string t = "decoder.pre_transformer";
-    c->in_w = c->upload(bf16(t + ".input_proj.weight", {kHidden, kPreConv}));
+    c->in_w = up_packed(bf16(t + ".input_proj.weight", {kHidden, kPreConv}), kHidden, kPreConv);
     c->in_b = up_f32(t + ".input_proj.bias", kHidden);
-    c->out_w = c->upload(bf16(t + ".output_proj.weight", {kPreConv, kHidden}));
+    c->out_w = up_packed(bf16(t + ".output_proj.weight", {kPreConv, kHidden}), kPreConv, kHidden);
     c->out_b = up_f32(t + ".output_proj.bias", kPreConv);
     c->norm = up_f32(t + ".norm.weight", kHidden);
     for (int i = 0; i < kLayers; ++i) {
@@ -170,13 +189,13 @@ Codec *codec_load(const std::string &model_dir, int64_t *device_bytes) {
       L.mlp_scale = up_f32(p + ".mlp_layer_scale.scale", kHidden);
       std::vector<uint16_t> qkv;
       for (const char *n : {"q_proj", "k_proj", "v_proj"}) st.append_bf16(p + ".self_attn." + n + ".weight", {kQ, kHidden}, qkv);
-      L.qkv = c->upload(qkv);
-      L.o = c->upload(bf16(p + ".self_attn.o_proj.weight", {kHidden, kQ}));
+      L.qkv = up_packed(qkv, 3 * kQ, kHidden);
+      L.o = up_packed(bf16(p + ".self_attn.o_proj.weight", {kHidden, kQ}), kHidden, kQ);
       std::vector<uint16_t> gu;
       st.append_bf16(p + ".mlp.gate_proj.weight", {kInter, kHidden}, gu);
       st.append_bf16(p + ".mlp.up_proj.weight", {kInter, kHidden}, gu);
-      L.gu = c->upload(gu);
-      L.down = c->upload(bf16(p + ".mlp.down_proj.weight", {kHidden, kInter}));
+      L.gu = up_packed(gu, 2 * kInter, kHidden);
+      L.down = up_packed(bf16(p + ".mlp.down_proj.weight", {kHidden, kInter}), kHidden, kInter);
     }
     {
       std::vector<float2> rope((size_t)kCodecMaxAttnRows * 32);
@@ -197,7 +216,7 @@ Codec *codec_load(const std::string &model_dir, int64_t *device_bytes) {
       for (int ph = 0; ph < 2; ++ph)
         for (int o = 0; o < kUp; ++o)
           for (int ci = 0; ci < kUp; ++ci) w[((size_t)ph * kUp + o) * kUp + ci] = tw[((size_t)ci * kUp + o) * 2 + ph];
-      U.tw = c->upload(w);
+      U.tw = up_packed(w, 2 * kUp, kUp);
       std::vector<float> tb = f32(p + ".0.conv.bias", kUp);
       tb.insert(tb.end(), tb.begin(), tb.end());
       U.tb = c->upload(tb);
@@ -205,9 +224,9 @@ Codec *codec_load(const std::string &model_dir, int64_t *device_bytes) {
       U.dw_b = up_f32(p + ".1.dwconv.conv.bias", kUp);
       U.ln_g = up_f32(p + ".1.norm.weight", kUp);
       U.ln_b = up_f32(p + ".1.norm.bias", kUp);
-      U.pw1 = c->upload(bf16(p + ".1.pwconv1.weight", {kConvNext, kUp}));
+      U.pw1 = up_packed(bf16(p + ".1.pwconv1.weight", {kConvNext, kUp}), kConvNext, kUp);
       U.pw1_b = up_f32(p + ".1.pwconv1.bias", kConvNext);
-      U.pw2 = c->upload(bf16(p + ".1.pwconv2.weight", {kUp, kConvNext}));
+      U.pw2 = up_packed(bf16(p + ".1.pwconv2.weight", {kUp, kConvNext}), kUp, kConvNext);
       U.pw2_b = up_f32(p + ".1.pwconv2.bias", kUp);
       U.gamma = up_f32(p + ".1.gamma", kUp);
     }
@@ -246,7 +265,7 @@ Codec *codec_load(const std::string &model_dir, int64_t *device_bytes) {
         Un.w1 = c->upload(codec_conv_pack(bf16(r + ".conv1.conv.weight", {co, co, 7}), co, co, 7, conv_at));
         Un.b1 = up_f32(r + ".conv1.conv.bias", co);
         const auto w2 = bf16(r + ".conv2.conv.weight", {co, co, 1});
-        Un.w2 = c->upload(codec_unit_ok(co) ? codec_conv_pack(w2, co, co, 1, conv_at) : w2);
+        Un.w2 = up_packed(w2, co, co);
         Un.b2 = up_f32(r + ".conv2.conv.bias", co);
       }
     }
@@ -307,7 +326,7 @@ namespace {
 size_t workspace_floats(size_t F) {
   const size_t big = (size_t)kCodecSamplesPerFrame * kFinal * F;  // largest T x C of the decoder blocks
   return 256 * 24 + F * 2 * kCodebookDim + (kPad + F) * kProjected + F * kPreConv + F * kHidden + F * 3 * kQ +
-         F * kQ + F * kInter + F + F * kPreConv + 2 * ((kPad + 4 * F) * kUp) + 4 * F * kUp + 4 * F * kConvNext +
+         F * kQ + F * kInter + F * kPreConv + 2 * ((kPad + 4 * F) * kUp) + 4 * F * kUp + 4 * F * kConvNext +
          (kPad * kFinal + big) + 2 * big;
 }
 
@@ -334,11 +353,10 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
   auto zero_pad = [&](float *buf, int C) { HIPC(hipMemsetAsync(buf, 0, (size_t)kPad * C * sizeof(float), s)); };
   auto gemm = [&](int epi, const float *X, int ldx, int M, const uint16_t *W, int N, int K, float *Y, int ldy,
                   const float *bias, const float *res = nullptr, int ldr = 0, const float *scale = nullptr,
-                  const float *row_scale = nullptr, const float *gamma = nullptr) {
+                  const float *gamma = nullptr) {
     GemmArgs g{};
     g.X = X; g.ldx = ldx; g.W = W; g.Y = Y; g.ldy = ldy; g.M = M; g.N = N; g.K = K;
-    g.bias = bias; g.res = res; g.ldr = ldr; g.scale = scale; g.row_scale = row_scale; g.gamma = gamma;
-    g.split_ws = c.split_ws; g.split_cap = Codec::kSplitFloats;
+    g.bias = bias; g.res = res; g.ldr = ldr; g.scale = scale; g.gamma = gamma; g.eps = kRmsEps; g.w_packed = 1;
     hip_check(launch_gemm(epi, g, s), "launch_gemm(codec)");
   };
 
@@ -358,21 +376,17 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
   float *QKV = take((size_t)F * 3 * kQ);
   float *ATT = take((size_t)F * kQ);
   float *ACT = take((size_t)F * kInter);
-  float *INV = take((size_t)F);
   gemm(EPI_BIAS, PC, kPreConv, F, c.in_w, kHidden, kPreConv, H, kHidden, c.in_b);
   for (int i = 0; i < kLayers; ++i) {
     const Codec::Layer &L = c.layers[i];
-    hip_check(launch_row_rms(H, kHidden, F, kHidden, kRmsEps, INV, s), "row_rms");
-    gemm(EPI_STORE, H, kHidden, F, L.qkv, 3 * kQ, kHidden, QKV, 3 * kQ, nullptr, nullptr, 0, nullptr, INV, L.g_in);
+    gemm(EPI_STORE, H, kHidden, F, L.qkv, 3 * kQ, kHidden, QKV, 3 * kQ, nullptr, nullptr, 0, nullptr, L.g_in);
     hip_check(launch_codec_attention(QKV, F, 3 * kQ, kHeads, c.rope, 0.125f, ATT, kQ, s), "codec_attention");
     gemm(EPI_AFFINE_RES, ATT, kQ, F, L.o, kHidden, kQ, H, kHidden, nullptr, H, kHidden, L.attn_scale);
-    hip_check(launch_row_rms(H, kHidden, F, kHidden, kRmsEps, INV, s), "row_rms");
-    gemm(EPI_SWIGLU, H, kHidden, F, L.gu, kInter, kHidden, ACT, kInter, nullptr, nullptr, 0, nullptr, INV, L.g_post);
+    gemm(EPI_SWIGLU, H, kHidden, F, L.gu, kInter, kHidden, ACT, kInter, nullptr, nullptr, 0, nullptr, L.g_post);
     gemm(EPI_AFFINE_RES, ACT, kInter, F, L.down, kHidden, kInter, H, kHidden, nullptr, H, kHidden, L.mlp_scale);
   }
   float *TR = take((size_t)F * kPreConv);
-  hip_check(launch_row_rms(H, kHidden, F, kHidden, kRmsEps, INV, s), "row_rms");
-  gemm(EPI_BIAS, H, kHidden, F, c.out_w, kPreConv, kHidden, TR, kPreConv, c.out_b, nullptr, 0, nullptr, INV, c.norm);
+  gemm(EPI_BIAS, H, kHidden, F, c.out_w, kPreConv, kHidden, TR, kPreConv, c.out_b, nullptr, 0, nullptr, c.norm);
 
   // 4. two upsample stages: transposed conv (stride 2) + ConvNeXt block
   float *Up = take((size_t)(kPad + 4 * F) * kUp);
@@ -431,8 +445,7 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
       GemmArgs g{};
       g.X = A2; g.ldx = co; g.W = Un.w2; g.Y = end ? S : R; g.ldy = co; g.M = T; g.N = co; g.K = co;
       g.bias = Un.b2; g.res = R; g.ldr = co;
-      g.snake_a = na; g.snake_b = nb;
-      g.split_ws = c.split_ws; g.split_cap = Codec::kSplitFloats;
+      g.snake_a = na; g.snake_b = nb; g.w_packed = 1;
       hip_check(launch_gemm(end ? EPI_RES_SNAKE : EPI_AFFINE_RES, g, s), "launch_gemm(1x1)");
     }
   }

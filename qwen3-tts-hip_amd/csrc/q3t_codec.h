@@ -50,7 +50,7 @@ struct CodecConvArgs {
   // A whole residual unit (7 taps, both Snakes, C = N, codec_unit_ok): the Snaked output goes on
   // through a 1x1 convolution in the same launch, Y = S(X + (b2 + w2 . out)), S the Snake of
   // ra / rb or, with null tables, the identity.
-  const uint16_t *w2;     // codec_conv_pack layout, one tap; null: no second half
+  const uint16_t *w2;     // [N][C] packed (launch_pack_weights); null: no second half
   const float *b2, *ra, *rb;
 };
 bool codec_unit_ok(int C);

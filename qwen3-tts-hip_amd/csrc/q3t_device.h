@@ -193,42 +193,34 @@ __host__ __device__ inline size_t t16_index(int m, int k) {
   return ((size_t)(k >> 5) * 64 + ((k >> 3) & 3) * 16 + m) * 8 + (k & 7);
 }
 
-// Y[M][N] = X[M][K] . W[N][K]^T with the GEMV epilogues (matrix-core path for many rows).
+// Y[M][N] = X[M][K] . W[N][K]^T with the GEMV epilogues (matrix-core path for many rows), the rows
+// of X normalised first when gamma is set.
 struct GemmArgs {
   const float *X;          // [M][ldx] fp32
-  const float *row_scale;  // [M] per-row multiplier on X (RMSNorm 1/rms) or null
-  const float *gamma;      // [K] per-column multiplier on X (RMSNorm gain) or null
-  const uint16_t *W;       // [N][K] bf16 (EPI_SWIGLU: [2N][K], gate rows then up rows)
+  const float *gamma;      // [K] RMSNorm gain of X's rows, or null: no RMSNorm
+  // bf16, packed (launch_pack_weights) as [N/16][K/32][64 lanes][8]: each k step of a 16-column
+  // tile is 1 KiB contiguous.  The last tile is padded; EPI_SWIGLU: the gate rows' tiles, then the
+  // up rows' tiles.  w_packed says so.
+  const uint16_t *W;
   float *Y;                // [M][ldy]
   const float *res;        // EPI_RESIDUAL: [M][ldr]
   const float *bias;       // EPI_BIAS: [N]
   const float *scale;      // EPI_AFFINE_RES: [N] or null
   const float *snake_a, *snake_b;  // EPI_RES_SNAKE: [N] exp(alpha), 1 / (exp(beta) + 1e-9)
   int32_t M, N, K, ldx, ldy, ldr;
-  // Segmented X rows (matrix-core GEMMs; a dilated convolution's taps): with xseg_len > 0,
-  // element k of row m is X[m * ldx + (k / xseg_len) * xseg_stride + k % xseg_len].
-  int32_t xseg_len, xseg_stride;
-  float eps;               // skinny GEMM with a fused RMSNorm
+  float eps;               // RMSNorm
   const int32_t *row_on;   // skinny GEMM: row m is stored only where row_on[m] (null: all rows)
-  // skinny GEMM layouts: X / Y / res in T16 (ld ignored) instead of row-major.  Its W must be
-  // packed (w_packed = 1) as [N/16][K/32][64 lanes][8] (each k step of a 16-column tile is
-  // 1 KiB contiguous).
+  // skinny GEMM layouts: X / Y / res in T16 (ld ignored) instead of row-major.
   int32_t x_t16, y_t16, r_t16, w_packed;
   // skinny GEMM, EPI_STORE: instead of Y, each workgroup (16 columns) stores every row's
   // largest order key (value, lowest column) at keys_out[m * keys_row + blockIdx.x].
   uint64_t *keys_out;
   int64_t keys_row;
-  // matrix-core GEMMs: a launch of few workgroups may split K over grid z, each split storing
-  // its raw sums to split_ws[z][M][N] (SwiGLU: [z][M][2N], the up sums at N + n; split_cap
-  // floats available); a second kernel adds the splits in order and applies the epilogue.
-  // Null: never split.
-  float *split_ws;
-  int64_t split_cap;
-  // skinny GEMM, EPI_RESIDUAL, T16 Y: K split in two halves over grid y.  Each half adds its
-  // sums to Y with an fp32 atomic add, so Y must hold zeros; two adds onto zero commute, so
-  // the result does not depend on their order.  The first half also adds the residual, and
-  // then stores zero to res_zero (T16, may be res itself) at the same element: the buffer
-  // the next split GEMM of the chain accumulates into.
+  // EPI_RESIDUAL, few rows (skinny GEMM: T16 Y; launch_gemm: up to kGemmSplitRows rows): K split in
+  // two halves over grid y.  Each half adds its sums to Y with an fp32 atomic add, so Y must hold
+  // zeros; two adds onto zero commute, so the result does not depend on their order.  The first
+  // half also adds the residual, and then stores zero to res_zero (laid out as res, may be res
+  // itself) at the same element: the buffer the next split GEMM of the chain accumulates into.
   int32_t split2;
   float *res_zero;
   // skinny GEMM: mb = 2 runs two 16-row blocks (two positions of the same stream rows, row m

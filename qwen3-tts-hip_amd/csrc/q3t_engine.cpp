@@ -87,7 +87,8 @@ Dims dims_from(const json::Value &c) {
 struct LayerW {
   const uint16_t *qkv, *o, *gu, *down;
   const float *g_in, *g_post, *gq, *gk;
-  // The same matrices in the skinny GEMM's packed layout (multi-stream engines only).
+  // The same matrices in the matrix-core GEMMs' packed layout (the Talker's always: its prefill;
+  // the CodePredictor's in multi-stream engines).
   const uint16_t *qkv_p = nullptr, *o_p = nullptr, *gu_p = nullptr, *down_p = nullptr;
 };
 
@@ -219,7 +220,12 @@ struct Pools {
   SlotParams *prm = nullptr;
   int32_t *row_on = nullptr;                            // [n] rows a batched launch covers
   int prefill_rows = 0;                                 // n * cap
-  float *px = nullptr, *pqkv = nullptr, *pattn = nullptr, *pact = nullptr, *pinv = nullptr;
+  float *px = nullptr, *pqkv = nullptr, *pattn = nullptr, *pact = nullptr;
+  // The mid-layer residual of a prefill of at most kGemmSplitRows rows (split O / down GEMMs): zeros
+  // except between a layer's O and down GEMMs.  pmid_dirty: a prefill stopped with an error, possibly
+  // between the two; the next one zeroes it first.
+  float *pmid = nullptr;
+  bool pmid_dirty = false;
   SlotState *h_states = nullptr;                        // pinned [n]
   int32_t *h_codes = nullptr;                           // pinned [n][codes_row], mirrors codes
   int32_t *h_row_on = nullptr;                          // pinned [n]
@@ -268,14 +274,11 @@ struct Engine {
   // raw q/k/v row of every input token, [groups-2][Vc][qkv_rows], and (projection only) the
   // projected input row, [groups-2][Vc][Hc].
   float *cp_qkv_table = nullptr, *cp_in_table = nullptr;
-  // K-split partial sums of prompt-prefill and text-projection GEMMs over few rows
-  static constexpr int64_t kSplitFloats = (int64_t)4 << 20;
-  float *split_ws = nullptr;
   // result of resolving the device's no-allocation scratch at creation
   hipError_t scratch_status = hipErrorNotInitialized;
   // Prompt preparation on the device (text.rs:516-603), when the checkpoint holds
   // talker.model.text_embedding.weight: the table [text_vocab][text_hidden] and the text
-  // projection fc1 [tp_inter][text_hidden] + bias, fc2 [H][tp_inter] + bias.
+  // projection fc1 [tp_inter][text_hidden] + bias, fc2 [H][tp_inter] + bias (matrices packed).
   uint16_t *text_emb = nullptr, *tp_fc1 = nullptr, *tp_fc2 = nullptr;
   float *tp_b1 = nullptr, *tp_b2 = nullptr;
   int text_vocab = 0, text_hidden = 0, tp_inter = 0;
@@ -465,13 +468,16 @@ struct Engine {
     if (M <= 0 || M > p.prefill_rows) fail(Q3T_ERR_CAPACITY, "prefill of %d rows exceeds the workspace", M);
     const size_t esz = kv_bf16 ? 2 : 4;
     const size_t cache_layer = (size_t)d.kv_heads * talker.cap * d.head_dim * esz;
+    // Few rows: the O and down GEMMs split K in two (GemmArgs::split2), O from px into pmid (zeros),
+    // zeroing px, and down from pmid back into px, zeroing pmid.
+    const bool split = M <= kGemmSplitRows;
+    if (split && p.pmid_dirty) HIPC(hipMemsetAsync(p.pmid, 0, (size_t)kGemmSplitRows * H * 4, s));
+    p.pmid_dirty = split;
     for (int l = 0; l < d.layers; ++l) {
       const LayerW &L = talker.layers[l];
-      hip_check(launch_row_rms(p.px, H, M, H, d.eps, p.pinv, s), "launch_row_rms");
       GemmArgs g{};
-      g.X = p.px; g.ldx = H; g.row_scale = p.pinv; g.gamma = L.g_in;
-      g.W = L.qkv; g.Y = p.pqkv; g.ldy = Q; g.M = M; g.N = Q; g.K = H;
-      g.split_ws = split_ws; g.split_cap = kSplitFloats;
+      g.X = p.px; g.ldx = H; g.gamma = L.g_in; g.eps = d.eps;
+      g.W = L.qkv_p; g.w_packed = 1; g.Y = p.pqkv; g.ldy = Q; g.M = M; g.N = Q; g.K = H;
       hip_check(launch_gemm(EPI_STORE, g, s), "launch_gemm(qkv)");
       PrefillBatchArgs pa{};
       pa.qkv = p.pqkv; pa.gq = L.gq; pa.gk = L.gk; pa.rope = talker.rope; pa.out = p.pattn;
@@ -488,22 +494,27 @@ struct Engine {
       }
       hip_check(launch_prefill_attention(pa, s), "launch_prefill_attention");
       g = GemmArgs{};
-      g.X = p.pattn; g.ldx = O; g.W = L.o; g.res = p.px; g.ldr = H; g.Y = p.px; g.ldy = H;
+      g.X = p.pattn; g.ldx = O; g.W = L.o_p; g.w_packed = 1; g.res = p.px; g.ldr = H; g.Y = p.px; g.ldy = H;
       g.M = M; g.N = H; g.K = O;
-      g.split_ws = split_ws; g.split_cap = kSplitFloats;
+      float *mid = p.px;
+      if (split) {
+        mid = p.pmid;
+        g.Y = mid; g.split2 = 1; g.res_zero = p.px;
+      }
       hip_check(launch_gemm(EPI_RESIDUAL, g, s), "launch_gemm(o)");
-      hip_check(launch_row_rms(p.px, H, M, H, d.eps, p.pinv, s), "launch_row_rms");
       g = GemmArgs{};
-      g.X = p.px; g.ldx = H; g.row_scale = p.pinv; g.gamma = L.g_post;
-      g.W = L.gu; g.Y = p.pact; g.ldy = I; g.M = M; g.N = I; g.K = H;
-      g.split_ws = split_ws; g.split_cap = kSplitFloats;
+      g.X = mid; g.ldx = H; g.gamma = L.g_post; g.eps = d.eps;
+      g.W = L.gu_p; g.w_packed = 1; g.Y = p.pact; g.ldy = I; g.M = M; g.N = I; g.K = H;
       hip_check(launch_gemm(EPI_SWIGLU, g, s), "launch_gemm(gate_up)");
       g = GemmArgs{};
-      g.X = p.pact; g.ldx = I; g.W = L.down; g.res = p.px; g.ldr = H; g.Y = p.px; g.ldy = H;
+      g.X = p.pact; g.ldx = I; g.W = L.down_p; g.w_packed = 1; g.res = mid; g.ldr = H; g.Y = p.px; g.ldy = H;
       g.M = M; g.N = H; g.K = I;
-      g.split_ws = split_ws; g.split_cap = kSplitFloats;
+      if (split) {
+        g.split2 = 1; g.res_zero = mid;
+      }
       hip_check(launch_gemm(EPI_RESIDUAL, g, s), "launch_gemm(down)");
     }
+    p.pmid_dirty = false;
     for (const PrefillSeg &sg : segs)
       HIPC(hipMemcpyAsync(slots[sg.slot].x_t, p.px + (size_t)(sg.row0 + sg.P - 1) * H, (size_t)H * 4,
                           hipMemcpyDeviceToDevice, s));
@@ -1091,7 +1102,7 @@ void alloc_pools(Engine &e, int n) {
   p.pqkv = dev_alloc<float>((size_t)p.prefill_rows * td.qkv_rows(), t);
   p.pattn = dev_alloc<float>((size_t)p.prefill_rows * td.q_out(), t);
   p.pact = dev_alloc<float>((size_t)p.prefill_rows * td.intermediate, t);
-  p.pinv = dev_alloc<float>((size_t)p.prefill_rows, t);
+  p.pmid = (float *)zeroed((size_t)kGemmSplitRows * Ht * 4);
   HIPC(hipHostMalloc((void **)&p.h_states, sizeof(SlotState) * n, hipHostMallocDefault));
   HIPC(hipHostMalloc((void **)&p.h_codes, (size_t)p.codes_row * n * 4, hipHostMallocDefault));
   HIPC(hipHostMalloc((void **)&p.h_row_on, sizeof(int32_t) * n, hipHostMallocDefault));
@@ -1146,13 +1157,41 @@ void free_pools(Engine &e) {
   void *ptrs[] = {p.t_k,      p.t_v,     p.c_k,   p.c_v,      p.x_t,      p.t_in,    p.qkv,  p.attn,
                   p.act,      p.logits_t, p.logits_c, p.x_c,  p.cp_prefix, p.cp_in,  p.cur,  p.emb_sum,
                   p.trailing, p.attn_part, p.trace_t, p.trace_c, p.codes,  p.st,      p.prm,  p.row_on,
-                  p.px,       p.pqkv,    p.pattn, p.pact,     p.pinv,    p.cp_keys, p.opart, p.x_mid, p.tok_cur};
+                  p.px,       p.pqkv,    p.pattn, p.pact,     p.pmid,    p.cp_keys, p.opart, p.x_mid, p.tok_cur};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   if (p.h_states) (void)hipHostFree(p.h_states);
   if (p.h_codes) (void)hipHostFree(p.h_codes);
   if (p.h_row_on) (void)hipHostFree(p.h_row_on);
   p = Pools();
+}
+
+// Packs rows x K of a device matrix (rows a multiple of 16) into its own allocation.
+uint16_t *pack_weights(const uint16_t *src, int rows, int K, int64_t &t) {
+  uint16_t *d = dev_alloc<uint16_t>((size_t)rows * K, t);
+  hip_check(launch_pack_weights(src, d, rows, K, nullptr), "launch_pack_weights");
+  return d;
+}
+
+// A second copy of a stack's matrices in the packed layout.
+void pack_stack(StackW &w, int64_t &t) {
+  const Dims &d = w.d;
+  const size_t per_layer = (size_t)d.qkv_rows() * d.hidden + (size_t)d.hidden * d.q_out() +
+                           (size_t)2 * d.intermediate * d.hidden + (size_t)d.hidden * d.intermediate;
+  w.mats_p = dev_alloc<uint16_t>(per_layer * d.layers, t);
+  for (LayerW &L : w.layers) {
+    auto at = [&](const uint16_t *m) { return w.mats_p + (m - w.mats); };
+    L.qkv_p = at(L.qkv);
+    L.o_p = at(L.o);
+    L.gu_p = at(L.gu);
+    L.down_p = at(L.down);
+    hip_check(launch_pack_weights(L.qkv, const_cast<uint16_t *>(L.qkv_p), d.qkv_rows(), d.hidden, nullptr), "pack");
+    hip_check(launch_pack_weights(L.o, const_cast<uint16_t *>(L.o_p), d.hidden, d.q_out(), nullptr), "pack");
+    hip_check(launch_pack_weights(L.gu, const_cast<uint16_t *>(L.gu_p), 2 * d.intermediate, d.hidden, nullptr),
+              "pack");
+    hip_check(launch_pack_weights(L.down, const_cast<uint16_t *>(L.down_p), d.hidden, d.intermediate, nullptr),
+              "pack");
+  }
 }
 
 // Greedy hand-off tables: layer 0's raw q/k/v row (and, with the projection, its input row)
@@ -1168,36 +1207,38 @@ void build_cp_tables(Engine &e) {
   if (e.has_proj) e.cp_in_table = dev_alloc<float>((size_t)n * Vc * Hc, t);
   int64_t scratch_bytes = 0;
   float *X = dev_alloc<float>((size_t)Vc * Ht, scratch_bytes);
-  float *inv = nullptr;
+  uint16_t *wq = nullptr, *wp = nullptr;
+  auto release = [&] {
+    for (void *q : {(void *)X, (void *)wq, (void *)wp})
+      if (q) (void)hipFree(q);
+  };
   try {
-    inv = dev_alloc<float>((size_t)Vc, scratch_bytes);
+    wq = pack_weights(e.cp.layers[0].qkv, Q, Hc, scratch_bytes);
+    if (e.has_proj) wp = pack_weights(e.proj_w, Hc, Ht, scratch_bytes);
     for (int g = 1; g <= n; ++g) {
       hip_check(launch_bf16_to_f32(e.cp_emb + (size_t)(g - 1) * Vc * Ht, X, (size_t)Vc * Ht, nullptr),
                 "launch_bf16_to_f32");
       const float *src = X;
       if (e.has_proj) {
         GemmArgs p{};
-        p.X = X; p.ldx = Ht; p.W = e.proj_w; p.bias = e.proj_b;
+        p.X = X; p.ldx = Ht; p.W = wp; p.w_packed = 1; p.bias = e.proj_b;
         p.Y = e.cp_in_table + (size_t)(g - 1) * Vc * Hc; p.ldy = Hc;
         p.M = Vc; p.N = Hc; p.K = Ht;
         hip_check(launch_gemm(EPI_BIAS, p, nullptr), "launch_gemm(projection table)");
         src = p.Y;
       }
-      hip_check(launch_row_rms(src, Hc, Vc, Hc, cd.eps, inv, nullptr), "launch_row_rms(table)");
       GemmArgs q{};
-      q.X = src; q.ldx = Hc; q.row_scale = inv; q.gamma = e.cp.layers[0].g_in; q.W = e.cp.layers[0].qkv;
+      q.X = src; q.ldx = Hc; q.gamma = e.cp.layers[0].g_in; q.eps = cd.eps; q.W = wq; q.w_packed = 1;
       q.Y = e.cp_qkv_table + (size_t)(g - 1) * Vc * Q; q.ldy = Q;
       q.M = Vc; q.N = Q; q.K = Hc;
       hip_check(launch_gemm(EPI_STORE, q, nullptr), "launch_gemm(q/k/v table)");
     }
     HIPC(hipDeviceSynchronize());
   } catch (...) {
-    (void)hipFree(X);
-    if (inv) (void)hipFree(inv);
+    release();
     throw;
   }
-  (void)hipFree(X);
-  (void)hipFree(inv);
+  release();
 }
 
 // Packed weight copies and T16 activations for the batched frame (engines with more than
@@ -1205,27 +1246,7 @@ void build_cp_tables(Engine &e) {
 void alloc_rows(Engine &e) {
   int64_t &t = e.device_bytes;
   const Dims &td = e.td, &cd = e.cd;
-  auto pack_stack = [&](StackW &w) {
-    const Dims &d = w.d;
-    const size_t per_layer = (size_t)d.qkv_rows() * d.hidden + (size_t)d.hidden * d.q_out() +
-                             (size_t)2 * d.intermediate * d.hidden + (size_t)d.hidden * d.intermediate;
-    w.mats_p = dev_alloc<uint16_t>(per_layer * d.layers, t);
-    for (LayerW &L : w.layers) {
-      auto at = [&](const uint16_t *m) { return w.mats_p + (m - w.mats); };
-      L.qkv_p = at(L.qkv);
-      L.o_p = at(L.o);
-      L.gu_p = at(L.gu);
-      L.down_p = at(L.down);
-      hip_check(launch_pack_weights(L.qkv, const_cast<uint16_t *>(L.qkv_p), d.qkv_rows(), d.hidden, nullptr), "pack");
-      hip_check(launch_pack_weights(L.o, const_cast<uint16_t *>(L.o_p), d.hidden, d.q_out(), nullptr), "pack");
-      hip_check(launch_pack_weights(L.gu, const_cast<uint16_t *>(L.gu_p), 2 * d.intermediate, d.hidden, nullptr),
-                "pack");
-      hip_check(launch_pack_weights(L.down, const_cast<uint16_t *>(L.down_p), d.hidden, d.intermediate, nullptr),
-                "pack");
-    }
-  };
-  pack_stack(e.talker);
-  pack_stack(e.cp);
+  pack_stack(e.cp, t);
   const int Ht = e.talker_hidden, Hc = cd.hidden, Vt = td.vocab, Vc = cd.vocab, nac = e.groups - 1;
   e.codec_head_p = dev_alloc<uint16_t>((size_t)Vt * Ht, t);
   hip_check(launch_pack_weights(e.codec_head, e.codec_head_p, Vt, Ht, nullptr), "pack");
@@ -1539,9 +1560,26 @@ int q3t_engine_create(const q3t_engine_options *opts, q3t_engine **out) {
       e->text_hidden = (int)ts[1];
       e->tp_inter = (int)f1[0];
       e->text_emb = upload_bf16({"talker.model.text_embedding.weight"}, ts);
-      e->tp_fc1 = upload_bf16({"talker.text_projection.linear_fc1.weight"}, f1);
+      auto upload_packed = [&](const std::string &n, const std::vector<int64_t> &shape) {
+        int64_t scratch = 0;
+        std::vector<uint16_t> host;
+        st.append_bf16(n, shape, host);
+        uint16_t *rows = dev_alloc<uint16_t>(host.size(), scratch);
+        uint16_t *packed = nullptr;
+        try {
+          HIPC(hipMemcpy(rows, host.data(), host.size() * 2, hipMemcpyHostToDevice));
+          packed = pack_weights(rows, (int)shape[0], (int)shape[1], tally);
+          HIPC(hipStreamSynchronize(nullptr));
+        } catch (...) {
+          (void)hipFree(rows);
+          throw;
+        }
+        (void)hipFree(rows);
+        return packed;
+      };
+      e->tp_fc1 = upload_packed("talker.text_projection.linear_fc1.weight", f1);
       e->tp_b1 = upload_f32("talker.text_projection.linear_fc1.bias", f1[0]);
-      e->tp_fc2 = upload_bf16({"talker.text_projection.linear_fc2.weight"}, f2);
+      e->tp_fc2 = upload_packed("talker.text_projection.linear_fc2.weight", f2);
       e->tp_b2 = upload_f32("talker.text_projection.linear_fc2.bias", Ht);
     }
     if (e->has_proj) {
@@ -1551,8 +1589,8 @@ int q3t_engine_create(const q3t_engine_options *opts, q3t_engine **out) {
     }
     try {
       alloc_pools(*e, nslots);
+      pack_stack(e->talker, tally);
       if (nslots > 1 && e->rows_ok) alloc_rows(*e);
-      e->split_ws = dev_alloc<float>((size_t)Engine::kSplitFloats, e->device_bytes);
       build_cp_tables(*e);
       e->codec = codec_load(dir, &e->device_bytes);
     } catch (...) {
@@ -1577,7 +1615,7 @@ int q3t_engine_destroy(q3t_engine *e) {
                     e->cp.mats_p,   e->codec_head_p, e->lm_heads_p,  e->proj_w_p,    e->bx_t,
                     e->bx_c,        e->battn,        e->bact,        e->bcp_in,      e->cp_qkv_table,
                     e->cp_in_table, e->text_emb,     e->tp_fc1,      e->tp_fc2,      e->tp_b1,
-                    e->tp_b2,       e->split_ws,    e->bmid,        e->bqkv2};
+                    e->tp_b2,       e->bmid,        e->bqkv2};
     for (void *p : ptrs)
       if (p) (void)hipFree(p);
     delete e;
@@ -1828,14 +1866,12 @@ void run_text_plan(Engine &e, const TextPlan &p, const TextWorkspace &w, float *
   hip_check(launch_text_gather(e.text_emb, e.text_hidden, ids, M, w.X, s), "launch_text_gather");
   GemmArgs g{};
   g.X = w.X; g.ldx = e.text_hidden; g.W = e.tp_fc1; g.bias = e.tp_b1; g.Y = w.Hd; g.ldy = e.tp_inter;
-  g.M = M; g.N = e.tp_inter; g.K = e.text_hidden;
-  g.split_ws = e.split_ws; g.split_cap = Engine::kSplitFloats;
+  g.M = M; g.N = e.tp_inter; g.K = e.text_hidden; g.w_packed = 1;
   hip_check(launch_gemm(EPI_BIAS, g, s), "launch_gemm(text fc1)");
   hip_check(launch_silu(w.Hd, (size_t)M * e.tp_inter, s), "launch_silu");
   g = GemmArgs{};
   g.X = w.Hd; g.ldx = e.tp_inter; g.W = e.tp_fc2; g.bias = e.tp_b2; g.Y = w.Y; g.ldy = H;
-  g.M = M; g.N = H; g.K = e.tp_inter;
-  g.split_ws = e.split_ws; g.split_cap = Engine::kSplitFloats;
+  g.M = M; g.N = H; g.K = e.tp_inter; g.w_packed = 1;
   hip_check(launch_gemm(EPI_BIAS, g, s), "launch_gemm(text fc2)");
   hip_check(launch_text_assemble(w.Y, H, M, codec, e.codec_emb, w.xvec, dst, prefill, trailing, pad, s),
             "launch_text_assemble");
@@ -2917,29 +2953,24 @@ int q3t_debug_gemm(q3t_engine *e, int32_t epi, const float *X, int32_t M, int32_
         for (void *p : owned) (void)hipFree(p);
         return;
       }
-      if (gemm_skinny_supports(M, K, gamma != nullptr)) {  // the batched-decode kernel (fused RMSNorm)
-        if (gamma) g.gamma = (const float *)up(gamma, (size_t)K * 4);
-        g.eps = eps;
-        // Packed weights in whole 16-column tiles: the last tile's missing rows are zeros.
-        if (N % 16 && epi == EPI_SWIGLU) fail(Q3T_ERR_INVALID, "the batched-decode SwiGLU GEMM needs N %% 16 == 0");
-        const size_t prows = (wrows + 15) / 16 * 16;
-        uint16_t *padded = (uint16_t *)up(nullptr, prows * K * 2);
-        HIPC(hipMemset(padded, 0, prows * K * 2));
-        HIPC(hipMemcpy(padded, g.W, wrows * K * 2, hipMemcpyDeviceToDevice));
-        uint16_t *packed = (uint16_t *)up(nullptr, prows * K * 2);
-        hip_check(launch_pack_weights(padded, packed, (int)prows, K, nullptr), "launch_pack_weights");
-        g.W = packed;
-        g.w_packed = 1;
-        hip_check(launch_gemm_skinny(epi, gamma != nullptr, g, nullptr), "launch_gemm_skinny");
-      } else {
-        if (gamma) {
-          g.gamma = (const float *)up(gamma, (size_t)K * 4);
-          float *inv = (float *)up(nullptr, (size_t)M * 4);
-          hip_check(launch_row_rms(g.X, K, M, K, eps, inv, nullptr), "launch_row_rms");
-          g.row_scale = inv;
-        }
-        hip_check(launch_gemm(epi, g, nullptr), "launch_gemm");
-      }
+      const bool skinny = gemm_skinny_supports(M, K, gamma != nullptr);  // the batched-decode kernel
+      if (skinny && N % 16 && epi == EPI_SWIGLU)
+        fail(Q3T_ERR_INVALID, "the batched-decode SwiGLU GEMM needs N %% 16 == 0");
+      if (gamma) g.gamma = (const float *)up(gamma, (size_t)K * 4);
+      g.eps = eps;
+      // Packed weights in whole 16-column tiles: the last tile's missing rows are zeros (SwiGLU:
+      // of the gate rows and of the up rows).
+      const size_t mats = epi == EPI_SWIGLU ? 2 : 1, prows = ((size_t)N + 15) / 16 * 16;
+      uint16_t *padded = (uint16_t *)up(nullptr, mats * prows * K * 2);
+      HIPC(hipMemset(padded, 0, mats * prows * K * 2));
+      for (size_t i = 0; i < mats; ++i)
+        HIPC(hipMemcpy(padded + i * prows * K, g.W + i * N * K, (size_t)N * K * 2, hipMemcpyDeviceToDevice));
+      uint16_t *packed = (uint16_t *)up(nullptr, mats * prows * K * 2);
+      hip_check(launch_pack_weights(padded, packed, (int)(mats * prows), K, nullptr), "launch_pack_weights");
+      g.W = packed;
+      g.w_packed = 1;
+      if (skinny) hip_check(launch_gemm_skinny(epi, gamma != nullptr, g, nullptr), "launch_gemm_skinny");
+      else hip_check(launch_gemm(epi, g, nullptr), "launch_gemm");
       HIPC(hipMemcpy(Y, g.Y, (size_t)M * N * 4, hipMemcpyDeviceToHost));
     } catch (...) {
       for (void *p : owned) (void)hipFree(p);

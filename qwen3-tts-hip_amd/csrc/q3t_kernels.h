@@ -62,11 +62,14 @@ int attn_chunks(int cap);
 // launch_attn_merge merges: 32 up to a 2,048-row cache, then 64 and 128.
 int attn_rows_chunk_len(int cap);
 
-// Matrix-core GEMM (bf16 weights, fp32 activations split into three bf16 terms, fp32 accumulate)
-// for many rows: prompt prefill and batched decode.  Requires K % 32 == 0.
+// Matrix-core GEMM (packed bf16 weights, fp32 activations split into three bf16 terms, fp32
+// accumulate) for many rows (q3t_gemm.hip): prompt prefill, text projection, codec linears.
+// Requires K % 32 == 0, ldx % 4 == 0, 16-byte aligned X, W, gamma.
 hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t stream);
+// GemmArgs::split2 (EPI_RESIDUAL without RMSNorm): up to kGemmSplitRows rows.
+constexpr int kGemmSplitRows = 64;
 // The same product for M <= 16 rows (batched decode); norm = fused RMSNorm of the rows with
-// gain gamma (row_scale must be null).  Requires K = 512 * c, c in {1, 2, 3, 4, 6, 8, 12}
+// gain gamma.  Requires K = 512 * c, c in {1, 2, 3, 4, 6, 8, 12}
 // (K <= 2048 with norm).
 bool gemm_skinny_supports(int M, int K, bool norm);
 // GemmArgs::split2 (EPI_RESIDUAL, T16 X and Y): K = 1024 * c, c in {1, 2, 3, 4, 6}.
@@ -75,9 +78,6 @@ hipError_t launch_gemm_skinny(int epi, bool norm, const GemmArgs &a, hipStream_t
 // dst = src [rows][K] bf16 in the skinny GEMM's packed layout (GemmArgs::w_packed).
 // Requires rows % 16 == 0 and K % 32 == 0.
 hipError_t launch_pack_weights(const uint16_t *src, uint16_t *dst, int rows, int K, hipStream_t stream);
-// inv_rms[m] = 1 / sqrt(mean(X[m]^2) + eps).
-hipError_t launch_row_rms(const float *X, int ldx, int M, int K, float eps, float *inv_rms, hipStream_t stream);
-
 // Prompt preparation: X[m] = fp32(table[ids[m]]) ([M][width]); x = silu(x) in place; and row m
 // of Y ([M][H], + codec_emb[codec[m]] where codec[m] >= 0) to dst[m] = (kind << 24) | row with
 // kind 0 prefill row, 1 trailing row, 2 the tts_pad row, 3 dropped.  The host validates ids.

@@ -1381,15 +1381,11 @@ __global__ __launch_bounds__(128) void k_attn_merge(AttnMergeArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Y[M][N] = X[M][K] . W[N][K]^T on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16).
-// W is the bf16 weight as stored; X is fp32 and enters the matrix cores as three bf16 terms
-// (three MFMAs per k-block, smallest term first, fp32 accumulation).  Optional per-row scale
-// and per-column gain on X (the RMSNorm of the rows) are applied while converting.
-// Wave tile: (16 * MB) rows x (16 * NB) columns, no LDS: every lane loads its own A fragment
-// (8 consecutive k of one row, fp32) and B fragment (8 consecutive k of one weight row, bf16).
+// Y[M][N] = X[M][K] . W[N][K]^T on the bf16 matrix cores (v_mfma_f32_16x16x32_bf16), for the few
+// rows of a batched frame (many rows: q3t_gemm.hip).  X is fp32 and enters as three bf16 terms
+// (three MFMAs per k-block, smallest term first, fp32 accumulation).
 // Operand layouts of the 16x16x32 instruction: A[i][k] in lane i + 16 (k / 8), element k % 8;
 // B[k][j] in lane j + 16 (k / 8), element k % 8; C[i][j] in lane j + 16 (i / 4), element i % 4.
-// SwiGLU: the first NB/2 column tiles are gate rows, the last NB/2 the matching up rows.
 // ---------------------------------------------------------------------------------------
 // x = hi + mid + lo, each a bf16: 24 significant bits, so every product with a bf16 weight
 // is exact and the GEMM matches an fp32 GEMV up to the order of the fp32 additions.
@@ -1410,203 +1406,6 @@ __device__ __forceinline__ void split_bf16x8(const float *x, bf16x8_t &hi, bf16x
   }
 }
 
-// Offset of X element (m, k) in the matrix-core GEMMs (k a multiple of 4 inside one 32-wide
-// k step, which never straddles an X segment).
-__device__ __forceinline__ size_t gemm_x_offset(const GemmArgs &a, int m, int k) {
-  size_t o = (size_t)m * a.ldx;
-  if (a.xseg_len > 0) o += (size_t)(k / a.xseg_len) * a.xseg_stride + k % a.xseg_len;
-  else o += k;
-  return o;
-}
-
-// Epilogues of the matrix-core GEMMs for element (m, n) with accumulated value v (not SwiGLU).
-template <int EPI>
-__device__ __forceinline__ float gemm_epilogue(const GemmArgs &a, int m, int n, float v) {
-  if constexpr (EPI == EPI_RESIDUAL) v = a.res[(size_t)m * a.ldr + n] + v;
-  if constexpr (EPI == EPI_BIAS) v = v + a.bias[n];
-  if constexpr (EPI == EPI_AFFINE_RES) {
-    if (a.bias) v = v + a.bias[n];
-    if (a.scale) v = v * a.scale[n];
-    v = a.res[(size_t)m * a.ldr + n] + v;
-  }
-  if constexpr (EPI == EPI_BIAS_GELU) {
-    v = v + a.bias[n];
-    v = 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
-  }
-  if constexpr (EPI == EPI_RES_SNAKE) {
-    v = a.res[(size_t)m * a.ldr + n] + (v + a.bias[n]);
-    const float ea = a.snake_a[n], ib = a.snake_b[n];
-    snake_n<1>(&v, &ea, &ib);
-  }
-  return v;
-}
-
-// gemm_epilogue with its operands loaded beforehand: r = res[m][n], b = bias[n] (when
-// given), c = scale[n] (when given; the Snake form: c = snake_a[n], c2 = snake_b[n]); the same
-// arithmetic in the same order.
-template <int EPI>
-__device__ __forceinline__ float gemm_epilogue_ops(const GemmArgs &a, float v, float r, float b, float c, float c2) {
-  if constexpr (EPI == EPI_RESIDUAL) v = r + v;
-  if constexpr (EPI == EPI_BIAS) v = v + b;
-  if constexpr (EPI == EPI_AFFINE_RES) {
-    if (a.bias) v = v + b;
-    if (a.scale) v = v * c;
-    v = r + v;
-  }
-  if constexpr (EPI == EPI_BIAS_GELU) {
-    v = v + b;
-    v = 0.5f * v * (1.0f + erff(v * 0.7071067811865476f));
-  }
-  if constexpr (EPI == EPI_RES_SNAKE) {
-    v = r + (v + b);
-    snake_n<1>(&v, &c, &c2);
-  }
-  return v;
-}
-
-template <int EPI, int MB, int NB>
-__global__ __launch_bounds__(256) void k_gemm_mfma(GemmArgs a) {
-  const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int li = lane & 15;   // row (A) / column (B, C) within a 16-tile
-  const int kb = lane >> 4;   // k-block of 8 within the 32-wide k step
-  constexpr int NTILE = (EPI == EPI_SWIGLU) ? NB / 2 : NB;  // output column tiles
-  const int m0 = blockIdx.y * 16 * MB;
-  const int n0 = (blockIdx.x * 4 + wave) * 16 * NTILE;  // first output column of this wave
-  if (n0 >= a.N) return;
-  // split z of gridDim.z: k steps [kt0, kt1) of 32
-  const int KT = a.K / 32, nsplit = gridDim.z, z = blockIdx.z;
-  const int kt0 = (int)((int64_t)KT * z / nsplit), kt1 = (int)((int64_t)KT * (z + 1) / nsplit);
-
-  f32x4_t acc[MB][NB];
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < NB; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  // rows / weight rows this lane feeds (clamped into range; padding results are not stored)
-  int arow[MB];
-  float rscale[MB];
-#pragma unroll
-  for (int i = 0; i < MB; ++i) {
-    arow[i] = min(m0 + 16 * i + li, a.M - 1);
-    rscale[i] = a.row_scale ? a.row_scale[arow[i]] : 1.f;
-  }
-  int wrow[NB];
-#pragma unroll
-  for (int j = 0; j < NB; ++j) {
-    int col;
-    if constexpr (EPI == EPI_SWIGLU)
-      col = (j < NTILE) ? n0 + 16 * j + li : a.N + n0 + 16 * (j - NTILE) + li;
-    else
-      col = n0 + 16 * j + li;
-    const int lim = (EPI == EPI_SWIGLU) ? 2 * a.N : a.N;
-    wrow[j] = min(col, lim - 1);
-  }
-
-  for (int k0 = kt0 * 32; k0 < kt1 * 32; k0 += 32) {
-    const int k = k0 + 8 * kb;
-    float xa[MB][8];
-#pragma unroll
-    for (int i = 0; i < MB; ++i) {
-      const float4 *px = reinterpret_cast<const float4 *>(a.X + gemm_x_offset(a, arow[i], k));
-      const float4 p0 = px[0], p1 = px[1];
-      xa[i][0] = p0.x; xa[i][1] = p0.y; xa[i][2] = p0.z; xa[i][3] = p0.w;
-      xa[i][4] = p1.x; xa[i][5] = p1.y; xa[i][6] = p1.z; xa[i][7] = p1.w;
-    }
-    uint4 wb[NB];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) wb[j] = *reinterpret_cast<const uint4 *>(a.W + (size_t)wrow[j] * a.K + k);
-    float g[8];
-    if (a.gamma) {
-      const float4 *pg = reinterpret_cast<const float4 *>(a.gamma + k);
-      const float4 g0 = pg[0], g1 = pg[1];
-      g[0] = g0.x; g[1] = g0.y; g[2] = g0.z; g[3] = g0.w; g[4] = g1.x; g[5] = g1.y; g[6] = g1.z; g[7] = g1.w;
-    }
-    bf16x8_t ahi[MB], amid[MB], alo[MB];
-#pragma unroll
-    for (int i = 0; i < MB; ++i) {
-      if (a.gamma) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xa[i][e] = (xa[i][e] * rscale[i]) * g[e];
-      } else if (a.row_scale) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xa[i][e] = xa[i][e] * rscale[i];
-      }
-      split_bf16x8(xa[i], ahi[i], amid[i], alo[i]);
-    }
-    // term-major (lo, mid, hi over all tiles): independent accumulations between two that depend
-    // on each other
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(alo[i], __builtin_bit_cast(bf16x8_t, wb[j]), acc[i][j], 0, 0, 0);
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(amid[i], __builtin_bit_cast(bf16x8_t, wb[j]), acc[i][j], 0, 0, 0);
-#pragma unroll
-    for (int j = 0; j < NB; ++j)
-#pragma unroll
-      for (int i = 0; i < MB; ++i)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ahi[i], __builtin_bit_cast(bf16x8_t, wb[j]), acc[i][j], 0, 0, 0);
-  }
-
-  // epilogue: lane holds C[4 * kb + e][li] of every tile
-  // The epilogue's operands are loaded before the first store (Y may be the residual itself:
-  // a load after a store that may alias it would wait for that store).
-  constexpr bool RES = EPI == EPI_RESIDUAL || EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE;
-  constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU || EPI == EPI_RES_SNAKE;
-  constexpr bool OPS = RES || BIAS;
-  float rv[OPS ? MB : 1][OPS ? NTILE : 1][4], bv[OPS ? NTILE : 1], cv[OPS ? NTILE : 1], c2v[OPS ? NTILE : 1];
-  if constexpr (OPS) {
-    if (nsplit == 1) {
-#pragma unroll
-      for (int j = 0; j < NTILE; ++j) {
-        const int nc = min(n0 + 16 * j + li, a.N - 1);
-        bv[j] = (BIAS && (EPI != EPI_AFFINE_RES || a.bias)) ? a.bias[nc] : 0.f;
-        cv[j] = (EPI == EPI_AFFINE_RES && a.scale) ? a.scale[nc] : (EPI == EPI_RES_SNAKE ? a.snake_a[nc] : 1.f);
-        c2v[j] = EPI == EPI_RES_SNAKE ? a.snake_b[nc] : 1.f;
-#pragma unroll
-        for (int i = 0; i < MB; ++i)
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            rv[i][j][e] = RES ? a.res[(size_t)min(m0 + 16 * i + 4 * kb + e, a.M - 1) * a.ldr + nc] : 0.f;
-      }
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < MB; ++i)
-#pragma unroll
-    for (int j = 0; j < NTILE; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = m0 + 16 * i + 4 * kb + e;
-        const int n = n0 + 16 * j + li;
-        if (m >= a.M || n >= a.N) continue;
-        float v = acc[i][j][e];
-        if constexpr (EPI == EPI_SWIGLU) {
-          const float u = acc[i][j + NTILE][e];
-          if (nsplit > 1) {  // raw gate and up sums: [split][M][2N], up at N + n
-            float *w = a.split_ws + ((size_t)z * a.M + m) * 2 * a.N;
-            w[n] = v;
-            w[a.N + n] = u;
-            continue;
-          }
-          v = v / (1.0f + expf(-v)) * u;
-        } else {
-          if (nsplit > 1) {
-            a.split_ws[((size_t)z * a.M + m) * a.N + n] = v;
-            continue;
-          }
-          if constexpr (OPS) v = gemm_epilogue_ops<EPI>(a, v, rv[i][j][e], bv[j], cv[j], c2v[j]);
-        }
-        a.Y[(size_t)m * a.ldy + n] = v;
-      }
-}
-
 // ---------------------------------------------------------------------------------------
 // Skinny GEMM for M <= 16 rows (one row per stream in batched decode): one 1024-thread
 // workgroup per 16-column output tile (a gate tile + up tile pair for SwiGLU); its 16 waves
@@ -1615,267 +1414,6 @@ __global__ __launch_bounds__(256) void k_gemm_mfma(GemmArgs a) {
 // NORM the rows' RMSNorm is computed from the same loads (sum of squares reduced across the
 // workgroup) and applied before the split.
 // ---------------------------------------------------------------------------------------
-// ---------------------------------------------------------------------------------------
-// Prefill GEMM, LDS-tiled: Y[M][N] = f(X)[M][K] . W[N][K]^T for many rows.
-// Block tile 128 rows x 128 weight rows, k step 32; four waves, each 32 rows x 128 weight rows
-// (2 x 8 tiles of v_mfma_f32_16x16x32_bf16), two blocks per CU.  Each wave's X rows are its
-// own: it loads them from global memory in matrix-core fragment order, scales them by the
-// row's 1/rms and the gain, and splits them in registers into the hi/mid/lo bf16 terms of
-// k_gemm_mfma.  Only the weight tile, shared by the four waves, goes through LDS (double
-// buffered, in fragment order: conflict-free 16-byte reads).  Global loads of the next k step
-// are in flight while the matrix cores work on this one.  SwiGLU blocks hold 64 gate rows and
-// the matching 64 up rows (64 outputs).  Requires K % 32 == 0 (and N % 64 == 0 for SwiGLU); a
-// partial last block of columns computes clamped weight rows and stores only columns below N.
-// XS: bit 0 = GemmArgs::row_scale given, bit 1 = gamma given (compile-time, so that the k
-// loop is one basic block).  BW = 96 (not SwiGLU): 96-column blocks, for N a multiple of 96
-// but not of 128 (the codec's 96- and 192-channel convolutions), where 128-column blocks
-// would leave a quarter of the matrix-core work on padding columns.
-// ---------------------------------------------------------------------------------------
-template <int EPI, int XS, int BW = 128>
-__global__ __launch_bounds__(256, 2) void k_gemm_lds(GemmArgs a) {
-  constexpr int BM = 128, BK = 32;
-  constexpr bool SW = EPI == EPI_SWIGLU;
-  static_assert(BW == 128 || (BW == 96 && !SW), "column block");
-  constexpr int NU = BW / 16;  // 16-column tiles per block
-  constexpr bool RS = XS & 1, GM = XS & 2;
-  // weight tile u (rows 16 u .. 16 u + 15 of the block) at Bs[buf][u]; lane li + 16 kb reads
-  // row 16 u + li, k = 8 kb .. 8 kb + 7, from entry 16 kb + (li ^ 4 kb).  The xor spreads the
-  // stores (four lanes of one row, k = 0 .. 31, see below) over distinct banks while every 16
-  // lanes of a read still cover all 16 bank groups.
-  __shared__ bf16x8_t Bs[2][BW / 16][64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, kb = lane >> 4;
-  // Block tile (mb, nb).  Workgroups go to the 8 XCDs round robin (linear id % 8), each with its
-  // own L2.  With few column blocks (gridDim.x <= 8) that would send every row block of one
-  // column block to the same XCD, which would then read all of X; instead each XCD takes a
-  // contiguous range of row-major tiles (all column blocks of its row blocks), so its L2 reads
-  // only its own X rows, once for all column blocks.
-  int mb = blockIdx.y, nb = blockIdx.x;
-  if (gridDim.x <= 8) {
-    const int total = gridDim.x * gridDim.y, L = blockIdx.y * gridDim.x + blockIdx.x;
-    const int xcd = L % 8, local = L / 8, C = (total + 7) / 8, r = total % 8;
-    const int t = (r == 0 || xcd < r) ? xcd * C + local : r * C + (xcd - r) * (C - 1) + local;
-    mb = t / gridDim.x;
-    nb = t % gridDim.x;
-  }
-  const int m0 = mb * BM + wave * 32;  // this wave's rows m0 .. m0 + 31
-  // split z of gridDim.z: k tiles [kt0, kt1)
-  const int KT = a.K / BK, nsplit = gridDim.z, z = blockIdx.z;
-  const int kt0 = (int)((int64_t)KT * z / nsplit), kt1 = (int)((int64_t)KT * (z + 1) / nsplit);
-
-  // weight row of block row r (a partial last block of a non-SwiGLU GEMM repeats the last row;
-  // its columns are not stored)
-  auto wrow = [&](int r) -> int {
-    if constexpr (SW) return r < 64 ? nb * 64 + r : a.N + nb * 64 + (r - 64);
-    else return min(nb * BW + r, a.N - 1);
-  };
-  // X: lane (li, kb) reads rows m0 + 16 t + li, k = 8 kb .. 8 kb + 7 (two float4 per tile t).
-  // W: thread tid reads block rows (tid + 256 i) / 4, k = 8 ((tid + 256 i) % 4) .. + 7 (four
-  // consecutive lanes read one row's 64 contiguous bytes).
-  // NCH 16-byte weight chunks per k step, NB per thread (the last one partial for BW = 96)
-  constexpr int NCH = BW * BK / 8, NB = (NCH + 255) / 256, CB = BK / 8;
-  const float *xp[2];
-  float rs[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int m = min(m0 + 16 * t + li, a.M - 1);
-    xp[t] = a.X + (size_t)m * a.ldx + 8 * kb;
-    rs[t] = RS ? a.row_scale[m] : 1.0f;
-  }
-  const uint16_t *wp[NB];
-#pragma unroll
-  for (int i = 0; i < NB; ++i) {
-    const int idx = tid + 256 * i, row = idx / CB, c = idx % CB;
-    wp[i] = a.W + (size_t)wrow(row) * a.K + 8 * c;
-  }
-  const float *gp = GM ? a.gamma + 8 * kb : nullptr;
-  // X offset of the current k step and the k left in its segment (X rows in segments of
-  // xseg_len, xseg_stride apart; a 32-wide step never straddles two): advanced per step
-  int xk, xleft;
-  {
-    const int k = kt0 * BK;
-    if (a.xseg_len > 0) {
-      xk = (k / a.xseg_len) * a.xseg_stride + k % a.xseg_len;
-      xleft = a.xseg_len - k % a.xseg_len;
-    } else {
-      xk = k;
-      xleft = 1 << 30;
-    }
-  }
-  float4 rx[2][2];  // X of the loaded step, [tile][half]
-  float4 rg[2];     // gain of the loaded step
-  bf16x8_t rb[NB];  // a native vector (a uint4 struct copy stays a memcpy through scratch in the IR)
-  auto gload = [&](int k0) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) rx[t][h] = *reinterpret_cast<const float4 *>(xp[t] + xk + 4 * h);
-    if constexpr (GM) {
-      rg[0] = *reinterpret_cast<const float4 *>(gp + k0);
-      rg[1] = *reinterpret_cast<const float4 *>(gp + k0 + 4);
-    }
-#pragma unroll
-    for (int i = 0; i < NB; ++i)
-      if (NCH % 256 == 0 || tid + 256 * i < NCH) rb[i] = *reinterpret_cast<const bf16x8_t *>(wp[i] + k0);
-    const bool wrap = xleft == BK;
-    xk += wrap ? BK + a.xseg_stride - a.xseg_len : BK;
-    xleft = wrap ? a.xseg_len : xleft - BK;
-  };
-  bf16x8_t aq[3][2];  // [lo, mid, hi][tile] of the step the matrix cores work on next
-  auto split = [&]() {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      float xv[8] = {rx[t][0].x, rx[t][0].y, rx[t][0].z, rx[t][0].w,
-                     rx[t][1].x, rx[t][1].y, rx[t][1].z, rx[t][1].w};
-      if constexpr (RS) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xv[e] *= rs[t];
-      }
-      if constexpr (GM) {
-        const float gv[8] = {rg[0].x, rg[0].y, rg[0].z, rg[0].w, rg[1].x, rg[1].y, rg[1].z, rg[1].w};
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xv[e] *= gv[e];
-      }
-      split_bf16x8_nc(xv, aq[2][t], aq[1][t], aq[0][t]);
-    }
-  };
-  auto bstore = [&](int buf) {
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-      const int idx = tid + 256 * i, row = idx / CB, c = idx % CB;
-      if (NCH % 256 == 0 || idx < NCH) Bs[buf][row >> 4][16 * c + ((row & 15) ^ (4 * c))] = rb[i];
-    }
-  };
-
-  f32x4_t acc[2][NU];
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int u = 0; u < NU; ++u) acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  auto mma = [&](int buf) {
-    bf16x8_t bq[NU];
-#pragma unroll
-    for (int u = 0; u < NU; ++u) bq[u] = Bs[buf][u][16 * kb + (li ^ (4 * kb))];
-    // term-major: 16 independent accumulations between two that depend on each other;
-    // each accumulator still adds lo, mid, hi in that order.
-#pragma unroll
-    for (int q = 0; q < 3; ++q)
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int u = 0; u < NU; ++u)
-          acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aq[q][t], bq[u], acc[t][u], 0, 0, 0);
-  };
-
-  gload(kt0 * BK);
-  split();
-  bstore(0);
-  __syncthreads();
-  // all but the last k step: load the next step's operands, multiply this one, split and store
-  // the next
-  int buf = 0;
-  for (int kt = kt0; kt < kt1 - 1; ++kt) {
-    // without the fences the scheduler sinks the loads among the MFMAs and waits for them there
-    gload((kt + 1) * BK);
-    __builtin_amdgcn_sched_barrier(0);
-    mma(buf);
-    __builtin_amdgcn_sched_barrier(0);
-    split();
-    bstore(buf ^ 1);
-    __syncthreads();
-    buf ^= 1;
-  }
-  mma(buf);
-
-  // C[i][j] of a tile sits in lane j + 16 (i / 4), element i % 4.
-#pragma unroll
-  for (int t = 0; t < 2; ++t)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int m = m0 + t * 16 + 4 * kb + e;
-      if (m >= a.M) continue;
-      if constexpr (SW) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const int n = nb * 64 + u * 16 + li;
-          const float g = acc[t][u][e], up = acc[t][u + 4][e];
-          if (nsplit > 1) {  // raw gate and up sums: [split][M][2N], up at N + n
-            float *w = a.split_ws + ((size_t)z * a.M + m) * 2 * a.N;
-            w[n] = g;
-            w[a.N + n] = up;
-          } else {
-            a.Y[(size_t)m * a.ldy + n] = g / (1.0f + expf(-g)) * up;
-          }
-        }
-      } else if (nsplit > 1) {
-#pragma unroll
-        for (int u = 0; u < NU; ++u) {
-          const int n = nb * BW + u * 16 + li;
-          if (n < a.N) a.split_ws[((size_t)z * a.M + m) * a.N + n] = acc[t][u][e];
-        }
-      }
-    }
-  if constexpr (!SW) {
-    if (nsplit > 1) return;
-    // Every epilogue operand is loaded before the first store: Y may be the residual itself
-    // (each element read and written by this lane only), and a load after a store that may
-    // alias it would wait for that store, one memory round trip per element.
-    constexpr bool RES = EPI == EPI_RESIDUAL || EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE;
-    constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU || EPI == EPI_RES_SNAKE;
-    constexpr bool SCALE = EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE;
-    float rv[2][4][RES ? NU : 1], bv[BIAS ? NU : 1], cv[SCALE ? NU : 1], c2v[EPI == EPI_RES_SNAKE ? NU : 1];
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      const int nc = min(nb * BW + u * 16 + li, a.N - 1);
-      if constexpr (BIAS) bv[u] = (EPI != EPI_AFFINE_RES || a.bias) ? a.bias[nc] : 0.f;
-      if constexpr (EPI == EPI_AFFINE_RES) cv[u] = a.scale ? a.scale[nc] : 1.f;
-      if constexpr (EPI == EPI_RES_SNAKE) {
-        cv[u] = a.snake_a[nc];
-        c2v[u] = a.snake_b[nc];
-      }
-    }
-    if constexpr (RES) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int u = 0; u < NU; ++u) {
-            const int mc = min(m0 + t * 16 + 4 * kb + e, a.M - 1), nc = min(nb * BW + u * 16 + li, a.N - 1);
-            rv[t][e][u] = a.res[(size_t)mc * a.ldr + nc];
-          }
-    }
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int m = m0 + t * 16 + 4 * kb + e;
-        if (m >= a.M) continue;
-        if constexpr (EPI == EPI_RES_SNAKE) {  // one row's column tiles through the Snake together
-          float v[NU];
-#pragma unroll
-          for (int u = 0; u < NU; ++u) v[u] = rv[t][e][u] + (acc[t][u][e] + bv[u]);
-          snake_n<NU>(v, cv, c2v);
-#pragma unroll
-          for (int u = 0; u < NU; ++u) {
-            const int n = nb * BW + u * 16 + li;
-            if (n < a.N) a.Y[(size_t)m * a.ldy + n] = v[u];
-          }
-          continue;
-        }
-#pragma unroll
-        for (int u = 0; u < NU; ++u) {
-          const int n = nb * BW + u * 16 + li;
-          if (n >= a.N) continue;
-          a.Y[(size_t)m * a.ldy + n] = gemm_epilogue_ops<EPI>(a, acc[t][u][e], RES ? rv[t][e][RES ? u : 0] : 0.f,
-                                                              BIAS ? bv[BIAS ? u : 0] : 0.f,
-                                                              SCALE ? cv[SCALE ? u : 0] : 1.f,
-                                                              EPI == EPI_RES_SNAKE ? c2v[EPI == EPI_RES_SNAKE ? u : 0] : 1.f);
-        }
-      }
-  }
-}
-
 // KEYS (EPI_STORE): store per-row argmax keys (GemmArgs::keys_out) instead of Y.  XT16: X is
 // a T16 block (else row-major with leading dimension ldx).  W is always in k_pack_w's layout,
 // in whole 16-column tiles (the last one padded).
@@ -2061,17 +1599,6 @@ __global__ __launch_bounds__(1024) void k_gemm_skinny(GemmArgs a) {
     y = (EPI == EPI_RESIDUAL) ? oadd + y : y + oadd;
   }
   a.Y[a.y_t16 ? (size_t)ob * 16 * a.N + t16_index(om, on) : (size_t)om * a.ldy + (size_t)ob * a.y_blk + on] = y;
-}
-
-// inv_rms[m] = 1 / sqrt(mean(X[m]^2) + eps), one wave per row.
-__global__ __launch_bounds__(256) void k_row_rms(const float *X, int ldx, int M, int K, float eps, float *inv_rms) {
-  const int lane = threadIdx.x & 63;
-  const int m = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (m >= M) return;
-  float ss = 0.f;
-  for (int k = lane; k < K; k += 64) ss = fmaf(X[(size_t)m * ldx + k], X[(size_t)m * ldx + k], ss);
-  ss = wave_sum(ss);
-  if (lane == 0) inv_rms[m] = 1.0f / sqrtf(ss / (float)K + eps);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -3399,95 +2926,6 @@ hipError_t launch_attn_oproj(const AttnArgs &a, int head_dim, hipStream_t s, con
   return hipGetLastError();
 }
 
-// Sum of the K splits in split order, then the epilogue: Y[m][n] = f(sum_z ws[z][m][n])
-// (SwiGLU: silu(sum_z gate) * sum_z up).
-template <int EPI>
-__global__ __launch_bounds__(256) void k_gemm_split_reduce(GemmArgs a, int nsplit) {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  const size_t mn = (size_t)a.M * a.N;
-  if (i >= mn) return;
-  const int m = (int)(i / a.N), n = (int)(i % a.N);
-  if constexpr (EPI == EPI_SWIGLU) {  // gate and up sums, each added in split order
-    const size_t gi = (size_t)m * 2 * a.N + n;
-    float g = a.split_ws[gi], u = a.split_ws[gi + a.N];
-    for (int z = 1; z < nsplit; ++z) {
-      g += a.split_ws[(size_t)z * 2 * mn + gi];
-      u += a.split_ws[(size_t)z * 2 * mn + gi + a.N];
-    }
-    a.Y[(size_t)m * a.ldy + n] = g / (1.0f + expf(-g)) * u;
-    return;
-  }
-  float v = a.split_ws[i];
-  for (int z = 1; z < nsplit; ++z) v += a.split_ws[(size_t)z * mn + i];
-  a.Y[(size_t)m * a.ldy + n] = gemm_epilogue<EPI>(a, m, n, v);
-}
-
-// K splits for a launch of `blocks` workgroups: enough to reach ~256 workgroups, at least
-// 4 k steps of 32 per split, at most 16 splits, within the workspace.
-static int gemm_splits(const GemmArgs &a, int blocks, bool swiglu) {
-  if (!a.split_ws || blocks >= 128) return 1;
-  int sp = std::min(std::min((256 + blocks - 1) / blocks, a.K / 32 / 4), 16);
-  // SwiGLU keeps the gate and the up sums apart until the reduction
-  while (sp > 1 && (int64_t)sp * a.M * a.N * (swiglu ? 2 : 1) > a.split_cap) --sp;
-  return std::max(sp, 1);
-}
-
-template <int EPI>
-static hipError_t gemm_epi(const GemmArgs &a, hipStream_t s) {
-  // 16-row tiles for short M (batched decode), 32-row tiles otherwise; 64 output columns
-  // per wave (2 x 32 for SwiGLU gate/up pairs).
-  constexpr int NB = 4;
-  constexpr int NT = (EPI == EPI_SWIGLU) ? NB / 2 : NB;
-  const int cols_per_wg = 4 * 16 * NT;
-  dim3 grid;
-  int path;
-  // 96-column blocks where N is a multiple of 96 but not of 128
-  const bool bw96 = EPI != EPI_SWIGLU && a.N % 128 != 0 && a.N % 96 == 0;
-  if (a.M >= 128 && a.K % 32 == 0 && (EPI != EPI_SWIGLU || a.N % 64 == 0) && a.ldx % 4 == 0) {
-    const int nout = EPI == EPI_SWIGLU ? 64 : (bw96 ? 96 : 128);
-    grid = dim3((a.N + nout - 1) / nout, (a.M + 127) / 128);
-    path = 0;
-  } else if (a.M <= 16) {
-    grid = dim3((a.N + cols_per_wg - 1) / cols_per_wg, (a.M + 15) / 16);
-    path = 1;
-  } else {
-    grid = dim3((a.N + cols_per_wg - 1) / cols_per_wg, (a.M + 31) / 32);
-    path = 2;
-  }
-  grid.z = gemm_splits(a, (int)(grid.x * grid.y), EPI == EPI_SWIGLU);
-  if (path == 0) {
-    const int xs = (a.row_scale ? 1 : 0) | (a.gamma ? 2 : 0);
-    bool launched = false;
-    if constexpr (EPI != EPI_SWIGLU) {
-      if (bw96) {
-        switch (xs) {
-          case 0: hipLaunchKernelGGL((k_gemm_lds<EPI, 0, 96>), grid, dim3(256), 0, s, a); break;
-          case 1: hipLaunchKernelGGL((k_gemm_lds<EPI, 1, 96>), grid, dim3(256), 0, s, a); break;
-          case 2: hipLaunchKernelGGL((k_gemm_lds<EPI, 2, 96>), grid, dim3(256), 0, s, a); break;
-          default: hipLaunchKernelGGL((k_gemm_lds<EPI, 3, 96>), grid, dim3(256), 0, s, a); break;
-        }
-        launched = true;
-      }
-    }
-    if (!launched) {
-      switch (xs) {
-        case 0: hipLaunchKernelGGL((k_gemm_lds<EPI, 0>), grid, dim3(256), 0, s, a); break;
-        case 1: hipLaunchKernelGGL((k_gemm_lds<EPI, 1>), grid, dim3(256), 0, s, a); break;
-        case 2: hipLaunchKernelGGL((k_gemm_lds<EPI, 2>), grid, dim3(256), 0, s, a); break;
-        default: hipLaunchKernelGGL((k_gemm_lds<EPI, 3>), grid, dim3(256), 0, s, a); break;
-      }
-    }
-  }
-  else if (path == 1) hipLaunchKernelGGL((k_gemm_mfma<EPI, 1, NB>), grid, dim3(256), 0, s, a);
-  else hipLaunchKernelGGL((k_gemm_mfma<EPI, 2, NB>), grid, dim3(256), 0, s, a);
-  if (grid.z > 1) {
-    const size_t mn = (size_t)a.M * a.N;
-    hipLaunchKernelGGL((k_gemm_split_reduce<EPI>), dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, a,
-                       (int)grid.z);
-  }
-  return hipGetLastError();
-}
-
 template <int EPI, bool NORM, bool XT16, bool WNT>
 static hipError_t skinny_ks(const GemmArgs &a, hipStream_t s) {
   const dim3 grid((a.N + 15) / 16), block(1024);
@@ -3577,7 +3015,7 @@ bool gemm_skinny_supports(int M, int K, bool norm) {
 }
 
 hipError_t launch_gemm_skinny(int epi, bool norm, const GemmArgs &a, hipStream_t s) {
-  if (!gemm_skinny_supports(a.M, a.K, norm) || a.N <= 0 || a.ldx % 4 || (norm && (!a.gamma || a.row_scale)))
+  if (!gemm_skinny_supports(a.M, a.K, norm) || a.N <= 0 || a.ldx % 4 || (norm && !a.gamma))
     return hipErrorInvalidValue;
   // T16 output / residual needs N % 32 (whole k steps).  The weights must be packed
   // (launch_pack_weights) in whole 16-column tiles, the last one padded; SwiGLU's up tiles
@@ -3612,23 +3050,6 @@ hipError_t launch_pack_weights(const uint16_t *src, uint16_t *dst, int rows, int
   return hipGetLastError();
 }
 
-hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
-  if (a.M <= 0 || a.N <= 0 || a.K <= 0 || a.K % 32 || a.ldx % 4) return hipErrorInvalidValue;
-  if (a.xseg_len && (a.xseg_len < 0 || a.xseg_len % 32 || a.K % a.xseg_len || a.xseg_stride % 4))
-    return hipErrorInvalidValue;
-  switch (epi) {
-    case EPI_STORE: return gemm_epi<EPI_STORE>(a, s);
-    case EPI_RESIDUAL: return gemm_epi<EPI_RESIDUAL>(a, s);
-    case EPI_SWIGLU: return gemm_epi<EPI_SWIGLU>(a, s);
-    case EPI_BIAS: return gemm_epi<EPI_BIAS>(a, s);
-    case EPI_AFFINE_RES: return a.res ? gemm_epi<EPI_AFFINE_RES>(a, s) : hipErrorInvalidValue;
-    case EPI_RES_SNAKE:
-      return a.res && a.bias && a.snake_a && a.snake_b ? gemm_epi<EPI_RES_SNAKE>(a, s) : hipErrorInvalidValue;
-    case EPI_BIAS_GELU: return a.bias ? gemm_epi<EPI_BIAS_GELU>(a, s) : hipErrorInvalidValue;
-  }
-  return hipErrorInvalidValue;
-}
-
 hipError_t launch_text_gather(const uint16_t *table, int width, const int32_t *ids, int M, float *X, hipStream_t s) {
   if (M <= 0 || width <= 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_text_gather, dim3(M), dim3(256), 0, s, table, width, ids, X);
@@ -3653,12 +3074,6 @@ hipError_t launch_text_assemble(const float *Y, int H, int M, const int32_t *cod
 hipError_t launch_bf16_to_f32(const uint16_t *src, float *dst, size_t n, hipStream_t s) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_bf16_to_f32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, src, dst, n);
-  return hipGetLastError();
-}
-
-hipError_t launch_row_rms(const float *X, int ldx, int M, int K, float eps, float *inv_rms, hipStream_t s) {
-  if (M <= 0 || K <= 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_row_rms, dim3((M + 3) / 4), dim3(256), 0, s, X, ldx, M, K, eps, inv_rms);
   return hipGetLastError();
 }
 

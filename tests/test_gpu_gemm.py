@@ -149,3 +149,36 @@ def test_prefill_tiles_all_epilogues(eng, M, K):
     _close(eng.debug_gemm(3, X, Wb[:N], N, bias=bias), X.astype(np.float64) @ W[:N].T + bias)
     gate, up = Xn @ W[:N].T, Xn @ W[N:].T
     _close(eng.debug_gemm(2, X, Wb, N, gamma=g), gate / (1 + np.exp(-gate)) * up)
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 48, 49, 64, 65, 128, 129, 193])
+@pytest.mark.parametrize("K", [32, 96, 160, 1056])
+def test_row_and_step_remainders(eng, M, K):
+    """Rows around the 16-row tiles of the few-row kernel (up to 64) and the 64-row blocks of the
+    tiled one, k steps that do not fill a wave's share, a chunk or a pair of chunks, and a partial
+    last column tile: residual with RMSNorm, bias, SwiGLU.  The tolerance is the module's."""
+    N = 84
+    rng = np.random.default_rng(M * 5 + K)
+    X = (rng.standard_normal((M, K)) * 2).astype(np.float32)
+    g = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
+    Xn = X.astype(np.float64) / np.sqrt((X.astype(np.float64) ** 2).mean(1, keepdims=True) + 1e-6) * g
+    Wb = _weights(2 * N, K, M + K)
+    W = synth.bf16_bits_to_f32(Wb).astype(np.float64)
+    res = rng.standard_normal((M, N)).astype(np.float32)
+    bias = rng.standard_normal(N).astype(np.float32)
+    print(f"[gpu] gemm remainders M={M} K={K}", flush=True)
+    _close(eng.debug_gemm(1, X, Wb[:N], N, gamma=g, res=res), res + Xn @ W[:N].T)
+    _close(eng.debug_gemm(3, X, Wb[:N], N, bias=bias), X.astype(np.float64) @ W[:N].T + bias)
+    gate, up = Xn @ W[:N].T, Xn @ W[N:].T
+    _close(eng.debug_gemm(2, X, Wb, N, gamma=g), gate / (1 + np.exp(-gate)) * up)
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 8192, 512), (200, 4100, 512), (520, 2050, 256)])
+def test_wide_tiles(eng, M, N, K):
+    """Enough 128-column blocks for every CU (the one-group kernel's 128- and 64-row weight tiles),
+    N not a multiple of 4 among them."""
+    print(f"[gpu] gemm wide M={M} N={N} K={K}", flush=True)
+    rng = np.random.default_rng(M)
+    X = rng.standard_normal((M, K)).astype(np.float32)
+    Wb = _weights(N, K, N)
+    _close(eng.debug_gemm(0, X, Wb, N), X.astype(np.float64) @ synth.bf16_bits_to_f32(Wb).astype(np.float64).T)

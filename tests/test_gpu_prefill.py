@@ -59,3 +59,20 @@ def test_prefill_tiles_per_wave(models, kv_bf16):
             tol = (2e-3, 2e-4) if kv_bf16 else (1e-5, 1e-6)
             _close(hidden, o.hidden, *tol, f"P={P} hidden")
             _close(logits, want, *tol, f"P={P} logits")
+
+
+def test_prefill_split_sums_leave_no_trace(models):
+    """Prompts of at most 64 rows accumulate the O and down projections into buffers that each GEMM
+    leaves zeroed for the next: the same prompt before and after others, longer ones (which take the
+    unsplit kernels) among them, gives the same bits."""
+    model, d = models.get("tiny", 0)
+    rng = np.random.default_rng(13)
+    xs = [(rng.standard_normal((P, model.spec.talker.hidden)) * 0.5).astype(np.float32) for P in (41, 64, 65, 3, 130)]
+    print("[gpu] prefill split sums", flush=True)
+    with E.HipTtsEngine(d, E.EngineOptions(max_cache_steps=CAP)) as eng:
+        first = [eng.debug_talker_prefill(x) for x in xs]
+        for x, (hidden, logits, token) in list(zip(xs, first))[::-1]:
+            h, l, t = eng.debug_talker_prefill(x)
+            np.testing.assert_array_equal(h, hidden)
+            np.testing.assert_array_equal(l, logits)
+            assert t == token
