@@ -34,16 +34,21 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, float *v, const
   if constexpr (EPI == EPI_RES_SNAKE) snake_n<4>(v, c, c2);
 }
 
-// Block tile 64 rows x BW packed weight rows (SwiGLU: BW / 2 gate rows and the matching up rows),
-// four waves as 2 x 2, per KG K group.  What bounds it where there are blocks for every CU is the
-// matrix cores (three MFMAs a product); with few blocks, the latency of one block's own chain of k
-// steps.  Hence:
+// Block tile 32 rows x 128 packed weight rows (SwiGLU: 64 gate rows and the matching up rows), four
+// waves side by side, per K group.  What bounds it: per CU, loading X and the weights (64 bytes a
+// clock) and splitting X (7 vector operations an element) take as long as the matrix cores do with
+// what is loaded (three MFMAs a product), so all three have to run at once, and a block's own chain
+// of k steps must never wait.  Hence:
 //   * Everything is loaded well ahead of use: the weights, straight from global memory in
-//     matrix-core order (1 KiB contiguous per 16 columns and step), in a ring of four k steps; X
-//     two 64-wide chunks ahead in registers.
+//     matrix-core order (1 KiB contiguous per 16 columns and step, read by one wave only), in a ring
+//     of four k steps; X two 64-wide chunks ahead in registers.  The loop is straight-line code with
+//     uniform addresses: a branch in it made the compiler copy the rings and wait for them.
 //   * X is split into its three terms once per block, into LDS planes of [step][row][4 slots of
 //     16 bytes], slots xor-ed with (row / 2) % 4 (any 8 rows of a slot in distinct bank columns),
 //     double buffered: one barrier per 64 k.
+//   * 32 rows rather than 64: 106-127 registers, four waves a SIMD from different blocks, so that one
+//     block's splitting runs under another's matrix-core work, and finer shares of the CUs.  521 rows,
+//     1024 -> 4096: 32 us (64 x 128 blocks) -> 25 us; 137 rows, 2048 -> 2 x 6144: 58 -> 35 us.
 //   * KG = 2: where blocks are few, two such groups of waves in a block take half of K each and add
 //     up through LDS.
 //   * RMSNorm needs no launch of its own: every block passes over its rows whole, so the staging
@@ -51,14 +56,17 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, float *v, const
 //     by 1 / rms (one scalar per row).
 //   * The weight tile is the A operand: a lane ends with four consecutive columns of one row, so
 //     loads and stores of the epilogue are 16 bytes wide.
-template <int EPI, bool NORM, int BW, int KG>
+//   * TAIL: K is not a whole number of pairs of chunks per group; what is missing is staged as zeros.
+template <int EPI, bool NORM, int KG, bool TAIL>
 __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) {
   constexpr bool SW = EPI == EPI_SWIGLU;
-  constexpr int RT = 2, CT = BW / 32, OT = SW ? CT / 2 : CT;  // row, weight and output tiles per wave
-  constexpr int BUF = 3 * 2 * 64 * 4;                         // 16-byte units of one staging buffer
-  extern __shared__ bf16x8_t lds[];                           // [KG][2][BUF], then row sums [KG][64]
-  const int grp = KG > 1 ? threadIdx.x >> 8 : 0, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;
-  const int li = lane & 15, kb = lane >> 4, wr = wave >> 1, wc = wave & 1;
+  constexpr int BM = 32, BW = 128;
+  constexpr int RT = 2, CT = 2, OT = SW ? 1 : 2;      // row, weight and output tiles per wave
+  constexpr int PLANE = 2 * BM * 4, BUF = 3 * PLANE;  // 16-byte units of a term, of a staging buffer
+  extern __shared__ bf16x8_t lds[];                   // [KG][2][BUF], then row sums [KG][64]
+  const int tid = threadIdx.x & 255, lane = tid & 63, li = lane & 15, kb = lane >> 4;
+  const int gwave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform for the compiler too
+  const int grp = KG > 1 ? gwave >> 2 : 0, wave = gwave & 3;
   bf16x8_t *xs = lds + grp * 2 * BUF;
   float *rsum = reinterpret_cast<float *>(lds + KG * 2 * BUF);
 
@@ -72,53 +80,56 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
     mb = t / gridDim.x;
     nb = t % gridDim.x;
   }
-  const int m0 = mb * 64;
-  const int n0 = nb * (SW ? BW / 2 : BW) + wc * OT * 16;  // this wave's first output column
+  const int m0 = mb * BM;
+  const int n0 = nb * (SW ? BW / 2 : BW) + wave * OT * 16;  // this wave's first output column
   // k steps [s0, s1) of 32 for this group, worked on in pairs of 64-wide chunks (four steps); what a
   // pair holds past s1 is staged as zeros
   const int steps = a.K / 32;
   const int s0 = (int)((int64_t)steps * grp / KG), s1 = (int)((int64_t)steps * (grp + 1) / KG);
   const int pairs = ((steps + KG - 1) / KG + 3) / 4;  // of the longest group: every wave meets every barrier
 
-  // X: this thread stages row tid / 4, k = 32 st + 8 (tid % 4) .. + 7 of a chunk's two steps st
-  const int srow = tid >> 2, slot = tid & 3;
-  const float *xp = a.X + (size_t)min(m0 + srow, a.M - 1) * a.ldx + 8 * slot;
-  const float *gp = NORM ? a.gamma + 8 * slot : nullptr;
-  f32x4_t xr[2][2][2], gr[NORM ? 2 : 1][2][2];  // [set][step][half]
+  // X: this thread stages row (tid % 128) / 4, k = 8 (tid % 4) .. + 7 of step tid / 128 of a chunk.
+  // Addresses are a uniform base (step) plus a 32-bit offset in the block.
+  const int srow = (tid & 127) >> 2, slot = tid & 3, sp = tid >> 7;
+  const float *xb = a.X + (size_t)m0 * a.ldx;
+  const uint32_t xo = (uint32_t)min(srow, a.M - 1 - m0) * (uint32_t)a.ldx + 8 * slot, go = 8 * slot;
+  f32x4_t xr[2][2], gr[NORM ? 2 : 1][2];  // [set][half]
   auto xload = [&](int st0, auto set) {
     constexpr int SET = decltype(set)::value;
+    const int st = min(st0, s1 - 1);
+    const uint32_t up = st0 + 1 < s1 ? 32u * (uint32_t)sp : 0u;  // the second step, if there is one
+    const float *xs0 = xb + 32 * st, *gs0 = NORM ? a.gamma + 32 * st : nullptr;
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const int st = min(st0 + p, s1 - 1);
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        xr[SET][p][h] = *reinterpret_cast<const f32x4_t *>(xp + 32 * st + 4 * h);
-        if constexpr (NORM) gr[SET][p][h] = *reinterpret_cast<const f32x4_t *>(gp + 32 * st + 4 * h);
-      }
+    for (int h = 0; h < 2; ++h) {
+      xr[SET][h] = *reinterpret_cast<const f32x4_t *>(xs0 + (xo + up + 4 * h));
+      if constexpr (NORM) gr[SET][h] = *reinterpret_cast<const f32x4_t *>(gs0 + (go + up + 4 * h));
     }
   };
   float ss = 0.f;
-  auto xstore = [&](int st0, auto set) {  // to the buffer of the same number
+  auto xstore = [&](int st0, auto set, bool live) {  // to the buffer of the same number
     constexpr int SET = decltype(set)::value;
+    float v[8];
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const bool in = st0 + p < s1;
-      float v[8];
+    for (int e = 0; e < 8; ++e) v[e] = xr[SET][e >> 2][e & 3];
+    if constexpr (TAIL) {
+      const bool in = st0 + sp < s1;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = in ? xr[SET][p][e >> 2][e & 3] : 0.f;
-      if constexpr (NORM) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss = __builtin_fmaf(v[e], v[e], ss);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] *= gr[SET][p][e >> 2][e & 3];
-      }
-      bf16x8_t hi, mid, lo;
-      split_bf16x8_nc(v, hi, mid, lo);
-      bf16x8_t *dst = xs + SET * BUF + (p * 64 + srow) * 4 + (slot ^ ((srow >> 1) & 3));
-      dst[0] = lo;
-      dst[2 * 64 * 4] = mid;
-      dst[2 * 2 * 64 * 4] = hi;
+      for (int e = 0; e < 8; ++e) v[e] = in ? v[e] : 0.f;
     }
+    if constexpr (NORM) {
+      float q = ss;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) q = __builtin_fmaf(v[e], v[e], q);
+      ss = live ? q : ss;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] *= gr[SET][e >> 2][e & 3];
+    }
+    bf16x8_t hi, mid, lo;
+    split_bf16x8_nc(v, hi, mid, lo);
+    bf16x8_t *dst = xs + SET * BUF + (sp * BM + srow) * 4 + (slot ^ ((srow >> 1) & 3));
+    dst[0] = lo;
+    dst[PLANE] = mid;
+    dst[2 * PLANE] = hi;
   };
 
   // Weight tiles of this wave (a partial last block repeats the last tile; nothing of it is stored)
@@ -127,13 +138,13 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
 #pragma unroll
   for (int u = 0; u < CT; ++u) {
     const int t = min(n0 / 16 + (SW ? u % OT : u), ntile - 1) + (SW && u >= OT ? ntile : 0);
-    wp[u] = a.W + (size_t)t * steps * 512 + lane * 8;
+    wp[u] = a.W + (size_t)t * steps * 512;
   }
   bf16x8_t w[4][CT];  // ring over k steps
   auto wload = [&](int st, auto at) {
 #pragma unroll
     for (int u = 0; u < CT; ++u)
-      w[decltype(at)::value][u] = *reinterpret_cast<const bf16x8_t *>(wp[u] + (size_t)min(st, s1 - 1) * 512);
+      w[decltype(at)::value][u] = *reinterpret_cast<const bf16x8_t *>(wp[u] + (size_t)min(st, s1 - 1) * 512 + lane * 8u);
   };
 
   // Sums over a pair (12 matrix-core additions) are added to the running total: short chains, so the
@@ -148,8 +159,7 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
   constexpr std::integral_constant<int, 1> I1{};
   constexpr std::integral_constant<int, 2> I2{};
   constexpr std::integral_constant<int, 3> I3{};
-  const int fr = wr * 32 + li;
-  const bf16x8_t *fsrc = xs + fr * 4 + (kb ^ ((fr >> 1) & 3));
+  const bf16x8_t *fsrc = xs + li * 4 + (kb ^ ((li >> 1) & 3));
   // step p of the chunk in buffer SET, weights in ring slot 2 SET + p
   auto mma = [&](auto set, auto step) {
     constexpr int SET = decltype(set)::value, PS = decltype(step)::value;
@@ -157,7 +167,7 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
     for (int q = 0; q < 3; ++q) {  // lo, mid, hi
       bf16x8_t x[RT];
 #pragma unroll
-      for (int t = 0; t < RT; ++t) x[t] = fsrc[SET * BUF + (q * 2 + PS) * 64 * 4 + 64 * t];
+      for (int t = 0; t < RT; ++t) x[t] = fsrc[SET * BUF + q * PLANE + PS * BM * 4 + 64 * t];
 #pragma unroll
       for (int t = 0; t < RT; ++t)
 #pragma unroll
@@ -172,7 +182,7 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
   xload(s0 + 2, I1);
   wload(s0 + 2, I2);
   wload(s0 + 3, I3);
-  xstore(s0, I0);
+  xstore(s0, I0, true);
   __syncthreads();
   // Straight-line pairs: no branch, so that the loads of the rings stay in flight across iterations.
   // Entering a pair: chunk st in buffer 0, chunk st + 2 in register set 1, weights of st .. st + 3.
@@ -188,7 +198,7 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
     mma(I0, I1);
     wload(st + 5, I1);
     __builtin_amdgcn_sched_barrier(0);
-    xstore(st + 2, I1);
+    xstore(st + 2, I1, true);
     __syncthreads();
     xload(st + 6, I1);
     __builtin_amdgcn_sched_barrier(0);
@@ -197,7 +207,7 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
     mma(I1, I1);
     wload(st + 7, I3);
     __builtin_amdgcn_sched_barrier(0);
-    xstore(st + 4, I0);
+    xstore(st + 4, I0, i + 1 < pairs);
 #pragma unroll
     for (int t = 0; t < RT; ++t)
 #pragma unroll
@@ -205,25 +215,29 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
     __syncthreads();
   }
 
-  if constexpr (NORM) {  // the row's sum of squares over its four staging threads, then over the groups
+  // The row's sum of squares over its staging threads: partial sums at rsum[part][row]
+  constexpr int NP = 2 * KG;
+  if constexpr (NORM) {
     ss += __shfl_xor(ss, 1, 64);
     ss += __shfl_xor(ss, 2, 64);
-    if (slot == 0) rsum[grp * 64 + srow] = ss;
+    if (slot == 0) rsum[(2 * grp + sp) * BM + srow] = ss;
   }
-  if constexpr (KG > 1) {  // the second group's sums, through its own staging buffers
-    f32x4_t *m = reinterpret_cast<f32x4_t *>(lds + 2 * BUF) + tid;
-    if (grp == 1) {
+  if constexpr (KG > 1) {  // the other groups' sums, through their own staging buffers, in group order
+    f32x4_t *m = reinterpret_cast<f32x4_t *>(lds) + tid;
+    if (grp > 0) {
 #pragma unroll
       for (int t = 0; t < RT; ++t)
 #pragma unroll
-        for (int u = 0; u < CT; ++u) m[(t * CT + u) * 256] = tot[t][u];
+        for (int u = 0; u < CT; ++u) m[grp * 2 * BUF + (t * CT + u) * 256] = tot[t][u];
     }
     __syncthreads();
-    if (grp == 1) return;
+    if (grp > 0) return;
 #pragma unroll
-    for (int t = 0; t < RT; ++t)
+    for (int k = 1; k < KG; ++k)
 #pragma unroll
-      for (int u = 0; u < CT; ++u) tot[t][u] += m[(t * CT + u) * 256];
+      for (int t = 0; t < RT; ++t)
+#pragma unroll
+        for (int u = 0; u < CT; ++u) tot[t][u] += m[k * 2 * BUF + (t * CT + u) * 256];
   } else if constexpr (NORM) {
     __syncthreads();
   }
@@ -232,8 +246,9 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
   for (int t = 0; t < RT; ++t) {
     inv[t] = 1.f;
     if constexpr (NORM) {
-      float s = rsum[wr * 32 + 16 * t + li];
-      if constexpr (KG > 1) s += rsum[64 + wr * 32 + 16 * t + li];
+      float s = rsum[16 * t + li];
+#pragma unroll
+      for (int i = 1; i < NP; ++i) s += rsum[i * BM + 16 * t + li];
       inv[t] = 1.0f / sqrtf(s / (float)a.K + a.eps);
     }
   }
@@ -263,14 +278,14 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
     if constexpr (RES) {
 #pragma unroll
       for (int t = 0; t < RT; ++t) {
-        const int m = min(m0 + wr * 32 + 16 * t + li, a.M - 1);
+        const int m = min(m0 + 16 * t + li, a.M - 1);
         rv[t][u] = quad(a.res + (size_t)m * a.ldr, n, true);
       }
     }
   }
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
-    const int m = m0 + wr * 32 + 16 * t + li;
+    const int m = m0 + 16 * t + li;
 #pragma unroll
     for (int u = 0; u < OT; ++u) {
       const int n = n0 + 16 * u + 4 * kb;
@@ -502,27 +517,30 @@ hipError_t rows_launch(const GemmArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int EPI, bool NORM, int BW, int KG>
+template <int EPI, bool NORM, int KG>
 hipError_t tile_launch(const GemmArgs &a, hipStream_t s) {
-  const int out = EPI == EPI_SWIGLU ? BW / 2 : BW;
-  const dim3 grid((a.N + out - 1) / out, (a.M + 63) / 64);
-  const size_t lds = (size_t)KG * 2 * 3 * 2 * 64 * 64 + (NORM ? (size_t)KG * 64 * 4 : 0);
-  hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, BW, KG>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
+  const int out = EPI == EPI_SWIGLU ? 64 : 128;
+  const dim3 grid((a.N + out - 1) / out, (a.M + 31) / 32);
+  const size_t lds = (size_t)KG * 2 * 3 * 2 * 32 * 64 + (NORM ? (size_t)KG * 2 * 32 * 4 : 0);
+  if (a.K % (128 * KG))
+    hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, KG, true>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
+  else
+    hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, KG, false>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
   return hipGetLastError();
 }
 
-// Up to 64 rows: k_gemm_rows.  More: 128-row weight tiles where they make a block for every CU, else 64-row ones; and where those are
-// still fewer than the CUs, two K groups a block.
+// Up to 64 rows: k_gemm_rows (whose X traffic per 16 columns is all rows: at 137 rows x 2048 it took
+// twice k_gemm_tile's time).  More: k_gemm_tile, with two K groups a block where there are fewer
+// blocks than CUs (137 rows, O and down of the 1.7B shape: whole prefill 4.63 -> 4.12 ms; with 544 blocks one group is 3% faster; four
+// groups measured as two).
 template <int EPI, bool NORM>
 hipError_t tile_shape(const GemmArgs &a, hipStream_t s) {
   if (a.M <= 16) return rows_launch<EPI, NORM, 1>(a, s);
   if (a.M <= 32) return rows_launch<EPI, NORM, 2>(a, s);
   if (a.M <= 48) return rows_launch<EPI, NORM, 3>(a, s);
   if (a.M <= 64) return rows_launch<EPI, NORM, 4>(a, s);
-  const int rows = (a.M + 63) / 64, n = EPI == EPI_SWIGLU ? 2 * a.N : a.N;
-  if (rows * ((n + 127) / 128) >= 256) return tile_launch<EPI, NORM, 128, 1>(a, s);
-  if (rows * ((n + 63) / 64) >= 256) return tile_launch<EPI, NORM, 64, 1>(a, s);
-  return a.K >= 128 ? tile_launch<EPI, NORM, 64, 2>(a, s) : tile_launch<EPI, NORM, 64, 1>(a, s);
+  const int n = EPI == EPI_SWIGLU ? 2 * a.N : a.N, blocks = (a.M + 31) / 32 * ((n + 127) / 128);
+  return blocks >= 256 || a.K < 128 ? tile_launch<EPI, NORM, 1>(a, s) : tile_launch<EPI, NORM, 2>(a, s);
 }
 
 template <int EPI>

@@ -154,7 +154,7 @@ def test_prefill_tiles_all_epilogues(eng, M, K):
 @pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 48, 49, 64, 65, 128, 129, 193])
 @pytest.mark.parametrize("K", [32, 96, 160, 1056])
 def test_row_and_step_remainders(eng, M, K):
-    """Rows around the 16-row tiles of the few-row kernel (up to 64) and the 64-row blocks of the
+    """Rows around the 16-row tiles of the few-row kernel (up to 64) and the 32-row blocks of the
     tiled one, k steps that do not fill a wave's share, a chunk or a pair of chunks, and a partial
     last column tile: residual with RMSNorm, bias, SwiGLU.  The tolerance is the module's."""
     N = 84
@@ -175,7 +175,7 @@ def test_row_and_step_remainders(eng, M, K):
 
 @pytest.mark.parametrize("M,N,K", [(70, 8192, 512), (200, 4100, 512), (520, 2050, 256)])
 def test_wide_tiles(eng, M, N, K):
-    """Enough 128-column blocks for every CU (the one-group kernel's 128- and 64-row weight tiles),
+    """Enough 128-column blocks for every CU (one K group a block),
     N not a multiple of 4 among them."""
     print(f"[gpu] gemm wide M={M} N={N} K={K}", flush=True)
     rng = np.random.default_rng(M)
