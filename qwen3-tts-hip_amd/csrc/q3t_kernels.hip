@@ -1387,25 +1387,6 @@ __global__ __launch_bounds__(128) void k_attn_merge(AttnMergeArgs a) {
 // Operand layouts of the 16x16x32 instruction: A[i][k] in lane i + 16 (k / 8), element k % 8;
 // B[k][j] in lane j + 16 (k / 8), element k % 8; C[i][j] in lane j + 16 (i / 4), element i % 4.
 // ---------------------------------------------------------------------------------------
-// x = hi + mid + lo, each a bf16: 24 significant bits, so every product with a bf16 weight
-// is exact and the GEMM matches an fp32 GEMV up to the order of the fp32 additions.
-// hi = bf16(x) (round to nearest even, v_cvt_pk_bf16_f32 on two lanes at a time); x - hi is
-// exact in fp32 and holds the remaining 16 bits, split the same way into mid and lo.
-__device__ __forceinline__ void split_bf16x8(const float *x, bf16x8_t &hi, bf16x8_t &mid, bf16x8_t &lo) {
-#pragma unroll
-  for (int e = 0; e < 8; e += 2) {
-    const f32x2_t v = {x[e], x[e + 1]};
-    const bf16x2_t h = __builtin_convertvector(v, bf16x2_t);
-    const f32x2_t r1 = v - __builtin_convertvector(h, f32x2_t);
-    const bf16x2_t m = __builtin_convertvector(r1, bf16x2_t);
-    const f32x2_t r2 = r1 - __builtin_convertvector(m, f32x2_t);
-    const bf16x2_t l = __builtin_convertvector(r2, bf16x2_t);
-    hi[e] = h[0]; hi[e + 1] = h[1];
-    mid[e] = m[0]; mid[e + 1] = m[1];
-    lo[e] = l[0]; lo[e + 1] = l[1];
-  }
-}
-
 // ---------------------------------------------------------------------------------------
 // Skinny GEMM for M <= 16 rows (one row per stream in batched decode): one 1024-thread
 // workgroup per 16-column output tile (a gate tile + up tile pair for SwiGLU); its 16 waves
@@ -1536,7 +1517,7 @@ __global__ __launch_bounds__(1024) void k_gemm_skinny(GemmArgs a) {
 #pragma unroll
       for (int b = 0; b < MB; ++b) {
         bf16x8_t hi, mid, lo;
-        split_bf16x8(xa[b][st], hi, mid, lo);
+        split_bf16x8_nc(xa[b][st], hi, mid, lo);
 #pragma unroll
         for (int t = 0; t < T; ++t) {
           const bf16x8_t w = __builtin_bit_cast(bf16x8_t, wb[st][t]);
