@@ -55,10 +55,11 @@ enum Epilogue : int32_t {
   EPI_RESIDUAL = 1,  // out[n] = res[n] + acc
   EPI_SWIGLU = 2,    // out[j] = silu(acc_gate_j) * acc_up_j; W holds gate rows then up rows
   EPI_BIAS = 3,      // out[n] = acc + bias[n]
-  // matrix-core GEMMs only (the codec decoder):
+  // matrix-core GEMMs only:
   EPI_AFFINE_RES = 4,  // out[n] = res[n] + (acc + bias[n]) * scale[n] (bias, scale optional)
   EPI_BIAS_GELU = 5,   // out[n] = gelu(acc + bias[n]), erf form
   EPI_RES_SNAKE = 6,   // out[n] = snake(res[n] + (acc + bias[n])), tables snake_a / snake_b
+  EPI_BIAS_SILU = 7,   // out[n] = silu(acc + bias[n]) (the text projection)
 };
 
 // Greedy token hand-off into a CodePredictor group (one stream): the group's input token is

@@ -29,6 +29,10 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, float *v, const
       v[e] = v[e] + b[e];
       v[e] = 0.5f * v[e] * (1.0f + erff(v[e] * 0.7071067811865476f));
     }
+    if constexpr (EPI == EPI_BIAS_SILU) {
+      v[e] = v[e] + b[e];
+      v[e] = v[e] / (1.0f + expf(-v[e]));
+    }
     if constexpr (EPI == EPI_RES_SNAKE) v[e] = r[e] + (v[e] + b[e]);
   }
   if constexpr (EPI == EPI_RES_SNAKE) snake_n<4>(v, c, c2);
@@ -256,7 +260,8 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
   // Lane (li, kb) holds columns 4 kb .. + 3 of row li of each tile.  Every operand is loaded before
   // the first store (Y may be the residual: each element is read and written by one lane only).
   constexpr bool RES = EPI == EPI_RESIDUAL || EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE;
-  constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU || EPI == EPI_RES_SNAKE;
+  constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU ||
+                        EPI == EPI_BIAS_SILU || EPI == EPI_RES_SNAKE;
   auto quad = [&](const float *p, int n, bool on) -> f32x4_t {  // columns n .. n + 3 of a row at p
     f32x4_t r{0.f, 0.f, 0.f, 0.f};
     if (!on) return r;
@@ -336,7 +341,8 @@ __global__ __launch_bounds__(512, 2) void k_gemm_rows(GemmArgs a, int vec) {
   constexpr bool SW = EPI == EPI_SWIGLU;
   constexpr int T = SW ? 2 : 1, W = 8, PS = MT == 1 ? 8 : (MT == 4 && SW && NORM ? 3 : 4);
   constexpr bool RES = EPI == EPI_RESIDUAL || EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE;
-  constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU || EPI == EPI_RES_SNAKE;
+  constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU ||
+                        EPI == EPI_BIAS_SILU || EPI == EPI_RES_SNAKE;
   __shared__ f32x4_t part[W][MT * T][64];
   __shared__ float ssq[W][MT * 16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
@@ -556,7 +562,7 @@ hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
       reinterpret_cast<uintptr_t>(a.gamma) % 16)
     return hipErrorInvalidValue;
   const bool res = epi == EPI_RESIDUAL || epi == EPI_AFFINE_RES || epi == EPI_RES_SNAKE;
-  const bool bias = epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_RES_SNAKE;
+  const bool bias = epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_BIAS_SILU || epi == EPI_RES_SNAKE;
   if ((res && !a.res) || (bias && !a.bias)) return hipErrorInvalidValue;
   if (a.split2 && (epi != EPI_RESIDUAL || a.gamma || a.M > kGemmSplitRows || !a.res_zero || a.K < 64))
     return hipErrorInvalidValue;
@@ -567,6 +573,7 @@ hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
     case EPI_BIAS: return tile_norm<EPI_BIAS>(a, s);
     case EPI_AFFINE_RES: return a.gamma ? hipErrorInvalidValue : tile_shape<EPI_AFFINE_RES, false>(a, s);
     case EPI_BIAS_GELU: return a.gamma ? hipErrorInvalidValue : tile_shape<EPI_BIAS_GELU, false>(a, s);
+    case EPI_BIAS_SILU: return a.gamma ? hipErrorInvalidValue : tile_shape<EPI_BIAS_SILU, false>(a, s);
     case EPI_RES_SNAKE:
       return a.gamma || !a.snake_a || !a.snake_b ? hipErrorInvalidValue : tile_shape<EPI_RES_SNAKE, false>(a, s);
   }

@@ -78,11 +78,10 @@ hipError_t launch_gemm_skinny(int epi, bool norm, const GemmArgs &a, hipStream_t
 // dst = src [rows][K] bf16 in the skinny GEMM's packed layout (GemmArgs::w_packed).
 // Requires rows % 16 == 0 and K % 32 == 0.
 hipError_t launch_pack_weights(const uint16_t *src, uint16_t *dst, int rows, int K, hipStream_t stream);
-// Prompt preparation: X[m] = fp32(table[ids[m]]) ([M][width]); x = silu(x) in place; and row m
-// of Y ([M][H], + codec_emb[codec[m]] where codec[m] >= 0) to dst[m] = (kind << 24) | row with
+// Prompt preparation: X[m] = fp32(table[ids[m]]) ([M][width]); and row m of
+// Y ([M][H], + codec_emb[codec[m]] where codec[m] >= 0) to dst[m] = (kind << 24) | row with
 // kind 0 prefill row, 1 trailing row, 2 the tts_pad row, 3 dropped.  The host validates ids.
 hipError_t launch_text_gather(const uint16_t *table, int width, const int32_t *ids, int M, float *X, hipStream_t stream);
-hipError_t launch_silu(float *x, size_t n, hipStream_t stream);
 // codec[m] value that adds the H-float row `xvec` (a voice-clone speaker embedding) instead of
 // a codec embedding row.
 constexpr int32_t kTextSpeakerRow = -2;

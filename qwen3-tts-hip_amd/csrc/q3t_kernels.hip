@@ -2539,12 +2539,6 @@ __global__ void k_text_gather(const uint16_t *table, int width, const int32_t *i
   for (int i = threadIdx.x; i < width; i += blockDim.x) dst[i] = bf16_to_f32(src[i]);
 }
 
-// x = x / (1 + e^-x) (text.rs:705-707).
-__global__ void k_silu(float *x, size_t n) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] = x[i] / (1.0f + expf(-x[i]));
-}
-
 // Row m of Y (+ codec_emb[codec[m]] where codec[m] >= 0, + xvec where codec[m] ==
 // kTextSpeakerRow) to its destination dst[m]: (kind << 24) | row, kind 0 = prefill row,
 // 1 = trailing row, 2 = the tts_pad row, 3 = none.
@@ -3034,12 +3028,6 @@ hipError_t launch_pack_weights(const uint16_t *src, uint16_t *dst, int rows, int
 hipError_t launch_text_gather(const uint16_t *table, int width, const int32_t *ids, int M, float *X, hipStream_t s) {
   if (M <= 0 || width <= 0) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_text_gather, dim3(M), dim3(256), 0, s, table, width, ids, X);
-  return hipGetLastError();
-}
-
-hipError_t launch_silu(float *x, size_t n, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_silu, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, x, n);
   return hipGetLastError();
 }
 

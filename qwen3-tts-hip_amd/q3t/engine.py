@@ -689,6 +689,12 @@ class HipTtsEngine:
         """The checkpoint holds the text-embedding table (q3t_prepare_text works)."""
         return self.info.get("text_vocab", 0) > 0
 
+    def _prompt_rows(self, n: int, lookahead: int):
+        """Arrays for q3t_prepare_text's rows, exactly as many as n ids and this lookahead give."""
+        H = self.info["talker_hidden"]
+        L = max(1, min(lookahead, n)) if n else 0
+        return (np.empty((9 + L, H), np.float32), np.empty((n - L + 1, H), np.float32), np.empty(H, np.float32))
+
     def prepare_text(self, content_ids: Sequence[int], speaker: str = "ryan", language: str = "english",
                      text_lookahead_tokens: int = 1 << 30, no_alloc: bool = False) -> PreparedInputs:
         """``TtsTextPrep::prepare_custom_voice_with_lookahead`` (text.rs:340-382) on the device
@@ -696,18 +702,16 @@ class HipTtsEngine:
         ``no_alloc`` runs ``q3t_prepare_text_noalloc`` instead: the same rows with no device
         allocation (a bounded prompt length; calls on one GPU must not overlap)."""
         ids = np.ascontiguousarray(np.asarray(content_ids, dtype=np.int64).astype(np.int32))
-        n, H = int(ids.size), self.info["talker_hidden"]
+        n = int(ids.size)
         opts = GenerateOptions(speaker=speaker, language=language)._c()
-        pre = np.zeros((9 + n, H), np.float32)
-        trail = np.zeros((n + 1, H), np.float32)
-        pad = np.zeros(H, np.float32)
-        P, T = ctypes.c_int32(), ctypes.c_int32()
         lookahead = min(int(text_lookahead_tokens), 0x7FFFFFFF)
+        pre, trail, pad = self._prompt_rows(n, lookahead)
+        P, T = ctypes.c_int32(), ctypes.c_int32()
         fn = _lib.q3t_prepare_text_noalloc if no_alloc else _lib.q3t_prepare_text
         _check(fn(self._h, _iptr(ids), n, opts.speaker, opts.language, lookahead, _fptr(pre),
                   ctypes.byref(P), _fptr(trail), ctypes.byref(T), _fptr(pad)))
-        return PreparedInputs(content_ids=ids.astype(np.int64), prefill=pre[:P.value].copy(),
-                              trailing_text=trail[:T.value].copy(), tts_pad_embed=pad)
+        return PreparedInputs(content_ids=ids.astype(np.int64), prefill=pre[:P.value], trailing_text=trail[:T.value],
+                              tts_pad_embed=pad)
 
     def start_stream_text(self, content_ids: Sequence[int], options: GenerateOptions = GenerateOptions(),
                           stream_options: StreamOptions = StreamOptions()) -> "HipTtsStream":
@@ -739,18 +743,16 @@ class HipTtsEngine:
         """``TtsTextPrep::prepare_voice_clone_xvector_with_lookahead`` (text.rs:432-490) on the
         device (``q3t_prepare_text_voice_clone``)."""
         ids, emb = self._voice_clone_args(inputs, prompt)
-        n, H = int(ids.size), self.info["talker_hidden"]
+        n = int(ids.size)
         lang = GenerateOptions(language=language)._c().language
-        pre = np.zeros((9 + n, H), np.float32)
-        trail = np.zeros((n + 1, H), np.float32)
-        pad = np.zeros(H, np.float32)
-        P, T = ctypes.c_int32(), ctypes.c_int32()
         lookahead = min(int(text_lookahead_tokens), 0x7FFFFFFF)
+        pre, trail, pad = self._prompt_rows(n, lookahead)
+        P, T = ctypes.c_int32(), ctypes.c_int32()
         _check(_lib.q3t_prepare_text_voice_clone(self._h, _iptr(ids), n, _fptr(emb), int(emb.size), lang, lookahead,
                                                  _fptr(pre), ctypes.byref(P), _fptr(trail), ctypes.byref(T),
                                                  _fptr(pad)))
-        return PreparedInputs(content_ids=ids.astype(np.int64), prefill=pre[:P.value].copy(),
-                              trailing_text=trail[:T.value].copy(), tts_pad_embed=pad)
+        return PreparedInputs(content_ids=ids.astype(np.int64), prefill=pre[:P.value], trailing_text=trail[:T.value],
+                              tts_pad_embed=pad)
 
     def start_voice_clone_stream(self, inputs: Union[str, Sequence[int]], prompt: VoiceClonePrompt,
                                  options: GenerateOptions = GenerateOptions(),

@@ -46,6 +46,22 @@ def test_prepare_text_matches_oracle(tiny_text, n, look, speaker, language):
     assert err <= TOL
 
 
+def test_prepare_text_sizes_in_turn(tiny_text):
+    """One engine over prompts that grow, shrink and pass the kept memory's limit: 64 and 65 rows (11
+    more than the ids; the two sides of the few-row GEMM) and 3011, with nothing left of the call
+    before.  The bound is the other tests'; results handed out earlier stay as they were."""
+    model, oracle, eng = tiny_text
+    kept = []
+    for n, look in [(53, 7), (3000, 5), (54, 1 << 30), (1, 1), (53, 7)]:
+        ids = textprep.random_prompt(n, 3 + n)
+        print(f"[gpu] prepare_text n={n} lookahead={look}", flush=True)
+        kept.append((eng.prepare_text(ids, "ryan", "english", look), oracle.prepare(ids, "ryan", "english", look)))
+    for got, ref in kept:
+        for a in ("prefill", "trailing_text", "tts_pad_embed"):
+            assert getattr(got, a).shape == getattr(ref, a).shape
+            assert float(np.abs(getattr(got, a) - getattr(ref, a)).max()) <= TOL
+
+
 @pytest.mark.parametrize("n,steps", [(32, 15), (0, 9)])
 def test_stream_from_ids_matches_oracle(tiny_text, n, steps):
     """A stream started from content ids (lookahead 6), including empty content: the 9-row
