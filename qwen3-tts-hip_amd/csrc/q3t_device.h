@@ -217,8 +217,8 @@ struct GemmArgs {
   // largest order key (value, lowest column) at keys_out[m * keys_row + blockIdx.x].
   uint64_t *keys_out;
   int64_t keys_row;
-  // EPI_RESIDUAL, few rows (skinny GEMM: T16 Y; launch_gemm: up to kGemmSplitRows rows): K split in
-  // two halves over grid y.  Each half adds its sums to Y with an fp32 atomic add, so Y must hold
+  // EPI_RESIDUAL, few rows (skinny GEMM: T16 Y; launch_gemm: up to gemm_split_rows rows): K split in
+  // two halves over grid y or z.  Each half adds its sums to Y with an fp32 atomic add, so Y must hold
   // zeros; two adds onto zero commute, so the result does not depend on their order.  The first
   // half also adds the residual, and then stores zero to res_zero (laid out as res, may be res
   // itself) at the same element: the buffer the next split GEMM of the chain accumulates into.

@@ -221,7 +221,7 @@ struct Pools {
   int32_t *row_on = nullptr;                            // [n] rows a batched launch covers
   int prefill_rows = 0;                                 // n * cap
   float *px = nullptr, *pqkv = nullptr, *pattn = nullptr, *pact = nullptr;
-  // The mid-layer residual of a prefill of at most kGemmSplitRows rows (split O / down GEMMs): zeros
+  // The mid-layer residual of a prefill of at most gemm_split_rows rows (split O / down GEMMs): zeros
   // except between a layer's O and down GEMMs.  pmid_dirty: a prefill stopped with an error, possibly
   // between the two; the next one zeroes it first.
   float *pmid = nullptr;
@@ -478,8 +478,8 @@ struct Engine {
     const size_t cache_layer = (size_t)d.kv_heads * talker.cap * d.head_dim * esz;
     // Few rows: the O and down GEMMs split K in two (GemmArgs::split2), O from px into pmid (zeros),
     // zeroing px, and down from pmid back into px, zeroing pmid.
-    const bool split = M <= kGemmSplitRows;
-    if (split && p.pmid_dirty) HIPC(hipMemsetAsync(p.pmid, 0, (size_t)kGemmSplitRows * H * 4, s));
+    const bool split = M <= gemm_split_rows(H);
+    if (split && p.pmid_dirty) HIPC(hipMemsetAsync(p.pmid, 0, (size_t)std::min(p.prefill_rows, gemm_split_rows(H)) * H * 4, s));
     p.pmid_dirty = split;
     for (int l = 0; l < d.layers; ++l) {
       const LayerW &L = talker.layers[l];
@@ -1110,7 +1110,7 @@ void alloc_pools(Engine &e, int n) {
   p.pqkv = dev_alloc<float>((size_t)p.prefill_rows * td.qkv_rows(), t);
   p.pattn = dev_alloc<float>((size_t)p.prefill_rows * td.q_out(), t);
   p.pact = dev_alloc<float>((size_t)p.prefill_rows * td.intermediate, t);
-  p.pmid = (float *)zeroed((size_t)kGemmSplitRows * Ht * 4);
+  p.pmid = (float *)zeroed((size_t)std::min(p.prefill_rows, gemm_split_rows(Ht)) * Ht * 4);
   HIPC(hipHostMalloc((void **)&p.h_states, sizeof(SlotState) * n, hipHostMallocDefault));
   HIPC(hipHostMalloc((void **)&p.h_codes, (size_t)p.codes_row * n * 4, hipHostMallocDefault));
   HIPC(hipHostMalloc((void **)&p.h_row_on, sizeof(int32_t) * n, hipHostMallocDefault));

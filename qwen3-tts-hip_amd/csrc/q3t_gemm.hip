@@ -38,6 +38,42 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, float *v, const
   if constexpr (EPI == EPI_RES_SNAKE) snake_n<4>(v, c, c2);
 }
 
+// GemmArgs::split2.  Two adds onto zero commute: the result does not depend on which half lands first.
+// The first half brings the residual and zeroes it for the GEMM that next accumulates into that buffer.
+// Four sums v of columns n .. n + 3 of row m go to t, this wave's LDS image of its ROWS x COLS outputs;
+// split_add then adds that image row by row, COLS consecutive columns at a time: an add is worked on
+// outside of the XCD, by whole lines.
+__device__ __forceinline__ void split_put(const GemmArgs &a, const float *v, const float *r, float *t, int m, int n,
+                                          int half, int vec) {
+  f32x4_t o{v[0], v[1], v[2], v[3]};
+  if (half == 0) {
+    o = f32x4_t{r[0] + v[0], r[1] + v[1], r[2] + v[2], r[3] + v[3]};
+    if (m < a.M) {
+      float *z = a.res_zero + (size_t)m * a.ldr + n;
+      if (vec) {
+        if (n < a.N) *reinterpret_cast<f32x4_t *>(z) = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (n + e < a.N) z[e] = 0.f;
+      }
+    }
+  }
+  *reinterpret_cast<f32x4_t *>(t) = o;
+}
+
+template <int ROWS, int COLS, int LD>
+__device__ __forceinline__ void split_add(const GemmArgs &a, const float *t, int m0, int n0, int lane) {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int r = lane / COLS, c = lane % COLS;
+#pragma unroll
+  for (int i = 0; i < ROWS; i += 64 / COLS)
+    if (m0 + i + r < a.M && n0 + c < a.N)
+      unsafeAtomicAdd(a.Y + (size_t)(m0 + i + r) * a.ldy + n0 + c, t[(i + r) * LD + c]);
+}
+
 // Block tile 32 rows x 128 packed weight rows (SwiGLU: 64 gate rows and the matching up rows), four
 // waves side by side, per K group.  What bounds it: per CU, loading X and the weights (64 bytes a
 // clock) and splitting X (7 vector operations an element) take as long as the matrix cores do with
@@ -61,8 +97,9 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, float *v, const
 //   * The weight tile is the A operand: a lane ends with four consecutive columns of one row, so
 //     loads and stores of the epilogue are 16 bytes wide.
 //   * TAIL: K is not a whole number of pairs of chunks per group; what is missing is staged as zeros.
-template <int EPI, bool NORM, int KG, bool TAIL>
+template <int EPI, bool NORM, int KG, bool TAIL, bool SPLIT>
 __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) {
+  static_assert(!SPLIT || EPI == EPI_RESIDUAL, "the K halves meet in a residual sum");
   constexpr bool SW = EPI == EPI_SWIGLU;
   constexpr int BM = 32, BW = 128;
   constexpr int RT = 2, CT = 2, OT = SW ? 1 : 2;      // row, weight and output tiles per wave
@@ -86,11 +123,12 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
   }
   const int m0 = mb * BM;
   const int n0 = nb * (SW ? BW / 2 : BW) + wave * OT * 16;  // this wave's first output column
-  // k steps [s0, s1) of 32 for this group, worked on in pairs of 64-wide chunks (four steps); what a
-  // pair holds past s1 is staged as zeros
-  const int steps = a.K / 32;
-  const int s0 = (int)((int64_t)steps * grp / KG), s1 = (int)((int64_t)steps * (grp + 1) / KG);
-  const int pairs = ((steps + KG - 1) / KG + 3) / 4;  // of the longest group: every wave meets every barrier
+  // k steps [s0, s1) of 32 for this group (SPLIT: of the workgroup's half), worked on in pairs of
+  // 64-wide chunks (four steps); what a pair holds past s1 is staged as zeros
+  const int steps = a.K / 32, h0 = SPLIT ? steps * (int)blockIdx.z / 2 : 0;
+  const int hn = (SPLIT ? steps * ((int)blockIdx.z + 1) / 2 : steps) - h0;
+  const int s0 = h0 + hn * grp / KG, s1 = h0 + hn * (grp + 1) / KG;
+  const int pairs = ((hn + KG - 1) / KG + 3) / 4;  // of the longest group: every wave meets every barrier
 
   // X: this thread stages row (tid % 128) / 4, k = 8 (tid % 4) .. + 7 of step tid / 128 of a chunk.
   // Addresses are a uniform base (step) plus a 32-bit offset in the block.
@@ -288,6 +326,8 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
       }
     }
   }
+  constexpr int LDI = 36;  // SPLIT: this wave's 32 x 32 outputs, in the staging space of group 0
+  float *image = reinterpret_cast<float *>(lds) + wave * BM * LDI;
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
     const int m = m0 + 16 * t + li;
@@ -313,6 +353,10 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
         c[e] = EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE ? cv[u][e] : 1.f;
         c2[e] = EPI == EPI_RES_SNAKE ? c2v[u][e] : 1.f;
       }
+      if constexpr (SPLIT) {
+        split_put(a, v, r, image + (16 * t + li) * LDI + 16 * u + 4 * kb, m, n, blockIdx.z, vec);
+        continue;
+      }
       tile_epilogue<EPI>(a, v, r, b, c, c2);
       if (m >= a.M || n >= a.N) continue;
       float *y = a.Y + (size_t)m * a.ldy + n;
@@ -325,6 +369,7 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
       }
     }
   }
+  if constexpr (SPLIT) split_add<BM, 32, LDI>(a, image, m0, n0, lane);
 }
 
 // Up to 64 rows (MT tiles of 16): a workgroup per 16-column tile (SwiGLU: a gate tile and its up
@@ -351,8 +396,10 @@ __global__ __launch_bounds__(512, 2) void k_gemm_rows(GemmArgs a, int vec) {
   const int h1 = SPLIT ? (int)((int64_t)steps * (blockIdx.y + 1) / 2) : steps;
   const int s0 = h0 + (h1 - h0) * wave / W, s1 = h0 + (h1 - h0) * (wave + 1) / W;
 
+  const int r0 = 16 * MT * blockIdx.z;  // first row
+
   // This thread's four outputs (threads below 64 MT): row om, columns on .. on + 3; operands first
-  const int ot = min(tid >> 6, MT - 1), om = 16 * ot + li, on = blockIdx.x * 16 + 4 * kb, cm = min(om, a.M - 1);
+  const int ot = min(tid >> 6, MT - 1), om = r0 + 16 * ot + li, on = blockIdx.x * 16 + 4 * kb, cm = min(om, a.M - 1);
   auto quad = [&](const float *p, bool have) -> f32x4_t {
     f32x4_t r{0.f, 0.f, 0.f, 0.f};
     if (!have) return r;
@@ -374,7 +421,7 @@ __global__ __launch_bounds__(512, 2) void k_gemm_rows(GemmArgs a, int vec) {
 
   const float *xp[MT];
 #pragma unroll
-  for (int t = 0; t < MT; ++t) xp[t] = a.X + (size_t)min(16 * t + li, a.M - 1) * a.ldx + 8 * kb;
+  for (int t = 0; t < MT; ++t) xp[t] = a.X + (size_t)min(r0 + 16 * t + li, a.M - 1) * a.ldx + 8 * kb;
   const uint16_t *wp[T];
 #pragma unroll
   for (int u = 0; u < T; ++u) wp[u] = a.W + (size_t)(blockIdx.x + u * ntile) * steps * 512 + lane * 8;
@@ -455,7 +502,7 @@ __global__ __launch_bounds__(512, 2) void k_gemm_rows(GemmArgs a, int vec) {
     if constexpr (NORM) {
       float q = 0.f;
 #pragma unroll
-      for (int k = 0; k < W; ++k) q += ssq[k][om];
+      for (int k = 0; k < W; ++k) q += ssq[k][16 * ot + li];
       inv = 1.0f / sqrtf(q / (float)a.K + a.eps);
     }
 #pragma unroll
@@ -464,22 +511,16 @@ __global__ __launch_bounds__(512, 2) void k_gemm_rows(GemmArgs a, int vec) {
       up[e] = NORM ? s[T - 1][e] * inv : s[T - 1][e];
     }
   }
-  if (om >= a.M || on >= a.N) return;
-  float *y = a.Y + (size_t)om * a.ldy + on;
   if constexpr (SPLIT) {
-    // Two adds onto zero commute: the result does not depend on which half lands first.  The first
-    // half brings the residual and zeroes it for the GEMM that next accumulates into that buffer.
+    float r[4], *image = reinterpret_cast<float *>(part[0][ot]);  // 16 x 16; this wave has read its sums
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      if (on + e >= a.N) break;
-      if (blockIdx.y == 0) {
-        v[e] = rv[e] + v[e];
-        a.res_zero[(size_t)om * a.ldr + on + e] = 0.f;
-      }
-      unsafeAtomicAdd(y + e, v[e]);
-    }
+    for (int e = 0; e < 4; ++e) r[e] = rv[e];
+    split_put(a, v, r, image + li * 16 + 4 * kb, om, on, blockIdx.y, vec);
+    split_add<16, 16, 16>(a, image, r0 + 16 * ot, blockIdx.x * 16, lane);
     return;
   }
+  if (om >= a.M || on >= a.N) return;
+  float *y = a.Y + (size_t)om * a.ldy + on;
   if constexpr (SW) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = v[e] / (1.0f + expf(-v[e])) * up[e];
@@ -512,7 +553,7 @@ int gemm_vec(const GemmArgs &a) {
 
 template <int EPI, bool NORM, int MT>
 hipError_t rows_launch(const GemmArgs &a, hipStream_t s) {
-  const dim3 grid((a.N + 15) / 16, a.split2 ? 2 : 1);
+  const dim3 grid((a.N + 15) / 16, a.split2 ? 2 : 1, (a.M + 16 * MT - 1) / (16 * MT));
   if constexpr (EPI == EPI_RESIDUAL && !NORM) {
     if (a.split2) {
       hipLaunchKernelGGL((k_gemm_rows<EPI, NORM, MT, true>), grid, dim3(512), 0, s, a, gemm_vec(a));
@@ -523,29 +564,45 @@ hipError_t rows_launch(const GemmArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-template <int EPI, bool NORM, int KG>
-hipError_t tile_launch(const GemmArgs &a, hipStream_t s) {
+template <int EPI, bool NORM, int KG, bool SPLIT>
+hipError_t tile_launch_split(const GemmArgs &a, hipStream_t s) {
   const int out = EPI == EPI_SWIGLU ? 64 : 128;
-  const dim3 grid((a.N + out - 1) / out, (a.M + 31) / 32);
+  const dim3 grid((a.N + out - 1) / out, (a.M + 31) / 32, SPLIT ? 2 : 1);
   const size_t lds = (size_t)KG * 2 * 3 * 2 * 32 * 64 + (NORM ? (size_t)KG * 2 * 32 * 4 : 0);
-  if (a.K % (128 * KG))
-    hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, KG, true>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
+  if (!SPLIT && a.K % (128 * KG))
+    hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, KG, !SPLIT, SPLIT>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
   else
-    hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, KG, false>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
+    hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, KG, false, SPLIT>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
   return hipGetLastError();
 }
 
+template <int EPI, bool NORM, int KG>
+hipError_t tile_launch(const GemmArgs &a, hipStream_t s) {
+  if constexpr (EPI == EPI_RESIDUAL && !NORM) {
+    if (a.split2) return tile_launch_split<EPI, NORM, KG, true>(a, s);
+  }
+  return tile_launch_split<EPI, NORM, KG, false>(a, s);
+}
+
 // Up to 64 rows: k_gemm_rows (whose X traffic per 16 columns is all rows: at 137 rows x 2048 it took
-// twice k_gemm_tile's time).  More: k_gemm_tile, with two K groups a block where there are fewer
-// blocks than CUs (137 rows, O and down of the 1.7B shape: whole prefill 4.63 -> 4.12 ms; with 544 blocks one group is 3% faster; four
-// groups measured as two).
+// twice k_gemm_tile's time), the rows in as many parts as bring the workgroups to one per CU at most (O
+// and down at 41 rows, 128 workgroups of three tiles: prefill 1.58 -> 1.46 ms with 256 of two and one;
+// with 384 of one tile each 1.65, a CU then waits for two).  More: k_gemm_tile, with two K groups a block
+// where there are fewer blocks than CUs (137 rows, O and down of the 1.7B shape: prefill 4.63 -> 4.12 ms;
+// with 544 blocks one group is 3% faster; four groups measured as two).
 template <int EPI, bool NORM>
 hipError_t tile_shape(const GemmArgs &a, hipStream_t s) {
-  if (a.M <= 16) return rows_launch<EPI, NORM, 1>(a, s);
-  if (a.M <= 32) return rows_launch<EPI, NORM, 2>(a, s);
-  if (a.M <= 48) return rows_launch<EPI, NORM, 3>(a, s);
-  if (a.M <= 64) return rows_launch<EPI, NORM, 4>(a, s);
-  const int n = EPI == EPI_SWIGLU ? 2 * a.N : a.N, blocks = (a.M + 31) / 32 * ((n + 127) / 128);
+  if (a.M <= 64) {
+    const int cols = (a.N + 15) / 16 * (a.split2 ? 2 : 1), tiles = (a.M + 15) / 16;
+    const int z = std::min(tiles, std::max(1, 256 / cols));
+    switch ((tiles + z - 1) / z) {
+      case 1: return rows_launch<EPI, NORM, 1>(a, s);
+      case 2: return rows_launch<EPI, NORM, 2>(a, s);
+      case 3: return rows_launch<EPI, NORM, 3>(a, s);
+      default: return rows_launch<EPI, NORM, 4>(a, s);
+    }
+  }
+  const int n = EPI == EPI_SWIGLU ? 2 * a.N : a.N, blocks = (a.M + 31) / 32 * ((n + 127) / 128) * (a.split2 ? 2 : 1);
   return blocks >= 256 || a.K < 128 ? tile_launch<EPI, NORM, 1>(a, s) : tile_launch<EPI, NORM, 2>(a, s);
 }
 
@@ -564,7 +621,8 @@ hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
   const bool res = epi == EPI_RESIDUAL || epi == EPI_AFFINE_RES || epi == EPI_RES_SNAKE;
   const bool bias = epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_BIAS_SILU || epi == EPI_RES_SNAKE;
   if ((res && !a.res) || (bias && !a.bias)) return hipErrorInvalidValue;
-  if (a.split2 && (epi != EPI_RESIDUAL || a.gamma || a.M > kGemmSplitRows || !a.res_zero || a.K < 64))
+  if (a.split2 && (epi != EPI_RESIDUAL || a.gamma || a.M > gemm_split_rows(a.N) || !a.res_zero || a.K < 64 ||
+                   (a.M > 64 && a.K % 512)))
     return hipErrorInvalidValue;
   switch (epi) {
     case EPI_STORE: return tile_norm<EPI_STORE>(a, s);

@@ -62,9 +62,9 @@ def test_prefill_tiles_per_wave(models, kv_bf16):
 
 
 def test_prefill_split_sums_leave_no_trace(models):
-    """Prompts of at most 64 rows accumulate the O and down projections into buffers that each GEMM
-    leaves zeroed for the next: the same prompt before and after others, longer ones (which take the
-    unsplit kernels) among them, gives the same bits."""
+    """Prompts of few rows accumulate the O and down projections into buffers that each GEMM leaves
+    zeroed for the next: the same prompt before and after others, on both sides of the 64 rows from
+    which the tiled kernel does it, gives the same bits."""
     model, d = models.get("tiny", 0)
     rng = np.random.default_rng(13)
     xs = [(rng.standard_normal((P, model.spec.talker.hidden)) * 0.5).astype(np.float32) for P in (41, 64, 65, 3, 130)]
@@ -76,3 +76,22 @@ def test_prefill_split_sums_leave_no_trace(models):
             np.testing.assert_array_equal(h, hidden)
             np.testing.assert_array_equal(l, logits)
             assert t == token
+
+
+@pytest.mark.parametrize("P", [65, 96, 97, 1023, 1024, 1025])
+def test_prefill_tiled_split_sums(models, P):
+    """O and down of 65 rows on in 32-row tiles: K halves up to 1,024 rows at hidden 512, whole sums
+    beyond; whole and partial last tiles, the same bits when run again."""
+    model, d = models.get("tiny", 0)
+    x = (np.random.default_rng(P).standard_normal((P, model.spec.talker.hidden)) * 0.5).astype(np.float32)
+    print(f"[gpu] prefill tiled split sums P={P}", flush=True)
+    with E.HipTtsEngine(d, E.EngineOptions(max_cache_steps=1040)) as eng:
+        hidden, logits, _ = eng.debug_talker_prefill(x)
+        again = eng.debug_talker_prefill(x)
+    np.testing.assert_array_equal(again[0], hidden)
+    np.testing.assert_array_equal(again[1], logits)
+    o = Oracle(model.tensors, model.config(), max_cache_steps=1040)
+    want = o.prefill(x.astype(np.float64))
+    # the bounds of test_prefill_lengths_match_oracle
+    _close(hidden, o.hidden, 1e-5, 1e-6, f"P={P} hidden")
+    _close(logits, want, 1e-5, 1e-6, f"P={P} logits")
