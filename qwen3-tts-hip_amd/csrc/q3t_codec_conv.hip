@@ -22,7 +22,8 @@
 //     so a lane ends with four consecutive columns of one row: 16-byte bias loads and stores.
 //   * BW = 192 where N allows it (every layer but N = 96, 288), else 96: all N are exact multiples.
 //   * BM = 64 (45 KB of LDS at dilation 9: up to three blocks a CU).  128-row blocks measured the
-//     same on long inputs and leave CUs idle on short ones.  A launch of few blocks splits the
+//     same on long inputs and leave CUs idle on short ones; residual units, which nothing splits,
+//     take BM = 32 when short.  A launch of few blocks splits the
 //     channel steps over grid z into split_ws, added in order by k_codec_conv_reduce.
 #include "q3t_codec.h"
 
@@ -87,11 +88,7 @@ __global__ __launch_bounds__(256, 2) void k_codec_conv(CodecConvArgs a) {
   };
   auto xstore = [&](int p, int buf) {
     const int idx = tid + 256 * p;
-    if (p == NP - 1 || NP == 1) {
-      if (idx >= units) return;
-    } else if (p >= 1 && 256 * (p + 1) > BM * 4 && idx >= units) {
-      return;
-    }
+    if (256 * (p + 1) > (BM + TAPS - 1) * 4 && idx >= units) return;
     float v[8] = {xr[p][0].x, xr[p][0].y, xr[p][0].z, xr[p][0].w, xr[p][1].x, xr[p][1].y, xr[p][1].z, xr[p][1].w};
     if constexpr (SIN) {
       const float ea[8] = {ta[0].x, ta[0].y, ta[0].z, ta[0].w, ta[1].x, ta[1].y, ta[1].z, ta[1].w};
@@ -360,6 +357,11 @@ hipError_t launch_codec_conv(int taps, const CodecConvArgs &a, hipStream_t s) {
     if (taps != 7 || !a.sa || !a.oa || a.C != a.N || !codec_unit_ok(a.C) || !a.b2 || (!a.ra != !a.rb) ||
         !aligned(a.w2) || !aligned(a.b2) || !aligned(a.ra) || !aligned(a.rb))
       return hipErrorInvalidValue;
+    // Fewer blocks than CUs: half the rows a block.  Decode of 6 frames 749 -> 710 us (60 blocks of 192
+    // channels, 180 of 96); of 31 (310 and 930 blocks) with half the rows 1139 -> 1180, each row block
+    // reading all the unit's weights.
+    if ((a.T + kConvRows - 1) / kConvRows < 256)
+      return a.C == 96 ? unit_launch<kConvRows / 2, 96>(a, s) : unit_launch<kConvRows / 2, 192>(a, s);
     return a.C == 96 ? unit_launch<kConvRows, 96>(a, s) : unit_launch<kConvRows, 192>(a, s);
   }
   if (taps == 7 && a.oa) return a.sa ? conv_shape<7, true, true>(a, s) : conv_shape<7, false, true>(a, s);

@@ -39,12 +39,14 @@ def test_decode_matches_oracle(codec_case, frames):
     assert err <= WAVE_TOL
 
 
-@pytest.mark.parametrize("frames", [1, 2, 5, 16, 17])
+@pytest.mark.parametrize("frames", [1, 2, 5, 8, 9, 16, 17, 25, 26])
 def test_decode_at_block_edges(codec_case, frames):
     """The decoder convolutions' 64-row blocks at half, exactly one and a remainder of a block
     (32 rows a frame after the first transposed convolution), split over channels, with rows
-    before time 0 in every block, and the attention's 16-row tiles (16, 17).  ~45 layers of fp32 sums of exact products end within 3.4e-6 of
-    float64 (2-norm) on inputs of 6 to 240 frames; four times that is allowed."""
+    before time 0 in every block; the attention's 16-row tiles (16, 17); and the frames at which the
+    residual units of 96 channels (8, 9) and of 192 (25, 26) go from 32- to 64-row blocks.  ~45 layers of
+    fp32 sums of exact products end within 3.4e-6 of float64 (2-norm) on inputs of 6 to 240 frames; four
+    times that is allowed."""
     eng, oracle = codec_case
     codes = np.random.default_rng(100 + frames).integers(0, 2048, (frames, 16)).astype(np.int32)
     print(f"[gpu] decode_codes frames={frames}", flush=True)
