@@ -327,7 +327,7 @@ size_t workspace_floats(size_t F) {
   const size_t big = (size_t)kCodecSamplesPerFrame * kFinal * F;  // largest T x C of the decoder blocks
   return 256 * 24 + F * 2 * kCodebookDim + (kPad + F) * kProjected + F * kPreConv + F * kHidden + F * 3 * kQ +
          F * kQ + F * kInter + F * kPreConv + 2 * ((kPad + 4 * F) * kUp) + 4 * F * kUp + 4 * F * kConvNext +
-         (kPad * kFinal + big) + 2 * big;
+         3 * big;
 }
 
 }  // namespace
@@ -412,8 +412,7 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
   // 5. decoder: causal conv kernel 7, four blocks, Snake, last conv, clamp
   const size_t big = (size_t)kCodecSamplesPerFrame * kFinal * F;
   float *R = take(big), *A2 = take(big);
-  float *Sp = take((size_t)kPad * kFinal + big);  // starts with the zero rows the last conv reads
-  float *S = Sp + (size_t)kPad * kFinal;          // Snaked input of the next transposed (or last) convolution
+  float *S = take(big);  // Snaked input of the next transposed (or last) convolution
   auto conv = [&](int taps, const float *X, int rows, int C, int d, const float *sa, const float *sb, const uint16_t *W,
                   const float *bias, const float *oa, const float *ob, float *Y, int N) {
     const CodecConvArgs a{X, rows, C, d, sa, sb, W, bias, oa, ob, Y, N, c.split_ws, Codec::kSplitFloats,
@@ -449,8 +448,7 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
       hip_check(launch_gemm(end ? EPI_RES_SNAKE : EPI_AFFINE_RES, g, s), "launch_gemm(1x1)");
     }
   }
-  HIPC(hipMemsetAsync(Sp, 0, (size_t)kPad * kFinal * sizeof(float), s));
-  hip_check(launch_codec_final(S - (size_t)6 * kFinal, c.fin_w, c.fin_bias, T, kFinal, 7, samples, s), "codec_final");
+  hip_check(launch_codec_final(S, c.fin_w, c.fin_bias, T, kFinal, 7, samples, s), "codec_final");
   HIPC(hipStreamSynchronize(s));
 }
 

@@ -67,7 +67,8 @@ hipError_t launch_codec_layernorm(const float *x, const float *g, const float *b
 // Causal attention with RoPE over raw qkv rows (64 dims a head; table [T][32] (cos, sin)).
 hipError_t launch_codec_attention(const float *qkv, int T, int ld, int heads, const float2 *table, float scale,
                                   float *out, int ldo, hipStream_t s);
-hipError_t launch_codec_final(const float *xin, const float *w, const float *b, int T, int C, int K, float *out,
+// Last convolution (C = 96, K = 7; rows x[t] of time t) and clamp.
+hipError_t launch_codec_final(const float *x, const float *w, const float *b, int T, int C, int K, float *out,
                               hipStream_t s);
 
 }  // namespace q3t

@@ -199,70 +199,57 @@ __global__ __launch_bounds__(256, 2) void k_codec_attention(const float *qkv, in
       make_float4(r[0] * inv, r[1] * inv, r[2] * inv, r[3] * inv);
 }
 
-// Last convolution to one channel + clamp to [-1, 1]: out[t] = clamp(b + sum_{j, c}
-// xin[t + j][c] w[j][c]) with xin row 0 = time -(K-1) (kernels.rs:742-770, 903-918).  A
-// workgroup stages the kFinalTile + K - 1 input rows its kFinalTile outputs read in LDS
-// (unit-stride loads), rows C + 1 floats apart so that the 64 lanes of a wave, which read
-// rows t .. t + 63 at one channel, fall in different banks (at a pitch of C = 96 every lane
-// hit the same bank); each thread then sums its K * C products in (j, c) order.
-constexpr int kFinalTile = 128, kFinalMaxC = 96, kFinalMaxK = 7;
+// Last convolution, 96 channels and 7 taps to one, + clamp to [-1, 1]: out[t] = clamp(b + sum_j P[t - 6 + j][j])
+// with P[t][j] = sum_c x[t][c] w[j][c], rows before time 0 zeros (kernels.rs:742-770, 903-918).
+//
+// What bounds it: reading x.  The products over channels are a GEMM with the taps as (seven of sixteen)
+// columns on v_mfma_f32_16x16x4_f32 (fp32 products and sums; 1.4 GFLOP at 240 frames, ~10 us), whose
+// operand is x as it lies in memory: lane (li, kk) loads 16 bytes of row li per 16 channels and their
+// four k's.  Only the seven sums a row go through LDS, to be added along the diagonal.  A thread per
+// output with the rows staged in LDS, 672 dependent products each and a wave per SIMD for want of LDS,
+// took 128 us at 240 frames (177 MB, 35 us at the copy rate) and 13 at 6.
+// A wave takes two 16-row tiles, all twelve loads in flight; a block's 128 rows give 122 outputs.
+constexpr int kFinalC = 96, kFinalK = 7, kFinalRows = 128, kFinalOut = kFinalRows - kFinalK + 1;
 
-__global__ __launch_bounds__(kFinalTile) void k_codec_final(const float *xin, const float *w, const float *b, int T,
-                                                            int C, int K, float *out) {
-  __shared__ float xs[(kFinalTile + kFinalMaxK - 1) * (kFinalMaxC + 1)];
-  __shared__ float ws[kFinalMaxK * kFinalMaxC];
-  const int t0 = blockIdx.x * kFinalTile;
-  const int rows = min(kFinalTile, T - t0) + K - 1;
-  const int pitch = C + 1;
-  const float *src = xin + (size_t)t0 * C;
-  for (int i = threadIdx.x; i < rows * C; i += kFinalTile) {
-    const int r = i / C;
-    xs[r * pitch + (i - r * C)] = src[i];
-  }
-  for (int i = threadIdx.x; i < K * C; i += kFinalTile) ws[i] = w[i];
-  __syncthreads();
-  const int t = t0 + (int)threadIdx.x;
-  if (t >= T) return;
-  float s = b[0];
-  for (int j = 0; j < K; ++j) {
-    const float *xr = xs + (threadIdx.x + j) * pitch;
-    for (int c = 0; c < C; ++c) s += xr[c] * ws[j * C + c];
-  }
-  out[t] = fminf(fmaxf(s, -1.0f), 1.0f);
-}
-
-// The same for C % 4 == 0: rows C + 4 floats apart (16-byte aligned; the 16 lanes of a
-// 128-bit LDS read start in distinct banks), x and w read four channels at a time, the
-// products still added one by one in (j, c) order.
-__global__ __launch_bounds__(kFinalTile) void k_codec_final4(const float *xin, const float *w, const float *b, int T,
-                                                             int C, int K, float *out) {
-  __shared__ float4 xs4[(kFinalTile + kFinalMaxK - 1) * (kFinalMaxC + 4) / 4];
-  __shared__ float4 ws4[kFinalMaxK * kFinalMaxC / 4];
-  const int t0 = blockIdx.x * kFinalTile;
-  const int rows = min(kFinalTile, T - t0) + K - 1;
-  const int c4 = C / 4, pitch4 = c4 + 1;
-  const float4 *src = reinterpret_cast<const float4 *>(xin + (size_t)t0 * C);
-  for (int i = threadIdx.x; i < rows * c4; i += kFinalTile) {
-    const int r = i / c4;
-    xs4[r * pitch4 + (i - r * c4)] = src[i];
-  }
-  for (int i = threadIdx.x; i < K * c4; i += kFinalTile) ws4[i] = reinterpret_cast<const float4 *>(w)[i];
-  __syncthreads();
-  const int t = t0 + (int)threadIdx.x;
-  if (t >= T) return;
-  float s = b[0];
-  for (int j = 0; j < K; ++j) {
-    const float4 *xr = xs4 + (threadIdx.x + j) * pitch4;
-    const float4 *wr = ws4 + j * c4;
-#pragma unroll 4
-    for (int c = 0; c < c4; ++c) {
-      const float4 x = xr[c], v = wr[c];
-      s += x.x * v.x;
-      s += x.y * v.y;
-      s += x.z * v.z;
-      s += x.w * v.w;
+__global__ __launch_bounds__(256) void k_codec_final(const float *x, const float *w, const float *b, int T,
+                                                     float *out) {
+  constexpr int NC = kFinalC / 16, RT = 2;
+  __shared__ float P[kFinalK][kFinalRows + 4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kk = lane >> 4;
+  const int t0 = blockIdx.x * kFinalOut;
+  f32x4_t xv[RT][NC], wv[NC];
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    const int g = t0 - (kFinalK - 1) + 16 * (RT * wave + t) + li;
+    const float *src = x + (size_t)min(max(g, 0), T - 1) * kFinalC + 4 * kk;
+#pragma unroll
+    for (int c = 0; c < NC; ++c) xv[t][c] = *reinterpret_cast<const f32x4_t *>(src + 16 * c);
+    if (g < 0) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c) xv[t][c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     }
   }
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    wv[c] = *reinterpret_cast<const f32x4_t *>(w + min(li, kFinalK - 1) * kFinalC + 16 * c + 4 * kk);
+    if (li >= kFinalK) wv[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll
+  for (int t = 0; t < RT; ++t) {
+    f32x4_t acc{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[t][c][s], wv[c][s], acc, 0, 0, 0);
+    // lane (li, kk) holds rows 4 kk .. + 3 of column li
+    if (li < kFinalK) *reinterpret_cast<f32x4_t *>(&P[li][16 * (RT * wave + t) + 4 * kk]) = acc;
+  }
+  __syncthreads();
+  const int t = t0 + tid;
+  if (tid >= kFinalOut || t >= T) return;
+  float s = b[0];
+#pragma unroll
+  for (int j = 0; j < kFinalK; ++j) s += P[j][tid + j];
   out[t] = fminf(fmaxf(s, -1.0f), 1.0f);
 }
 
@@ -306,15 +293,11 @@ hipError_t launch_codec_attention(const float *qkv, int T, int ld, int heads, co
   return hipGetLastError();
 }
 
-hipError_t launch_codec_final(const float *xin, const float *w, const float *b, int T, int C, int K, float *out,
+hipError_t launch_codec_final(const float *x, const float *w, const float *b, int T, int C, int K, float *out,
                               hipStream_t s) {
-  if (T <= 0 || C <= 0 || K <= 0 || C > kFinalMaxC || K > kFinalMaxK) return hipErrorInvalidValue;
   auto aligned = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
-  if (C % 4 == 0 && aligned(xin) && aligned(w))
-    hipLaunchKernelGGL(k_codec_final4, dim3(blocks_for(T, kFinalTile)), dim3(kFinalTile), 0, s, xin, w, b, T, C, K,
-                       out);
-  else
-    hipLaunchKernelGGL(k_codec_final, dim3(blocks_for(T, kFinalTile)), dim3(kFinalTile), 0, s, xin, w, b, T, C, K, out);
+  if (T <= 0 || C != kFinalC || K != kFinalK || !aligned(x) || !aligned(w)) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_codec_final, dim3(blocks_for(T, kFinalOut)), dim3(256), 0, s, x, w, b, T, out);
   return hipGetLastError();
 }
 
