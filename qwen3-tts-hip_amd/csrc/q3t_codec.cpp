@@ -326,7 +326,7 @@ namespace {
 size_t workspace_floats(size_t F) {
   const size_t big = (size_t)kCodecSamplesPerFrame * kFinal * F;  // largest T x C of the decoder blocks
   return 256 * 24 + F * 2 * kCodebookDim + (kPad + F) * kProjected + F * kPreConv + F * kHidden + F * 3 * kQ +
-         F * kQ + F * kInter + F * kPreConv + 2 * ((kPad + 4 * F) * kUp) + 4 * F * kUp + 4 * F * kConvNext +
+         F * kQ + F * kInter + F * kPreConv + 3 * 4 * F * kUp + 4 * F * kConvNext +
          3 * big;
 }
 
@@ -350,7 +350,6 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
     if (off > c.ws_floats) fail(Q3T_ERR_INVALID, "codec workspace plan is too small");
     return p;
   };
-  auto zero_pad = [&](float *buf, int C) { HIPC(hipMemsetAsync(buf, 0, (size_t)kPad * C * sizeof(float), s)); };
   auto gemm = [&](int epi, const float *X, int ldx, int M, const uint16_t *W, int N, int K, float *Y, int ldy,
                   const float *bias, const float *res = nullptr, int ldr = 0, const float *scale = nullptr,
                   const float *gamma = nullptr) {
@@ -364,7 +363,7 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
   float *E = take((size_t)F * 2 * kCodebookDim);
   hip_check(launch_codec_rvq(codes, F, groups, c.cb_first, c.cb_rest, kCodebook, kCodebookDim, E, s), "rvq");
   float *Qp = take((size_t)(kPad + F) * kProjected);
-  zero_pad(Qp, kProjected);
+  HIPC(hipMemsetAsync(Qp, 0, (size_t)kPad * kProjected * sizeof(float), s));  // the rows before time 0
   float *Q = Qp + (size_t)kPad * kProjected;
   gemm(EPI_STORE, E, 2 * kCodebookDim, F, c.w_rvq, kProjected, 2 * kCodebookDim, Q, kProjected, nullptr);
   float *PC = take((size_t)F * kPreConv);
@@ -389,22 +388,17 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
   gemm(EPI_BIAS, H, kHidden, F, c.out_w, kPreConv, kHidden, TR, kPreConv, c.out_b, nullptr, 0, nullptr, c.norm);
 
   // 4. two upsample stages: transposed conv (stride 2) + ConvNeXt block
-  float *Up = take((size_t)(kPad + 4 * F) * kUp);
-  float *Uo = take((size_t)(kPad + 4 * F) * kUp);
+  float *Y = take((size_t)4 * F * kUp), *O = take((size_t)4 * F * kUp);
   float *D = take((size_t)4 * F * kUp);
   float *G = take((size_t)4 * F * kConvNext);
   const float *xin = TR;
   int T = F;
   for (int i = 0; i < 2; ++i) {
     const Codec::Up &U = c.up[i];
-    zero_pad(Up, kUp);
-    float *Y = Up + (size_t)kPad * kUp;
     gemm(EPI_BIAS, xin, kUp, T, U.tw, 2 * kUp, kUp, Y, 2 * kUp, U.tb);
     T *= 2;
-    hip_check(launch_codec_dwconv(Up + (size_t)(kPad - 6) * kUp, U.dw_w, U.dw_b, T, kUp, 7, D, s), "dwconv");
-    hip_check(launch_codec_layernorm(D, U.ln_g, U.ln_b, T, kUp, kLnEps, D, s), "layernorm");
+    hip_check(launch_codec_dwconv_norm(Y, U.dw_w, U.dw_b, U.ln_g, U.ln_b, T, kUp, 7, kLnEps, D, s), "dwconv_norm");
     gemm(EPI_BIAS_GELU, D, kUp, T, U.pw1, kConvNext, kUp, G, kConvNext, U.pw1_b);
-    float *O = Uo + (size_t)kPad * kUp;
     gemm(EPI_AFFINE_RES, G, kConvNext, T, U.pw2, kUp, kConvNext, O, kUp, U.pw2_b, Y, kUp, U.gamma);
     xin = O;
   }

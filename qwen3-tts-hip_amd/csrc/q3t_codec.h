@@ -60,10 +60,9 @@ hipError_t launch_codec_conv(int taps, const CodecConvArgs &a, hipStream_t s);
 // source index of column n, channel c, tap j.
 std::vector<uint16_t> codec_conv_pack(const std::vector<uint16_t> &w, int N, int C, int taps,
                                       size_t (*at)(int n, int c, int j, int N, int C, int taps));
-hipError_t launch_codec_dwconv(const float *xin, const float *w, const float *b, int T, int C, int K, float *out,
-                               hipStream_t s);
-hipError_t launch_codec_layernorm(const float *x, const float *g, const float *b, int T, int C, float eps, float *out,
-                                  hipStream_t s);
+// Depthwise convolution (C = 1024, K = 7; w [C][K]) and LayerNorm of its rows.
+hipError_t launch_codec_dwconv_norm(const float *x, const float *w, const float *wb, const float *g, const float *b,
+                                    int T, int C, int K, float eps, float *out, hipStream_t s);
 // Causal attention with RoPE over raw qkv rows (64 dims a head; table [T][32] (cos, sin)).
 hipError_t launch_codec_attention(const float *qkv, int T, int ld, int heads, const float2 *table, float scale,
                                   float *out, int ldo, hipStream_t s);

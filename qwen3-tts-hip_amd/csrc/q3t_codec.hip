@@ -41,41 +41,51 @@ __global__ void k_codec_snake_prep(float *alpha, float *beta, int C) {
   beta[c] = 1.0f / (expf(beta[c]) + 1.0e-9f);
 }
 
-// Depthwise causal conv, kernel K: out[t][c] = b[c] + sum_j xin[t + j][c] w[c][j], where xin
-// row 0 is time -(K-1) (codec_depthwise_causal_conv1d_f32, kernels.rs:642-667).
-__global__ void k_codec_dwconv(const float *xin, const float *w, const float *b, int T, int C, int K, float *out) {
-  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= (size_t)T * C) return;
-  const int c = (int)(i % C);
-  const size_t t = i / C;
-  float s = b[c];
-  for (int j = 0; j < K; ++j) s += xin[(t + j) * C + c] * w[c * K + j];
-  out[i] = s;
-}
+// ConvNeXt's depthwise causal convolution, 7 taps, rows before time 0 zeros
+// (codec_depthwise_causal_conv1d_f32, kernels.rs:642-667), and the LayerNorm of its rows
+// (codec_layernorm_f32, kernels.rs:582-612): variance E[x^2] - mean^2, clamped at 0.  A 256-thread
+// workgroup per row of 1,024 channels, a thread's four channels 256 apart and in registers between
+// the two.  Latency-bound: two kernels and a memset of the rows before time 0 were three launches of
+// ~4 us each.
+constexpr int kDwC = 1024, kDwK = 7;
 
-// LayerNorm of each row (codec_layernorm_f32, kernels.rs:582-612): variance E[x^2] - mean^2,
-// clamped at 0.  One 256-thread workgroup per row.
-__global__ void k_codec_layernorm(const float *x, const float *g, const float *b, int C, float eps, float *out) {
-  const float *r = x + (size_t)blockIdx.x * C;
-  float *o = out + (size_t)blockIdx.x * C;
+__global__ __launch_bounds__(256) void k_codec_dwconv_norm(const float *x, const float *w, const float *wb,
+                                                           const float *g, const float *b, float eps, float *out) {
+  constexpr int N = kDwC / 256;
   __shared__ float ps[4], pq[4];
-  float s = 0.f, q = 0.f;
-  for (int c = threadIdx.x; c < C; c += 256) {
-    const float v = r[c];
-    s += v;
-    q += v * v;
+  const int tid = threadIdx.x, t = blockIdx.x;
+  float v[N], s = 0.f, q = 0.f;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int c = tid + 256 * i;
+    v[i] = wb[c];
+#pragma unroll
+    for (int j = 0; j < kDwK; ++j) {
+      const int r = t - (kDwK - 1) + j;
+      const float e = x[(size_t)max(r, 0) * kDwC + c];
+      v[i] += (r >= 0 ? e : 0.f) * w[c * kDwK + j];
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    s += v[i];
+    q += v[i] * v[i];
   }
   s = wave_sum64(s);
   q = wave_sum64(q);
-  if ((threadIdx.x & 63) == 0) {
-    ps[threadIdx.x >> 6] = s;
-    pq[threadIdx.x >> 6] = q;
+  if ((tid & 63) == 0) {
+    ps[tid >> 6] = s;
+    pq[tid >> 6] = q;
   }
   __syncthreads();
-  const float mean = (((ps[0] + ps[1]) + ps[2]) + ps[3]) / (float)C;
-  const float var = fmaxf((((pq[0] + pq[1]) + pq[2]) + pq[3]) / (float)C - mean * mean, 0.f);
+  const float mean = (((ps[0] + ps[1]) + ps[2]) + ps[3]) / (float)kDwC;
+  const float var = fmaxf((((pq[0] + pq[1]) + pq[2]) + pq[3]) / (float)kDwC - mean * mean, 0.f);
   const float inv = rsqrtf(var + eps);
-  for (int c = threadIdx.x; c < C; c += 256) o[c] = (r[c] - mean) * inv * g[c] + b[c];
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int c = tid + 256 * i;
+    out[(size_t)t * kDwC + c] = (v[i] - mean) * inv * g[c] + b[c];
+  }
 }
 
 // Causal attention over rows 0..t for query row t and head h: rotate-half RoPE on q and k
@@ -270,17 +280,10 @@ hipError_t launch_codec_snake_prep(float *alpha, float *beta, int C, hipStream_t
   return hipGetLastError();
 }
 
-hipError_t launch_codec_dwconv(const float *xin, const float *w, const float *b, int T, int C, int K, float *out,
-                               hipStream_t s) {
-  if (T <= 0 || C <= 0 || K <= 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_codec_dwconv, dim3(blocks_for((size_t)T * C, 256)), dim3(256), 0, s, xin, w, b, T, C, K, out);
-  return hipGetLastError();
-}
-
-hipError_t launch_codec_layernorm(const float *x, const float *g, const float *b, int T, int C, float eps, float *out,
-                                  hipStream_t s) {
-  if (T <= 0 || C <= 0) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_codec_layernorm, dim3(T), dim3(256), 0, s, x, g, b, C, eps, out);
+hipError_t launch_codec_dwconv_norm(const float *x, const float *w, const float *wb, const float *g, const float *b,
+                                    int T, int C, int K, float eps, float *out, hipStream_t s) {
+  if (T <= 0 || C != kDwC || K != kDwK) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_codec_dwconv_norm, dim3(T), dim3(256), 0, s, x, w, wb, g, b, eps, out);
   return hipGetLastError();
 }
 
