@@ -45,6 +45,45 @@ __device__ __forceinline__ void split_bf16x8_nc(const float *x, bf16x8_t &hi, bf
   split_bf16_nc<8>(x, hi, mid, lo);
 }
 
+// The same value in three terms rounded to nearest, the form of the GEMMs (the sums of a GEMM depend
+// on the terms in their last bits).  The conversion issues at about a fifth of the rate of the mask and
+// permute above.
+__device__ __forceinline__ void split_bf16x8_rn(const float *x, bf16x8_t &hi, bf16x8_t &mid, bf16x8_t &lo) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    const f32x2_t v = {x[e], x[e + 1]};
+    const bf16x2_t h = __builtin_convertvector(v, bf16x2_t);
+    const f32x2_t r1 = v - __builtin_convertvector(h, f32x2_t);
+    const bf16x2_t m = __builtin_convertvector(r1, bf16x2_t);
+    const f32x2_t r2 = r1 - __builtin_convertvector(m, f32x2_t);
+    const bf16x2_t l = __builtin_convertvector(r2, bf16x2_t);
+    hi[e] = h[0]; hi[e + 1] = h[1];
+    mid[e] = m[0]; mid[e + 1] = m[1];
+    lo[e] = l[0]; lo[e + 1] = l[1];
+  }
+}
+
+// Of a product x g: the first term is the rounded product's, the others hold what the exact product has
+// past it.
+__device__ __forceinline__ void split_bf16x8_rn_mul(const float *x, const float *g, bf16x8_t &hi, bf16x8_t &mid,
+                                                    bf16x8_t &lo) {
+#pragma clang fp contract(off)
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    const f32x2_t v = {x[e] * g[e], x[e + 1] * g[e + 1]};
+    const bf16x2_t h = __builtin_convertvector(v, bf16x2_t);
+    const f32x2_t hf = __builtin_convertvector(h, f32x2_t);
+    const f32x2_t r1 = {__builtin_fmaf(x[e], g[e], -hf[0]), __builtin_fmaf(x[e + 1], g[e + 1], -hf[1])};
+    const bf16x2_t m = __builtin_convertvector(r1, bf16x2_t);
+    const f32x2_t r2 = r1 - __builtin_convertvector(m, f32x2_t);
+    const bf16x2_t l = __builtin_convertvector(r2, bf16x2_t);
+    hi[e] = h[0]; hi[e + 1] = h[1];
+    mid[e] = m[0]; mid[e + 1] = m[1];
+    lo[e] = l[0]; lo[e + 1] = l[1];
+  }
+}
+
 // Snake: v + sin(v ea)^2 ib, with the per-channel tables ea = exp(alpha), ib = 1 / (exp(beta) +
 // 1e-9) (codec_snake_beta_f32, kernels.rs:692-710).
 //

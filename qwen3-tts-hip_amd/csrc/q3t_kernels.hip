@@ -1505,10 +1505,6 @@ __global__ __launch_bounds__(1024) void k_gemm_skinny(GemmArgs a) {
         ss = pair16_sum(ss);  // the four lanes of a row (kb = 0..3)
         ss = pair32_sum(ss);
         if (kb == 0) ssq[wave][b * 16 + li] = ss;
-#pragma unroll
-        for (int st = 0; st < KP; ++st)
-#pragma unroll
-          for (int e = 0; e < 8; ++e) xa[b][st][e] = xa[b][st][e] * ga[st][e];
       }
     }
 
@@ -1517,7 +1513,8 @@ __global__ __launch_bounds__(1024) void k_gemm_skinny(GemmArgs a) {
 #pragma unroll
       for (int b = 0; b < MB; ++b) {
         bf16x8_t hi, mid, lo;
-        split_bf16x8_nc(xa[b][st], hi, mid, lo);
+        if constexpr (NORM) split_bf16x8_rn_mul(xa[b][st], ga[st], hi, mid, lo);
+        else split_bf16x8_rn(xa[b][st], hi, mid, lo);
 #pragma unroll
         for (int t = 0; t < T; ++t) {
           const bf16x8_t w = __builtin_bit_cast(bf16x8_t, wb[st][t]);
