@@ -1,5 +1,5 @@
-// Device helpers shared by the matrix-core kernels: the three-term bf16 form of an fp32 value,
-// and the codec's Snake activation.
+// Device helpers shared by the kernels: wave sums, the three-term bf16 form of an fp32 value, and the
+// codec's Snake activation.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -12,6 +12,32 @@ typedef float f32x2_t __attribute__((ext_vector_type(2)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
+
+// Cross-lane reductions on DPP (data-parallel primitives: VALU lane permutes, no LDS round
+// trip).  Each step adds a permuted copy: quad_perm [1,0,3,2] and [2,3,0,1] (quads),
+// row_half_mirror and row_mirror (rows of 16), then row_bcast:15 / row_bcast:31 fold the
+// four rows into lane 63.  The order is fixed, so results are deterministic.
+template <int CTRL, int ROWS = 0xf>
+__device__ __forceinline__ float dpp_f(float v, float fill) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, fill), __builtin_bit_cast(int, v),
+                                                               CTRL, ROWS, 0xf, false));
+}
+
+// Sum over each row of 16 lanes, in every lane of the row.
+__device__ __forceinline__ float row16_sum(float v) {
+  v += dpp_f<0xB1>(v, 0.f);
+  v += dpp_f<0x4E>(v, 0.f);
+  v += dpp_f<0x141>(v, 0.f);
+  v += dpp_f<0x140>(v, 0.f);
+  return v;
+}
+
+__device__ __forceinline__ float wave_sum(float v) {
+  v = row16_sum(v);
+  v += dpp_f<0x142, 0xa>(v, 0.f);
+  v += dpp_f<0x143, 0xc>(v, 0.f);
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+}
 
 // x = hi + mid + lo, each bf16, exactly: hi is the upper half of x (its top 8 significant bits), x -
 // hi is exact in fp32 and holds the other 16, mid is the upper half of that and lo the rest.  Every

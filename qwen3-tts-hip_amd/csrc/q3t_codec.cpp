@@ -356,6 +356,7 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
     GemmArgs g{};
     g.X = X; g.ldx = ldx; g.W = W; g.Y = Y; g.ldy = ldy; g.M = M; g.N = N; g.K = K;
     g.bias = bias; g.res = res; g.ldr = ldr; g.scale = scale; g.gamma = gamma; g.eps = kRmsEps; g.w_packed = 1;
+    g.k_parts = gemm_k_parts(epi, M, N, K);
     hip_check(launch_gemm(epi, g, s), "launch_gemm(codec)");
   };
 
@@ -438,7 +439,7 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
       GemmArgs g{};
       g.X = A2; g.ldx = co; g.W = Un.w2; g.Y = end ? S : R; g.ldy = co; g.M = T; g.N = co; g.K = co;
       g.bias = Un.b2; g.res = R; g.ldr = co;
-      g.snake_a = na; g.snake_b = nb; g.w_packed = 1;
+      g.snake_a = na; g.snake_b = nb; g.w_packed = 1; g.k_parts = gemm_k_parts(EPI_AFFINE_RES, T, co, co);
       hip_check(launch_gemm(end ? EPI_RES_SNAKE : EPI_AFFINE_RES, g, s), "launch_gemm(1x1)");
     }
   }

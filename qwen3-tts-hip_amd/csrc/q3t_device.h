@@ -217,11 +217,15 @@ struct GemmArgs {
   // largest order key (value, lowest column) at keys_out[m * keys_row + blockIdx.x].
   uint64_t *keys_out;
   int64_t keys_row;
-  // EPI_RESIDUAL, few rows (skinny GEMM: T16 Y; launch_gemm: up to gemm_split_rows rows): K split in
-  // two halves over grid y or z.  Each half adds its sums to Y with an fp32 atomic add, so Y must hold
-  // zeros; two adds onto zero commute, so the result does not depend on their order.  The first
-  // half also adds the residual, and then stores zero to res_zero (laid out as res, may be res
-  // itself) at the same element: the buffer the next split GEMM of the chain accumulates into.
+  // launch_gemm: K in so many parts (gemm_k_parts; 0: one), part z the 32-wide steps S z / k_parts ..
+  // S (z + 1) / k_parts of S.  A part's sum starts at zero and takes a step's low, middle and high terms'
+  // products in turn; the parts are added in order.
+  int32_t k_parts;
+  // skinny GEMM, EPI_RESIDUAL, T16 Y: K split in two halves over grid y.  Each half adds its
+  // sums to Y with an fp32 atomic add, so Y must hold zeros; two adds onto zero commute, so
+  // the result does not depend on their order.  The first half also adds the residual, and
+  // then stores zero to res_zero (T16, may be res itself) at the same element: the buffer
+  // the next split GEMM of the chain accumulates into.
   int32_t split2;
   float *res_zero;
   // skinny GEMM: mb = 2 runs two 16-row blocks (two positions of the same stream rows, row m

@@ -221,11 +221,6 @@ struct Pools {
   int32_t *row_on = nullptr;                            // [n] rows a batched launch covers
   int prefill_rows = 0;                                 // n * cap
   float *px = nullptr, *pqkv = nullptr, *pattn = nullptr, *pact = nullptr;
-  // The mid-layer residual of a prefill of at most gemm_split_rows rows (split O / down GEMMs): zeros
-  // except between a layer's O and down GEMMs.  pmid_dirty: a prefill stopped with an error, possibly
-  // between the two; the next one zeroes it first.
-  float *pmid = nullptr;
-  bool pmid_dirty = false;
   SlotState *h_states = nullptr;                        // pinned [n]
   int32_t *h_codes = nullptr;                           // pinned [n][codes_row], mirrors codes
   int32_t *h_row_on = nullptr;                          // pinned [n]
@@ -476,16 +471,12 @@ struct Engine {
     if (M <= 0 || M > p.prefill_rows) fail(Q3T_ERR_CAPACITY, "prefill of %d rows exceeds the workspace", M);
     const size_t esz = kv_bf16 ? 2 : 4;
     const size_t cache_layer = (size_t)d.kv_heads * talker.cap * d.head_dim * esz;
-    // Few rows: the O and down GEMMs split K in two (GemmArgs::split2), O from px into pmid (zeros),
-    // zeroing px, and down from pmid back into px, zeroing pmid.
-    const bool split = M <= gemm_split_rows(H);
-    if (split && p.pmid_dirty) HIPC(hipMemsetAsync(p.pmid, 0, (size_t)std::min(p.prefill_rows, gemm_split_rows(H)) * H * 4, s));
-    p.pmid_dirty = split;
     for (int l = 0; l < d.layers; ++l) {
       const LayerW &L = talker.layers[l];
       GemmArgs g{};
       g.X = p.px; g.ldx = H; g.gamma = L.g_in; g.eps = d.eps;
       g.W = L.qkv_p; g.w_packed = 1; g.Y = p.pqkv; g.ldy = Q; g.M = M; g.N = Q; g.K = H;
+      g.k_parts = gemm_k_parts(EPI_STORE, M, Q, H);
       hip_check(launch_gemm(EPI_STORE, g, s), "launch_gemm(qkv)");
       PrefillBatchArgs pa{};
       pa.qkv = p.pqkv; pa.gq = L.gq; pa.gk = L.gk; pa.rope = talker.rope; pa.out = p.pattn;
@@ -504,25 +495,19 @@ struct Engine {
       g = GemmArgs{};
       g.X = p.pattn; g.ldx = O; g.W = L.o_p; g.w_packed = 1; g.res = p.px; g.ldr = H; g.Y = p.px; g.ldy = H;
       g.M = M; g.N = H; g.K = O;
-      float *mid = p.px;
-      if (split) {
-        mid = p.pmid;
-        g.Y = mid; g.split2 = 1; g.res_zero = p.px;
-      }
+      g.k_parts = gemm_k_parts(EPI_RESIDUAL, M, H, O);
       hip_check(launch_gemm(EPI_RESIDUAL, g, s), "launch_gemm(o)");
       g = GemmArgs{};
-      g.X = mid; g.ldx = H; g.gamma = L.g_post; g.eps = d.eps;
+      g.X = p.px; g.ldx = H; g.gamma = L.g_post; g.eps = d.eps;
       g.W = L.gu_p; g.w_packed = 1; g.Y = p.pact; g.ldy = I; g.M = M; g.N = I; g.K = H;
+      g.k_parts = gemm_k_parts(EPI_SWIGLU, M, I, H);
       hip_check(launch_gemm(EPI_SWIGLU, g, s), "launch_gemm(gate_up)");
       g = GemmArgs{};
-      g.X = p.pact; g.ldx = I; g.W = L.down_p; g.w_packed = 1; g.res = mid; g.ldr = H; g.Y = p.px; g.ldy = H;
+      g.X = p.pact; g.ldx = I; g.W = L.down_p; g.w_packed = 1; g.res = p.px; g.ldr = H; g.Y = p.px; g.ldy = H;
       g.M = M; g.N = H; g.K = I;
-      if (split) {
-        g.split2 = 1; g.res_zero = mid;
-      }
+      g.k_parts = gemm_k_parts(EPI_RESIDUAL, M, H, I);
       hip_check(launch_gemm(EPI_RESIDUAL, g, s), "launch_gemm(down)");
     }
-    p.pmid_dirty = false;
     for (const PrefillSeg &sg : segs)
       HIPC(hipMemcpyAsync(slots[sg.slot].x_t, p.px + (size_t)(sg.row0 + sg.P - 1) * H, (size_t)H * 4,
                           hipMemcpyDeviceToDevice, s));
@@ -1110,7 +1095,6 @@ void alloc_pools(Engine &e, int n) {
   p.pqkv = dev_alloc<float>((size_t)p.prefill_rows * td.qkv_rows(), t);
   p.pattn = dev_alloc<float>((size_t)p.prefill_rows * td.q_out(), t);
   p.pact = dev_alloc<float>((size_t)p.prefill_rows * td.intermediate, t);
-  p.pmid = (float *)zeroed((size_t)std::min(p.prefill_rows, gemm_split_rows(Ht)) * Ht * 4);
   HIPC(hipHostMalloc((void **)&p.h_states, sizeof(SlotState) * n, hipHostMallocDefault));
   HIPC(hipHostMalloc((void **)&p.h_codes, (size_t)p.codes_row * n * 4, hipHostMallocDefault));
   HIPC(hipHostMalloc((void **)&p.h_row_on, sizeof(int32_t) * n, hipHostMallocDefault));
@@ -1165,7 +1149,7 @@ void free_pools(Engine &e) {
   void *ptrs[] = {p.t_k,      p.t_v,     p.c_k,   p.c_v,      p.x_t,      p.t_in,    p.qkv,  p.attn,
                   p.act,      p.logits_t, p.logits_c, p.x_c,  p.cp_prefix, p.cp_in,  p.cur,  p.emb_sum,
                   p.trailing, p.attn_part, p.trace_t, p.trace_c, p.codes,  p.st,      p.prm,  p.row_on,
-                  p.px,       p.pqkv,    p.pattn, p.pact,     p.pmid,    p.cp_keys, p.opart, p.x_mid, p.tok_cur};
+                  p.px,       p.pqkv,    p.pattn, p.pact,     p.cp_keys, p.opart, p.x_mid, p.tok_cur};
   for (void *q : ptrs)
     if (q) (void)hipFree(q);
   if (p.h_states) (void)hipHostFree(p.h_states);
@@ -1889,10 +1873,12 @@ void run_text_plan(Engine &e, const TextPlan &p, const TextWorkspace &w, float *
   GemmArgs g{};
   g.X = w.X; g.ldx = e.text_hidden; g.W = e.tp_fc1; g.bias = e.tp_b1; g.Y = w.Hd; g.ldy = e.tp_inter;
   g.M = M; g.N = e.tp_inter; g.K = e.text_hidden; g.w_packed = 1;
+  g.k_parts = gemm_k_parts(EPI_BIAS_SILU, M, g.N, g.K);
   hip_check(launch_gemm(EPI_BIAS_SILU, g, s), "launch_gemm(text fc1)");
   g = GemmArgs{};
   g.X = w.Hd; g.ldx = e.tp_inter; g.W = e.tp_fc2; g.bias = e.tp_b2; g.Y = w.Y; g.ldy = H;
   g.M = M; g.N = H; g.K = e.tp_inter; g.w_packed = 1;
+  g.k_parts = gemm_k_parts(EPI_BIAS, M, g.N, g.K);
   hip_check(launch_gemm(EPI_BIAS, g, s), "launch_gemm(text fc2)");
   hip_check(launch_text_assemble(w.Y, H, M, codec, e.codec_emb, w.xvec, dst, prefill, trailing, pad, s),
             "launch_text_assemble");

@@ -1,6 +1,10 @@
 // Matrix-core GEMM for many rows (prompt prefill, text projection, codec linears and table builds):
 // Y[M][N] = f(X[M][K] . W[N][K]^T), bf16 weights in packed order (GemmArgs::w_packed), fp32
 // activations as three exact bf16 terms, fp32 accumulation; optional RMSNorm of the rows.
+//
+// The order of the additions is part of what a GEMM returns (launch_gemm), whichever kernel computes it:
+// tokens are argmaxes or draws over logits, a stream of a few hundred frames comes across logits that
+// are equal to a bit or two, and a sum in another order then turns its codes from there on.
 #include "q3t_kernels.h"
 
 #include <algorithm>
@@ -38,78 +42,81 @@ __device__ __forceinline__ void tile_epilogue(const GemmArgs &a, float *v, const
   if constexpr (EPI == EPI_RES_SNAKE) snake_n<4>(v, c, c2);
 }
 
-// GemmArgs::split2.  Two adds onto zero commute: the result does not depend on which half lands first.
-// The first half brings the residual and zeroes it for the GEMM that next accumulates into that buffer.
-// Four sums v of columns n .. n + 3 of row m go to t, this wave's LDS image of its ROWS x COLS outputs;
-// split_add then adds that image row by row, COLS consecutive columns at a time: an add is worked on
-// outside of the XCD, by whole lines.
-__device__ __forceinline__ void split_put(const GemmArgs &a, const float *v, const float *r, float *t, int m, int n,
-                                          int half, int vec) {
-  f32x4_t o{v[0], v[1], v[2], v[3]};
-  if (half == 0) {
-    o = f32x4_t{r[0] + v[0], r[1] + v[1], r[2] + v[2], r[3] + v[3]};
-    if (m < a.M) {
-      float *z = a.res_zero + (size_t)m * a.ldr + n;
-      if (vec) {
-        if (n < a.N) *reinterpret_cast<f32x4_t *>(z) = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      } else {
+// 1 / rms of rows r0 .. r0 + rows - 1 (past the last row: of the last), into inv[rows], by all waves:
+// lane sums of every 64th square, then wave_sum.  RB rows a wave and 512 columns a round: two round
+// trips to the L2 for rows of 1,024.  A launch of its own per norm costs what the round trips do
+// and the gap before it.
+template <int RB>
+__device__ __forceinline__ void rows_inv_rms(const GemmArgs &a, int r0, int rows, int wave, int waves, int lane,
+                                             float *inv) {
+  constexpr int U = 8;
+  for (int r = wave; r < rows; r += RB * waves) {
+    const float *x[RB];
+    float ss[RB] = {};
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-          if (n + e < a.N) z[e] = 0.f;
-      }
+    for (int i = 0; i < RB; ++i) x[i] = a.X + (size_t)min(r0 + min(r + i * waves, rows - 1), a.M - 1) * a.ldx;
+    int k0 = 0;
+    for (; k0 + 64 * U <= a.K; k0 += 64 * U) {
+      float v[RB][U];
+#pragma unroll
+      for (int i = 0; i < RB; ++i)
+#pragma unroll
+        for (int e = 0; e < U; ++e) v[i][e] = (x[i] + k0)[lane + 64 * e];
+      __builtin_amdgcn_sched_barrier(0);  // every load before the first sum
+#pragma unroll
+      for (int e = 0; e < U; ++e)
+#pragma unroll
+        for (int i = 0; i < RB; ++i) ss[i] = __builtin_fmaf(v[i][e], v[i][e], ss[i]);
     }
-  }
-  *reinterpret_cast<f32x4_t *>(t) = o;
-}
-
-template <int ROWS, int COLS, int LD>
-__device__ __forceinline__ void split_add(const GemmArgs &a, const float *t, int m0, int n0, int lane) {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const int r = lane / COLS, c = lane % COLS;
+    for (int k = k0 + lane; k < a.K; k += 64)
 #pragma unroll
-  for (int i = 0; i < ROWS; i += 64 / COLS)
-    if (m0 + i + r < a.M && n0 + c < a.N)
-      unsafeAtomicAdd(a.Y + (size_t)(m0 + i + r) * a.ldy + n0 + c, t[(i + r) * LD + c]);
+      for (int i = 0; i < RB; ++i) ss[i] = __builtin_fmaf(x[i][k], x[i][k], ss[i]);
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      const float w = wave_sum(ss[i]);
+      s = lane == i ? w : s;
+    }
+    if (lane < RB && r + lane * waves < rows) inv[r + lane * waves] = 1.0f / sqrtf(s / (float)a.K + a.eps);
+  }
 }
 
-// Block tile 32 rows x 128 packed weight rows (SwiGLU: 64 gate rows and the matching up rows), four
+// Block tile 32 rows x 64 CT packed weight rows (SwiGLU: 64 gate rows and the matching up rows), four
 // waves side by side, per K group.  What bounds it: per CU, loading X and the weights (64 bytes a
-// clock) and splitting X (7 vector operations an element) take as long as the matrix cores do with
+// clock) and splitting X (~9 vector operations an element) take as long as the matrix cores do with
 // what is loaded (three MFMAs a product), so all three have to run at once, and a block's own chain
 // of k steps must never wait.  Hence:
 //   * Everything is loaded well ahead of use: the weights, straight from global memory in
 //     matrix-core order (1 KiB contiguous per 16 columns and step, read by one wave only), in a ring
-//     of four k steps; X two 64-wide chunks ahead in registers.  The loop is straight-line code with
-//     uniform addresses: a branch in it made the compiler copy the rings and wait for them.
+//     of four k steps; X two 64-wide chunks ahead in registers.  Addresses are uniform and the loads
+//     are outside of every branch.
 //   * X is split into its three terms once per block, into LDS planes of [step][row][4 slots of
 //     16 bytes], slots xor-ed with (row / 2) % 4 (any 8 rows of a slot in distinct bank columns),
 //     double buffered: one barrier per 64 k.
-//   * 32 rows rather than 64: 106-127 registers, four waves a SIMD from different blocks, so that one
-//     block's splitting runs under another's matrix-core work, and finer shares of the CUs.  521 rows,
-//     1024 -> 4096: 32 us (64 x 128 blocks) -> 25 us; 137 rows, 2048 -> 2 x 6144: 58 -> 35 us.
-//   * KG = 2: where blocks are few, two such groups of waves in a block take half of K each and add
-//     up through LDS.
-//   * RMSNorm needs no launch of its own: every block passes over its rows whole, so the staging
-//     threads sum the squares, the matrix cores take x * gain, and the epilogue scales the sums
-//     by 1 / rms (one scalar per row).
+//   * 32 rows rather than 64: four waves a SIMD from different blocks, so that one
+//     block's splitting runs under another's matrix-core work, and finer shares of the CUs.
 //   * The weight tile is the A operand: a lane ends with four consecutive columns of one row, so
 //     loads and stores of the epilogue are 16 bytes wide.
-//   * TAIL: K is not a whole number of pairs of chunks per group; what is missing is staged as zeros.
-template <int EPI, bool NORM, int KG, bool TAIL, bool SPLIT>
+//   * PARTS (GemmArgs::k_parts above one): each part's sum is a chain of its own; the parts' sums are
+//     added in part order.  KG = 2: two such groups of waves in a block take the parts' first and
+//     second half; the second's sums wait in LDS, one image a part.
+//   * TAIL: a group's k steps are not whole pairs of chunks; what is missing is staged as zeros and
+//     not multiplied.
+template <int EPI, bool NORM, int KG, int CT, bool TAIL, bool PARTS>
 __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) {
-  static_assert(!SPLIT || EPI == EPI_RESIDUAL, "the K halves meet in a residual sum");
   constexpr bool SW = EPI == EPI_SWIGLU;
-  constexpr int BM = 32, BW = 128;
-  constexpr int RT = 2, CT = 2, OT = SW ? 1 : 2;      // row, weight and output tiles per wave
+  static_assert(KG == 1 || PARTS, "the groups take whole parts");
+  static_assert(!SW || CT == 2, "a gate tile and its up tile");
+  constexpr int BM = 32, BW = 64 * CT;
+  constexpr int RT = 2, OT = SW ? 1 : CT;             // row and output tiles per wave, CT weight tiles
   constexpr int PLANE = 2 * BM * 4, BUF = 3 * PLANE;  // 16-byte units of a term, of a staging buffer
-  extern __shared__ bf16x8_t lds[];                   // [KG][2][BUF], then row sums [KG][64]
+  extern __shared__ bf16x8_t lds[];                   // [KG][2][BUF], row scales [BM], KG = 2: images
   const int tid = threadIdx.x & 255, lane = tid & 63, li = lane & 15, kb = lane >> 4;
   const int gwave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform for the compiler too
   const int grp = KG > 1 ? gwave >> 2 : 0, wave = gwave & 3;
   bf16x8_t *xs = lds + grp * 2 * BUF;
-  float *rsum = reinterpret_cast<float *>(lds + KG * 2 * BUF);
+  float *rinv = reinterpret_cast<float *>(lds + KG * 2 * BUF);
+  f32x4_t *image = reinterpret_cast<f32x4_t *>(rinv + BM) + tid;  // [part - half][RT * CT][256]
 
   // Few column blocks: each XCD (workgroup id % 8) takes a contiguous range of row-major block
   // tiles, so that its L2 reads only its own X rows, once for all column blocks.
@@ -123,12 +130,13 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
   }
   const int m0 = mb * BM;
   const int n0 = nb * (SW ? BW / 2 : BW) + wave * OT * 16;  // this wave's first output column
-  // k steps [s0, s1) of 32 for this group (SPLIT: of the workgroup's half), worked on in pairs of
-  // 64-wide chunks (four steps); what a pair holds past s1 is staged as zeros
-  const int steps = a.K / 32, h0 = SPLIT ? steps * (int)blockIdx.z / 2 : 0;
-  const int hn = (SPLIT ? steps * ((int)blockIdx.z + 1) / 2 : steps) - h0;
-  const int s0 = h0 + hn * grp / KG, s1 = h0 + hn * (grp + 1) / KG;
-  const int pairs = ((hn + KG - 1) / KG + 3) / 4;  // of the longest group: every wave meets every barrier
+  // k steps [s0, s1) of 32 for this group, parts [part, ..), worked on in pairs of 64-wide chunks (four
+  // steps)
+  const int steps = a.K / 32, parts = PARTS ? a.k_parts : 1, half = (parts + 1) / 2, mid = steps * half / parts;
+  const int s0 = KG > 1 && grp ? mid : 0, s1 = KG > 1 && !grp ? mid : steps;
+  int part = KG > 1 && grp ? half : 0, bound = steps * (part + 1) / parts;
+  // of the longer group: every wave meets every barrier
+  const int pairs = ((KG > 1 ? max(mid, steps - mid) : steps) + 3) / 4;
 
   // X: this thread stages row (tid % 128) / 4, k = 8 (tid % 4) .. + 7 of step tid / 128 of a chunk.
   // Addresses are a uniform base (step) plus a 32-bit offset in the block.
@@ -147,8 +155,8 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
       if constexpr (NORM) gr[SET][h] = *reinterpret_cast<const f32x4_t *>(gs0 + (go + up + 4 * h));
     }
   };
-  float ss = 0.f;
-  auto xstore = [&](int st0, auto set, bool live) {  // to the buffer of the same number
+  float rs = 1.f;
+  auto xstore = [&](int st0, auto set) {  // to the buffer of the same number
     constexpr int SET = decltype(set)::value;
     float v[8];
 #pragma unroll
@@ -159,15 +167,11 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
       for (int e = 0; e < 8; ++e) v[e] = in ? v[e] : 0.f;
     }
     if constexpr (NORM) {
-      float q = ss;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) q = __builtin_fmaf(v[e], v[e], q);
-      ss = live ? q : ss;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] *= gr[SET][e >> 2][e & 3];
+      for (int e = 0; e < 8; ++e) v[e] = (v[e] * rs) * gr[SET][e >> 2][e & 3];
     }
     bf16x8_t hi, mid, lo;
-    split_bf16x8_nc(v, hi, mid, lo);
+    split_bf16x8_rn(v, hi, mid, lo);
     bf16x8_t *dst = xs + SET * BUF + (sp * BM + srow) * 4 + (slot ^ ((srow >> 1) & 3));
     dst[0] = lo;
     dst[PLANE] = mid;
@@ -189,22 +193,24 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
       w[decltype(at)::value][u] = *reinterpret_cast<const bf16x8_t *>(wp[u] + (size_t)min(st, s1 - 1) * 512 + lane * 8u);
   };
 
-  // Sums over a pair (12 matrix-core additions) are added to the running total: short chains, so the
-  // rounding error over a long K stays that of a blocked sum.
-  f32x4_t tot[RT][CT], acc[RT][CT];
+  f32x4_t acc[RT][CT], tot[PARTS ? RT : 1][PARTS ? CT : 1];
 #pragma unroll
   for (int t = 0; t < RT; ++t)
 #pragma unroll
-    for (int u = 0; u < CT; ++u) tot[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < CT; ++u) {
+      acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if constexpr (PARTS) tot[t][u] = f32x4_t{-0.f, -0.f, -0.f, -0.f};  // -0 + v = v, -0 too
+    }
 
   constexpr std::integral_constant<int, 0> I0{};
   constexpr std::integral_constant<int, 1> I1{};
   constexpr std::integral_constant<int, 2> I2{};
   constexpr std::integral_constant<int, 3> I3{};
   const bf16x8_t *fsrc = xs + li * 4 + (kb ^ ((li >> 1) & 3));
-  // step p of the chunk in buffer SET, weights in ring slot 2 SET + p
-  auto mma = [&](auto set, auto step) {
+  // step st = step p of the chunk in buffer SET, weights in ring slot 2 SET + p
+  auto mma = [&](auto set, auto step, int st) {
     constexpr int SET = decltype(set)::value, PS = decltype(step)::value;
+    if (TAIL && st >= s1) return;
 #pragma unroll
     for (int q = 0; q < 3; ++q) {  // lo, mid, hi
       bf16x8_t x[RT];
@@ -216,83 +222,65 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
         for (int u = 0; u < CT; ++u)
           acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[2 * SET + PS][u], x[t], acc[t][u], 0, 0, 0);
     }
+    if constexpr (PARTS) {
+      if (st + 1 == bound) {  // the part's sum is whole
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+          for (int u = 0; u < CT; ++u) {
+            if (KG > 1 && grp) image[((part - half) * RT * CT + t * CT + u) * 256] = acc[t][u];
+            else tot[t][u] += acc[t][u];
+            acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          }
+        ++part;
+        bound = steps * (part + 1) / parts;
+      }
+    }
   };
 
-  xload(s0, I0);
   wload(s0, I0);
   wload(s0 + 1, I1);
-  xload(s0 + 2, I1);
   wload(s0 + 2, I2);
   wload(s0 + 3, I3);
-  xstore(s0, I0, true);
+  if constexpr (NORM) {
+    __builtin_amdgcn_sched_barrier(0);
+    rows_inv_rms<BM / (4 * KG)>(a, m0, BM, gwave, 4 * KG, lane, rinv);
+    __syncthreads();
+    rs = rinv[srow];
+  }
+  xload(s0, I0);
+  xload(s0 + 2, I1);
+  xstore(s0, I0);
   __syncthreads();
-  // Straight-line pairs: no branch, so that the loads of the rings stay in flight across iterations.
   // Entering a pair: chunk st in buffer 0, chunk st + 2 in register set 1, weights of st .. st + 3.
   for (int i = 0, st = s0; i < pairs; ++i, st += 4) {
-#pragma unroll
-    for (int t = 0; t < RT; ++t)
-#pragma unroll
-      for (int u = 0; u < CT; ++u) acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
     xload(st + 4, I0);
     __builtin_amdgcn_sched_barrier(0);
-    mma(I0, I0);
+    mma(I0, I0, st);
     wload(st + 4, I0);
-    mma(I0, I1);
+    mma(I0, I1, st + 1);
     wload(st + 5, I1);
     __builtin_amdgcn_sched_barrier(0);
-    xstore(st + 2, I1, true);
+    xstore(st + 2, I1);
     __syncthreads();
     xload(st + 6, I1);
     __builtin_amdgcn_sched_barrier(0);
-    mma(I1, I0);
+    mma(I1, I0, st + 2);
     wload(st + 6, I2);
-    mma(I1, I1);
+    mma(I1, I1, st + 3);
     wload(st + 7, I3);
     __builtin_amdgcn_sched_barrier(0);
-    xstore(st + 4, I0, i + 1 < pairs);
-#pragma unroll
-    for (int t = 0; t < RT; ++t)
-#pragma unroll
-      for (int u = 0; u < CT; ++u) tot[t][u] += acc[t][u];
+    xstore(st + 4, I0);
     __syncthreads();
   }
 
-  // The row's sum of squares over its staging threads: partial sums at rsum[part][row]
-  constexpr int NP = 2 * KG;
-  if constexpr (NORM) {
-    ss += __shfl_xor(ss, 1, 64);
-    ss += __shfl_xor(ss, 2, 64);
-    if (slot == 0) rsum[(2 * grp + sp) * BM + srow] = ss;
-  }
-  if constexpr (KG > 1) {  // the other groups' sums, through their own staging buffers, in group order
-    f32x4_t *m = reinterpret_cast<f32x4_t *>(lds) + tid;
-    if (grp > 0) {
+  if constexpr (KG > 1) {  // every image was written before the loop's last barrier
+    if (grp) return;
+    for (int p = half; p < parts; ++p)
 #pragma unroll
       for (int t = 0; t < RT; ++t)
 #pragma unroll
-        for (int u = 0; u < CT; ++u) m[grp * 2 * BUF + (t * CT + u) * 256] = tot[t][u];
-    }
-    __syncthreads();
-    if (grp > 0) return;
-#pragma unroll
-    for (int k = 1; k < KG; ++k)
-#pragma unroll
-      for (int t = 0; t < RT; ++t)
-#pragma unroll
-        for (int u = 0; u < CT; ++u) tot[t][u] += m[k * 2 * BUF + (t * CT + u) * 256];
-  } else if constexpr (NORM) {
-    __syncthreads();
-  }
-  float inv[RT];
-#pragma unroll
-  for (int t = 0; t < RT; ++t) {
-    inv[t] = 1.f;
-    if constexpr (NORM) {
-      float s = rsum[16 * t + li];
-#pragma unroll
-      for (int i = 1; i < NP; ++i) s += rsum[i * BM + 16 * t + li];
-      inv[t] = 1.0f / sqrtf(s / (float)a.K + a.eps);
-    }
+        for (int u = 0; u < CT; ++u) tot[t][u] += image[((p - half) * RT * CT + t * CT + u) * 256];
   }
 
   // Lane (li, kb) holds columns 4 kb .. + 3 of row li of each tile.  Every operand is loaded before
@@ -326,8 +314,6 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
       }
     }
   }
-  constexpr int LDI = 36;  // SPLIT: this wave's 32 x 32 outputs, in the staging space of group 0
-  float *image = reinterpret_cast<float *>(lds) + wave * BM * LDI;
 #pragma unroll
   for (int t = 0; t < RT; ++t) {
     const int m = m0 + 16 * t + li;
@@ -337,11 +323,12 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
       float v[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        v[e] = tot[t][u][e];
-        if constexpr (NORM) v[e] *= inv[t];
+        if constexpr (PARTS) v[e] = tot[t][u][e];
+        else v[e] = acc[t][u][e];
         if constexpr (SW) {
-          float up = tot[t][u + OT][e];
-          if constexpr (NORM) up *= inv[t];
+          float up;
+          if constexpr (PARTS) up = tot[t][u + OT][e];
+          else up = acc[t][u + OT][e];
           v[e] = v[e] / (1.0f + expf(-v[e])) * up;
         }
       }
@@ -352,10 +339,6 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
         b[e] = BIAS ? bv[u][e] : 0.f;
         c[e] = EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE ? cv[u][e] : 1.f;
         c2[e] = EPI == EPI_RES_SNAKE ? c2v[u][e] : 1.f;
-      }
-      if constexpr (SPLIT) {
-        split_put(a, v, r, image + (16 * t + li) * LDI + 16 * u + 4 * kb, m, n, blockIdx.z, vec);
-        continue;
       }
       tile_epilogue<EPI>(a, v, r, b, c, c2);
       if (m >= a.M || n >= a.N) continue;
@@ -369,34 +352,30 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
       }
     }
   }
-  if constexpr (SPLIT) split_add<BM, 32, LDI>(a, image, m0, n0, lane);
 }
 
-// Up to 64 rows (MT tiles of 16): a workgroup per 16-column tile (SwiGLU: a gate tile and its up
-// tile) and, with GemmArgs::split2, K half.  Eight waves take contiguous shares of K; each issues the
-// loads of PS steps together, weights and X straight from global memory in matrix-core order, and the
-// waves' sums meet in LDS in wave order.  With so few rows a launch lasts as long as one workgroup:
-// one memory round trip, plus what its CU can load (64 bytes a clock, rows x K x 4 of X above all) and
-// split.  So the columns are spread as thin as the matrix cores take them, over every CU, nothing is
-// waited for between a wave's loads, and no second launch adds up partial sums.
-// Same arithmetic as k_gemm_tile: the matrix cores take x * gain, the sums are scaled by 1 / rms.
-template <int EPI, bool NORM, int MT, bool SPLIT>
-__global__ __launch_bounds__(512, 2) void k_gemm_rows(GemmArgs a, int vec) {
-  static_assert(!SPLIT || EPI == EPI_RESIDUAL, "the K halves meet in a residual sum");
+// Few rows: a workgroup per 16-column tile (SwiGLU: a gate tile and its up tile) and MT tiles of 16 rows.
+// A wave's job is one K part (GemmArgs::k_parts): it issues the loads of PS k steps together, weights and X
+// straight from global memory in matrix-core order, and leaves its sums in LDS, where the
+// parts are added in part order.  With so few rows a launch lasts as long as one workgroup: one memory
+// round trip or two, plus what its CU can load (64 bytes a clock, rows x K x 4 of X above all) and split.
+// So the columns are spread as thin as the matrix cores take them, over every CU, nothing is waited
+// for between a wave's loads, and no second launch adds up the parts.
+constexpr int rows_waves(int MT) { return MT == 1 ? 16 : 8; }  // at most: registers for the loads in flight
+
+template <int EPI, bool NORM, int MT>
+__global__ __launch_bounds__(64 * rows_waves(MT)) void k_gemm_rows(GemmArgs a, int vec) {
   constexpr bool SW = EPI == EPI_SWIGLU;
-  constexpr int T = SW ? 2 : 1, W = 8, PS = MT == 1 ? 8 : (MT == 4 && SW && NORM ? 3 : 4);
+  constexpr int T = SW ? 2 : 1, PS = MT > 1 ? 6 : SW ? 3 : NORM ? 4 : 6;
   constexpr bool RES = EPI == EPI_RESIDUAL || EPI == EPI_AFFINE_RES || EPI == EPI_RES_SNAKE;
   constexpr bool BIAS = EPI == EPI_BIAS || EPI == EPI_AFFINE_RES || EPI == EPI_BIAS_GELU ||
                         EPI == EPI_BIAS_SILU || EPI == EPI_RES_SNAKE;
-  __shared__ f32x4_t part[W][MT * T][64];
-  __shared__ float ssq[W][MT * 16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, kb = lane >> 4;
-  const int ntile = (a.N + 15) / 16, steps = a.K / 32;
-  const int h0 = SPLIT ? (int)((int64_t)steps * blockIdx.y / 2) : 0;
-  const int h1 = SPLIT ? (int)((int64_t)steps * (blockIdx.y + 1) / 2) : steps;
-  const int s0 = h0 + (h1 - h0) * wave / W, s1 = h0 + (h1 - h0) * (wave + 1) / W;
-
-  const int r0 = 16 * MT * blockIdx.z;  // first row
+  extern __shared__ f32x4_t part[];  // [k_parts][MT * T][64], then row scales [16 MT]
+  const int tid = threadIdx.x, lane = tid & 63, li = lane & 15, kb = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
+  const int ntile = (a.N + 15) / 16, steps = a.K / 32, parts = a.k_parts;
+  const int r0 = 16 * MT * blockIdx.y;  // first row
+  float *rinv = reinterpret_cast<float *>(part + parts * MT * T * 64);
 
   // This thread's four outputs (threads below 64 MT): row om, columns on .. on + 3; operands first
   const int ot = min(tid >> 6, MT - 1), om = r0 + 16 * ot + li, on = blockIdx.x * 16 + 4 * kb, cm = min(om, a.M - 1);
@@ -419,36 +398,58 @@ __global__ __launch_bounds__(512, 2) void k_gemm_rows(GemmArgs a, int vec) {
     }
   }
 
-  const float *xp[MT];
-#pragma unroll
-  for (int t = 0; t < MT; ++t) xp[t] = a.X + (size_t)min(r0 + 16 * t + li, a.M - 1) * a.ldx + 8 * kb;
   const uint16_t *wp[T];
 #pragma unroll
   for (int u = 0; u < T; ++u) wp[u] = a.W + (size_t)(blockIdx.x + u * ntile) * steps * 512 + lane * 8;
-
-  // The high terms' sum apart from the two small ones': a third of the roundings at full magnitude
-  f32x4_t acc[MT][T], low[MT][T];
+  bf16x8_t w[PS][T];
+  auto wload = [&](int p0, int s1) {
 #pragma unroll
-  for (int t = 0; t < MT; ++t)
+    for (int i = 0; i < PS; ++i)
 #pragma unroll
-    for (int u = 0; u < T; ++u) acc[t][u] = low[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  float ss[MT] = {};
-  for (int p0 = s0; p0 < s1; p0 += PS) {
-    f32x4_t x[PS][MT][2], g[NORM ? PS : 1][2];
-    bf16x8_t w[PS][T];
+      for (int u = 0; u < T; ++u)
+        w[i][u] = *reinterpret_cast<const bf16x8_t *>(wp[u] + (size_t)min(p0 + i, s1 - 1) * 512);
+  };
+  const float *xp[MT];
 #pragma unroll
-    for (int i = 0; i < PS; ++i) {
-      const int st = min(p0 + i, s1 - 1);
+  for (int t = 0; t < MT; ++t) xp[t] = a.X + (size_t)min(r0 + 16 * t + li, a.M - 1) * a.ldx + 8 * kb;
+  f32x4_t x[PS][MT][2];
+  auto xload = [&](int p0, int s1) {
+#pragma unroll
+    for (int i = 0; i < PS; ++i)
 #pragma unroll
       for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int h = 0; h < 2; ++h) x[i][t][h] = *reinterpret_cast<const f32x4_t *>(xp[t] + 32 * st + 4 * h);
-      if constexpr (NORM) {
+        for (int h = 0; h < 2; ++h)
+          x[i][t][h] = *reinterpret_cast<const f32x4_t *>(xp[t] + 32 * min(p0 + i, s1 - 1) + 4 * h);
+  };
+  // A wave's parts, PS steps at a time.  The first loads are under way before the norm's: together the waves'
+  // cover X or most of it, and the norm finds it in the L2.  A wave past the last part loads as the last
+  // does, and works on none.
+  int z = min(wave, parts - 1), p0 = steps * z / parts, s1 = steps * (z + 1) / parts;
+  wload(p0, s1);
+  xload(p0, s1);
+  float rs[MT];
+  if constexpr (NORM) {
+    __builtin_amdgcn_sched_barrier(0);
+    rows_inv_rms<16 * MT / rows_waves(MT)>(a, r0, 16 * MT, wave, waves, lane, rinv);
+    __syncthreads();
 #pragma unroll
-        for (int h = 0; h < 2; ++h) g[i][h] = *reinterpret_cast<const f32x4_t *>(a.gamma + 32 * st + 8 * kb + 4 * h);
-      }
+    for (int t = 0; t < MT; ++t) rs[t] = rinv[16 * t + li];
+  }
+  f32x4_t acc[MT][T];
 #pragma unroll
-      for (int u = 0; u < T; ++u) w[i][u] = *reinterpret_cast<const bf16x8_t *>(wp[u] + (size_t)st * 512);
+  for (int t = 0; t < MT; ++t)
+#pragma unroll
+    for (int u = 0; u < T; ++u) acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  z = wave;
+  while (z < parts) {
+    f32x4_t g[NORM ? PS : 1][2];
+    if constexpr (NORM) {
+#pragma unroll
+      for (int i = 0; i < PS; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          g[i][h] = *reinterpret_cast<const f32x4_t *>(a.gamma + 32 * min(p0 + i, s1 - 1) + 8 * kb + 4 * h);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -458,34 +459,36 @@ __global__ __launch_bounds__(512, 2) void k_gemm_rows(GemmArgs a, int vec) {
       for (int t = 0; t < MT; ++t) {
         float v[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = x[i][t][e >> 2][e & 3];
-        if constexpr (NORM) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) ss[t] = __builtin_fmaf(v[e], v[e], ss[t]);
-#pragma unroll
-          for (int e = 0; e < 8; ++e) v[e] *= g[i][e >> 2][e & 3];
+        for (int e = 0; e < 8; ++e) {
+          v[e] = x[i][t][e >> 2][e & 3];
+          if constexpr (NORM) v[e] = (v[e] * rs[t]) * g[i][e >> 2][e & 3];
         }
         bf16x8_t hi, mid, lo;
-        split_bf16x8_nc(v, hi, mid, lo);
+        split_bf16x8_rn(v, hi, mid, lo);
 #pragma unroll
         for (int u = 0; u < T; ++u) {
-          low[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i][u], lo, low[t][u], 0, 0, 0);
-          low[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i][u], mid, low[t][u], 0, 0, 0);
+          acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i][u], lo, acc[t][u], 0, 0, 0);
+          acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i][u], mid, acc[t][u], 0, 0, 0);
           acc[t][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i][u], hi, acc[t][u], 0, 0, 0);
         }
       }
     }
-  }
+    p0 += PS;
+    if (p0 >= s1) {
 #pragma unroll
-  for (int t = 0; t < MT; ++t) {
+      for (int t = 0; t < MT; ++t)
 #pragma unroll
-    for (int u = 0; u < T; ++u) part[wave][t * T + u][lane] = acc[t][u] + low[t][u];
-    if constexpr (NORM) {
-      float q = ss[t];
-      q += __shfl_xor(q, 16, 64);
-      q += __shfl_xor(q, 32, 64);
-      if (kb == 0) ssq[wave][16 * t + li] = q;
+        for (int u = 0; u < T; ++u) {
+          part[((z * MT + t) * T + u) * 64 + lane] = acc[t][u];
+          acc[t][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+      z += waves;
+      if (z >= parts) break;
+      p0 = steps * z / parts;
+      s1 = steps * (z + 1) / parts;
     }
+    wload(p0, s1);
+    xload(p0, s1);
   }
   __syncthreads();
   if (tid >= 64 * MT) return;
@@ -493,31 +496,15 @@ __global__ __launch_bounds__(512, 2) void k_gemm_rows(GemmArgs a, int vec) {
   {
     f32x4_t s[T];
 #pragma unroll
-    for (int u = 0; u < T; ++u) {
-      s[u] = part[0][ot * T + u][lane];
+    for (int u = 0; u < T; ++u) s[u] = part[(ot * T + u) * 64 + lane];
+    for (int z = 1; z < parts; ++z)
 #pragma unroll
-      for (int k = 1; k < W; ++k) s[u] += part[k][ot * T + u][lane];
-    }
-    float inv = 1.f;
-    if constexpr (NORM) {
-      float q = 0.f;
-#pragma unroll
-      for (int k = 0; k < W; ++k) q += ssq[k][16 * ot + li];
-      inv = 1.0f / sqrtf(q / (float)a.K + a.eps);
-    }
+      for (int u = 0; u < T; ++u) s[u] += part[((z * MT + ot) * T + u) * 64 + lane];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      v[e] = NORM ? s[0][e] * inv : s[0][e];
-      up[e] = NORM ? s[T - 1][e] * inv : s[T - 1][e];
+      v[e] = s[0][e];
+      up[e] = s[T - 1][e];
     }
-  }
-  if constexpr (SPLIT) {
-    float r[4], *image = reinterpret_cast<float *>(part[0][ot]);  // 16 x 16; this wave has read its sums
-#pragma unroll
-    for (int e = 0; e < 4; ++e) r[e] = rv[e];
-    split_put(a, v, r, image + li * 16 + 4 * kb, om, on, blockIdx.y, vec);
-    split_add<16, 16, 16>(a, image, r0 + 16 * ot, blockIdx.x * 16, lane);
-    return;
   }
   if (om >= a.M || on >= a.N) return;
   float *y = a.Y + (size_t)om * a.ldy + on;
@@ -553,57 +540,53 @@ int gemm_vec(const GemmArgs &a) {
 
 template <int EPI, bool NORM, int MT>
 hipError_t rows_launch(const GemmArgs &a, hipStream_t s) {
-  const dim3 grid((a.N + 15) / 16, a.split2 ? 2 : 1, (a.M + 16 * MT - 1) / (16 * MT));
-  if constexpr (EPI == EPI_RESIDUAL && !NORM) {
-    if (a.split2) {
-      hipLaunchKernelGGL((k_gemm_rows<EPI, NORM, MT, true>), grid, dim3(512), 0, s, a, gemm_vec(a));
-      return hipGetLastError();
-    }
-  }
-  hipLaunchKernelGGL((k_gemm_rows<EPI, NORM, MT, false>), grid, dim3(512), 0, s, a, gemm_vec(a));
+  constexpr int T = EPI == EPI_SWIGLU ? 2 : 1;
+  const dim3 grid((a.N + 15) / 16, (a.M + 16 * MT - 1) / (16 * MT));
+  // all waves for the norm; else as many as give them the same number of parts, one for each tile of outputs
+  const int rounds = (a.k_parts + rows_waves(MT) - 1) / rows_waves(MT);
+  const int waves = NORM ? rows_waves(MT) : std::max((a.k_parts + rounds - 1) / rounds, MT);
+  const size_t lds = (size_t)a.k_parts * MT * T * 1024 + (NORM ? 16 * MT * 4 : 0);
+  hipLaunchKernelGGL((k_gemm_rows<EPI, NORM, MT>), grid, dim3(64 * waves), lds, s, a, gemm_vec(a));
   return hipGetLastError();
 }
 
-template <int EPI, bool NORM, int KG, bool SPLIT>
-hipError_t tile_launch_split(const GemmArgs &a, hipStream_t s) {
-  const int out = EPI == EPI_SWIGLU ? 64 : 128;
-  const dim3 grid((a.N + out - 1) / out, (a.M + 31) / 32, SPLIT ? 2 : 1);
-  const size_t lds = (size_t)KG * 2 * 3 * 2 * 32 * 64 + (NORM ? (size_t)KG * 2 * 32 * 4 : 0);
-  if (!SPLIT && a.K % (128 * KG))
-    hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, KG, !SPLIT, SPLIT>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
-  else
-    hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, KG, false, SPLIT>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
-  return hipGetLastError();
-}
-
-template <int EPI, bool NORM, int KG>
+template <int EPI, bool NORM, int KG, int CT, bool TAIL, bool PARTS>
 hipError_t tile_launch(const GemmArgs &a, hipStream_t s) {
-  if constexpr (EPI == EPI_RESIDUAL && !NORM) {
-    if (a.split2) return tile_launch_split<EPI, NORM, KG, true>(a, s);
-  }
-  return tile_launch_split<EPI, NORM, KG, false>(a, s);
+  const int out = EPI == EPI_SWIGLU ? 64 : 64 * CT;
+  const dim3 grid((a.N + out - 1) / out, (a.M + 31) / 32);
+  const size_t lds = (size_t)KG * 2 * 3 * 2 * 32 * 64 + 32 * 4 + (KG > 1 ? (size_t)(a.k_parts / 2) * CT * 8192 : 0);
+  hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, KG, CT, TAIL, PARTS>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
+  return hipGetLastError();
 }
 
-// Up to 64 rows: k_gemm_rows (whose X traffic per 16 columns is all rows: at 137 rows x 2048 it took
-// twice k_gemm_tile's time), the rows in as many parts as bring the workgroups to one per CU at most (O
-// and down at 41 rows, 128 workgroups of three tiles: prefill 1.58 -> 1.46 ms with 256 of two and one;
-// with 384 of one tile each 1.65, a CU then waits for two).  More: k_gemm_tile, with two K groups a block
-// where there are fewer blocks than CUs (137 rows, O and down of the 1.7B shape: prefill 4.63 -> 4.12 ms;
-// with 544 blocks one group is 3% faster; four groups measured as two).
+// One K part: no groups.  Parts: two groups a block where there are fewer blocks than CUs, of 64 columns
+// where those find a CU each (O and down of the 1.7B shape at 137 rows, 80 blocks of 128 columns: 30 -> 25 us;
+// O and down of the 0.6B shape at 521 rows, 136 blocks: 23 -> 25, QKV at 137 rows, 160 blocks: 22 -> 27).  16 parts of 128
+// columns leave no LDS for the second group's sums.
+template <int EPI, bool NORM>
+hipError_t tile_parts(const GemmArgs &a, hipStream_t s) {
+  if (a.k_parts == 1)
+    return a.K % 128 == 0 ? tile_launch<EPI, NORM, 1, 2, false, false>(a, s)
+                          : tile_launch<EPI, NORM, 1, 2, true, false>(a, s);
+  constexpr int out = EPI == EPI_SWIGLU ? 64 : 128;
+  const int64_t blocks = (int64_t)((a.N + out - 1) / out) * ((a.M + 31) / 32);
+  if constexpr (EPI != EPI_SWIGLU)
+    if (2 * blocks <= 256) return tile_launch<EPI, NORM, 2, 1, true, true>(a, s);
+  if (blocks < 256 && a.k_parts <= 12) return tile_launch<EPI, NORM, 2, 2, true, true>(a, s);
+  return tile_launch<EPI, NORM, 1, 2, true, true>(a, s);
+}
+
+// One row tile, or few 16 x 16 output tiles (two a CU) and five or more K parts for the waves to share:
+// k_gemm_rows, the rows in workgroups of one tile up to a workgroup a CU, of two past that.  Else k_gemm_tile.
+// Prefill in us with k_gemm_rows to twice the tiles and at any number of parts, and so: 41 rows 1,783 and
+// 1,710, 80 rows 2,730 and 2,165, 200 rows 3,160 and 2,740 (0.6B shape), 24 rows 2,820 and 2,330, 41 rows
+// 4,230 and 2,980 (1.7B shape); with it only from 16 parts on, 24 rows 1,705 and 1,642 (0.6B).
 template <int EPI, bool NORM>
 hipError_t tile_shape(const GemmArgs &a, hipStream_t s) {
-  if (a.M <= 64) {
-    const int cols = (a.N + 15) / 16 * (a.split2 ? 2 : 1), tiles = (a.M + 15) / 16;
-    const int z = std::min(tiles, std::max(1, 256 / cols));
-    switch ((tiles + z - 1) / z) {
-      case 1: return rows_launch<EPI, NORM, 1>(a, s);
-      case 2: return rows_launch<EPI, NORM, 2>(a, s);
-      case 3: return rows_launch<EPI, NORM, 3>(a, s);
-      default: return rows_launch<EPI, NORM, 4>(a, s);
-    }
-  }
-  const int n = EPI == EPI_SWIGLU ? 2 * a.N : a.N, blocks = (a.M + 31) / 32 * ((n + 127) / 128) * (a.split2 ? 2 : 1);
-  return blocks >= 256 || a.K < 128 ? tile_launch<EPI, NORM, 1>(a, s) : tile_launch<EPI, NORM, 2>(a, s);
+  const int cols = (a.N + 15) / 16;
+  const int64_t tiles = ((int64_t)a.M + 15) / 16;
+  if (tiles > 1 && (a.k_parts < 5 || tiles * cols > 512)) return tile_parts<EPI, NORM>(a, s);
+  return tiles == 1 || tiles * cols <= 256 ? rows_launch<EPI, NORM, 1>(a, s) : rows_launch<EPI, NORM, 2>(a, s);
 }
 
 template <int EPI>
@@ -613,17 +596,28 @@ hipError_t tile_norm(const GemmArgs &a, hipStream_t s) {
 
 }  // namespace
 
-hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t s) {
-  if (a.M <= 0 || a.N <= 0 || a.K <= 0 || a.K % 32 || a.ldx % 4 || !a.w_packed || !a.X || !a.W || !a.Y ||
-      reinterpret_cast<uintptr_t>(a.X) % 16 || reinterpret_cast<uintptr_t>(a.W) % 16 ||
-      reinterpret_cast<uintptr_t>(a.gamma) % 16)
+int gemm_k_parts(int epi, int M, int N, int K) {
+  const bool sw = epi == EPI_SWIGLU;
+  auto blocks_of = [&](int cols, int rows) { return (int64_t)((N + cols - 1) / cols) * ((M + rows - 1) / rows); };
+  int64_t blocks;
+  if (M >= 128 && (!sw || N % 64 == 0)) blocks = blocks_of(sw ? 64 : (N % 128 && N % 96 == 0 ? 96 : 128), 128);
+  else blocks = blocks_of(sw ? 128 : 256, M <= 16 ? 16 : 32);
+  if (blocks >= 128) return 1;
+  int p = std::min({(int)((256 + blocks - 1) / blocks), K / 128, kGemmMaxParts});
+  while (p > 1 && (int64_t)p * M * N * (sw ? 2 : 1) > (int64_t)4 << 20) --p;
+  return std::max(p, 1);
+}
+
+hipError_t launch_gemm(int epi, const GemmArgs &args, hipStream_t s) {
+  GemmArgs a = args;
+  if (a.k_parts == 0) a.k_parts = 1;
+  if (a.M <= 0 || a.N <= 0 || a.K <= 0 || a.K % 32 || a.ldx % 4 || !a.w_packed || !a.X || !a.W || !a.Y || a.split2 ||
+      a.k_parts < 1 || a.k_parts > std::min(a.K / 32, kGemmMaxParts) || reinterpret_cast<uintptr_t>(a.X) % 16 ||
+      reinterpret_cast<uintptr_t>(a.W) % 16 || reinterpret_cast<uintptr_t>(a.gamma) % 16)
     return hipErrorInvalidValue;
   const bool res = epi == EPI_RESIDUAL || epi == EPI_AFFINE_RES || epi == EPI_RES_SNAKE;
   const bool bias = epi == EPI_BIAS || epi == EPI_BIAS_GELU || epi == EPI_BIAS_SILU || epi == EPI_RES_SNAKE;
   if ((res && !a.res) || (bias && !a.bias)) return hipErrorInvalidValue;
-  if (a.split2 && (epi != EPI_RESIDUAL || a.gamma || a.M > gemm_split_rows(a.N) || !a.res_zero || a.K < 64 ||
-                   (a.M > 64 && a.K % 512)))
-    return hipErrorInvalidValue;
   switch (epi) {
     case EPI_STORE: return tile_norm<EPI_STORE>(a, s);
     case EPI_RESIDUAL: return tile_norm<EPI_RESIDUAL>(a, s);

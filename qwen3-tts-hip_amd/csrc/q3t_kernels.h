@@ -66,13 +66,12 @@ int attn_rows_chunk_len(int cap);
 // accumulate) for many rows (q3t_gemm.hip): prompt prefill, text projection, codec linears.
 // Requires K % 32 == 0, ldx % 4 == 0, 16-byte aligned X, W, gamma.
 hipError_t launch_gemm(int epi, const GemmArgs &a, hipStream_t stream);
-// GemmArgs::split2 (EPI_RESIDUAL without RMSNorm, K >= 64, past 64 rows K % 512 == 0): up to this many rows, where the two halves of
-// all blocks of 32 x 128 outputs find a CU each (or 64 rows).  137 rows of the 1.7B shape, 80 blocks in
-// 256 CUs: prefill 3.41 -> 2.92 ms; 521 rows of the 0.6B shape, 136 blocks: 3.57 -> 3.62 ms, not split.
-constexpr int gemm_split_rows(int N) {
-  const int rows = 32 * (128 / ((N + 127) / 128));
-  return rows > 64 ? rows : 64;
-}
+// The K parts of a GEMM of this shape, a function of the shape alone: as many as bring 128-row (below 128
+// rows 16- or 32-row) blocks of columns to 256 workgroups, four k steps a part, 16 parts and 4 M sums at most.
+// What a prompt or a codec window returns is defined by it, so it stays as it is whatever the kernels
+// that compute the sums make of it.
+int gemm_k_parts(int epi, int M, int N, int K);
+constexpr int kGemmMaxParts = 16;
 // The same product for M <= 16 rows (batched decode); norm = fused RMSNorm of the rows with
 // gain gamma.  Requires K = 512 * c, c in {1, 2, 3, 4, 6, 8, 12}
 // (K <= 2048 with norm).

@@ -30,32 +30,6 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
   return (uint16_t)(u >> 16);
 }
 
-// Cross-lane reductions on DPP (data-parallel primitives: VALU lane permutes, no LDS round
-// trip).  Each step adds a permuted copy: quad_perm [1,0,3,2] and [2,3,0,1] (quads),
-// row_half_mirror and row_mirror (rows of 16), then row_bcast:15 / row_bcast:31 fold the
-// four rows into lane 63.  The order is fixed, so results are deterministic.
-template <int CTRL, int ROWS = 0xf>
-__device__ __forceinline__ float dpp_f(float v, float fill) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, fill), __builtin_bit_cast(int, v),
-                                                               CTRL, ROWS, 0xf, false));
-}
-
-// Sum over each row of 16 lanes, in every lane of the row.
-__device__ __forceinline__ float row16_sum(float v) {
-  v += dpp_f<0xB1>(v, 0.f);
-  v += dpp_f<0x4E>(v, 0.f);
-  v += dpp_f<0x141>(v, 0.f);
-  v += dpp_f<0x140>(v, 0.f);
-  return v;
-}
-
-__device__ __forceinline__ float wave_sum(float v) {
-  v = row16_sum(v);
-  v += dpp_f<0x142, 0xa>(v, 0.f);
-  v += dpp_f<0x143, 0xc>(v, 0.f);
-  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
-}
-
 __device__ __forceinline__ float wave_max(float v) {
   v = fmaxf(v, dpp_f<0xB1>(v, v));
   v = fmaxf(v, dpp_f<0x4E>(v, v));

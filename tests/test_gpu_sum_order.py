@@ -102,6 +102,21 @@ def test_frame_gemm(tiny, golden, M, N, K):
     assert gemm_digest(tiny, M, N, K) == golden[f"gemm {M} {N} {K}"]
 
 
+@pytest.mark.parametrize("M,N,K", GEMMS)
+def test_gemm(tiny, golden, M, N, K):
+    print(f"[gpu] sum order, gemm M={M} N={N} K={K}", flush=True)
+    assert gemm_digest(tiny, M, N, K) == golden[f"gemm {M} {N} {K}"]
+
+
+@pytest.mark.parametrize("spec", ["tiny", "0.6b"])
+def test_prompt_rows(models, golden, spec):
+    _, eng = _engine(models, spec, text=True)
+    with eng:
+        for n in PROMPTS:
+            print(f"[gpu] sum order, prompt {spec} ids={n}", flush=True)
+            assert prompt_digest(eng, n) == golden[f"prompt {spec} {n}"], n
+
+
 if __name__ == "__main__":
     from conftest import _ModelCache
 
