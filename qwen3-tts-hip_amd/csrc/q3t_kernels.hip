@@ -1745,8 +1745,8 @@ __global__ __launch_bounds__(256) void k_attn_prefix(PrefillAttnArgs a) {
   }
 }
 
-// 8 consecutive cache elements as loaded, converted where they are used: a load can be in flight
-// across other work.
+// Consecutive cache elements as loaded, converted where they are used: a load can be in flight across
+// other work.
 template <typename KVT>
 struct KvRaw8;
 template <>
@@ -1764,30 +1764,48 @@ struct KvRaw8<uint16_t> {
   __device__ __forceinline__ void load(const uint16_t *p) { w = *reinterpret_cast<const u32x4 *>(p); }
   __device__ __forceinline__ float operator[](int i) const { return (i & 1) ? bf_hi(w[i >> 1]) : bf_lo(w[i >> 1]); }
 };
+template <typename KVT>
+struct KvRaw2;
+template <>
+struct KvRaw2<float> {
+  f32x2_t a;
+  __device__ __forceinline__ void load(const float *p) { a = *reinterpret_cast<const f32x2_t *>(p); }
+  __device__ __forceinline__ float operator[](int i) const { return a[i]; }
+};
+template <>
+struct KvRaw2<uint16_t> {
+  uint32_t w;
+  __device__ __forceinline__ void load(const uint16_t *p) { w = *reinterpret_cast<const uint32_t *>(p); }
+  __device__ __forceinline__ float operator[](int i) const { return i ? bf_hi(w) : bf_lo(w); }
+};
 
 // One workgroup per unit (stream s, query head hq, query rows q0 .. q0 + 15), units in
 // PrefillBatchArgs::unit0 order: per stream, the last query block first (the longest causal
-// range).  The four waves take every fourth 16-key tile and merge at the end: a unit is a serial
-// chain of tiles (load, 32 dependent matrix-core steps, softmax, 32 more), and a prompt has few
-// units against 1,024 SIMDs, so the longest chain sets the time (521 rows, 16 heads, bf16 cache:
-// 79 us as one wave per unit, ~25 us so).  Each wave's next tile is in flight while it works on
-// this one.  v_mfma_f32_16x16x4_f32 (fp32 products and sums):
-//   S^T = K Q^T per 16-key tile: lane (li, kk) supplies key row li and query row li, dims
+// range).  A query's output is one chain over its 16-key tiles in order, an online softmax: what the
+// attention returns is defined by it (launch_gemm says why).  A unit as one wave is a serial chain of
+// load, 32 dependent matrix-core steps, softmax, 32 more per tile, and a prompt has few units against
+// 1,024 SIMDs (521 rows, 16 heads, bf16 cache: 79 us).  So four waves share a unit without touching
+// the chain's order, four tiles a round (29 us; with a chain of its own for each wave, merged at the
+// end, 25):
+//   * Wave w scores tile 4 r + w (S^T = K Q^T): lane (li, kk) supplies key row li and query row li, dims
 //     32 kk + s at step s (32 steps: the four lane groups cover the 128 dims in quarters), and
-//     holds scores of keys 4 kk + e (e = 0..3) for query li.
-//   O^T += V^T P^T: step s' takes keys 4 kk + s' (lane group kk), so each lane's own score
-//     e = s' is its B operand; A row i of output tile t is dim 8 i + t, so a lane reads 8
-//     consecutive elements of a value row and ends up holding dims 32 kk .. 32 kk + 31 of query li.
-//   Online softmax per query over the wave's tiles: the tile max over the four lane groups by lane
-//     exchanges, per-lane partial sums of p (added across the groups at the end).
-//   Merge: (m, l, O) of the four waves through LDS in wave order; wave w stores dims
-//     32 kk + 8 w .. + 7 of each query.
+//     holds scores of keys 4 kk + e (e = 0..3) for query li.  The tile's maximum per query goes to LDS.
+//   * With the four maxima every wave follows the running maximum, and wave w turns its scores into p
+//     and the tile's rescaling factor, in LDS.
+//   * Wave w runs the chain O^T = O^T corr + V^T P^T over the round's tiles for its 32 dims: step s' takes
+//     keys 4 kk + s' (lane group kk), so a lane reads its own p's of the scoring lane's place; A row i of
+//     output tile t is dim 32 w + 2 i + t, so a lane reads 2 consecutive elements of a value row (16 lanes
+//     a 128-byte line) and ends up holding dims 32 w + 8 kk .. + 7 of query li.  Each wave also keeps l,
+//     lane sums of p that are added across the lane groups at the end.
+// The next round's K and V are in flight while a round is worked on.  v_mfma_f32_16x16x4_f32: fp32
+// products and sums.
 template <typename KVT>
 __global__ __launch_bounds__(256, 2) void k_attn_prefill(PrefillBatchArgs a) {
   constexpr int D = 128, W = 4;
-  __shared__ float mo[W][32][64];  // [wave][8 e' + t]: element (tile t, e') of each lane
-  __shared__ float mm[W][16], ml[W][16];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, kk = lane >> 4;
+  __shared__ f32x4_t ps[W][64];              // p of tile w, as its scoring lanes hold it
+  __shared__ float mts[W][16], corrs[W][16];  // per tile of the round and query: maximum, rescaling factor
+  const int lane = threadIdx.x & 63, li = lane & 15, kk = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int u = blockIdx.x;
   int sg = 0;
   while (sg + 1 < a.nseg && u >= a.unit0[sg + 1]) ++sg;
@@ -1800,14 +1818,19 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(PrefillBatchArgs a) {
   const KVT *vb = reinterpret_cast<const KVT *>(a.vcache[sg]) + (size_t)kvh * a.cap * D;
   const int nkt = (min(q0 + 16, P) + 15) / 16;  // key tiles up to the block's last row
 
-  KvRaw8<KVT> kv[4], vv[4], kn[4], vn[4];
-  auto load = [&](int kt, KvRaw8<KVT> *k, KvRaw8<KVT> *v) {
-    const KVT *kp = kb + (size_t)min(16 * kt + li, P - 1) * D + 32 * kk;
+  KvRaw8<KVT> kv[4];
+  KvRaw2<KVT> vv[W][4];
+  auto load = [&](int kt0) {  // the round's tiles from kt0 on, clamped to the last
+    const KVT *kp = kb + (size_t)min(16 * (kt0 + wave) + li, P - 1) * D + 32 * kk;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) k[c].load(kp + 8 * c);
+    for (int c = 0; c < 4; ++c) kv[c].load(kp + 8 * c);
 #pragma unroll
-    for (int s2 = 0; s2 < 4; ++s2) v[s2].load(vb + (size_t)min(16 * kt + 4 * kk + s2, P - 1) * D + 8 * li);
+    for (int j = 0; j < W; ++j)
+#pragma unroll
+      for (int s2 = 0; s2 < 4; ++s2)
+        vv[j][s2].load(vb + (size_t)min(16 * (kt0 + j) + 4 * kk + s2, P - 1) * D + 32 * wave + 2 * li);
   };
+  load(0);
   float q[32];
   {
     const float *qp = qkv + (size_t)min(q0 + li, P - 1) * a.ldq + hq * D + 32 * kk;
@@ -1817,74 +1840,74 @@ __global__ __launch_bounds__(256, 2) void k_attn_prefill(PrefillBatchArgs a) {
       q[4 * c] = x.x; q[4 * c + 1] = x.y; q[4 * c + 2] = x.z; q[4 * c + 3] = x.w;
     }
   }
-  f32x4_t o[8];
+  f32x4_t o[2];
 #pragma unroll
-  for (int t = 0; t < 8; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  for (int t = 0; t < 2; ++t) o[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
   float m_run = -FLT_MAX, l = 0.f;
   const int qrow = q0 + li;  // this lane's query (rows >= P are not stored)
-  if (wave < nkt) load(wave, kv, vv);
-  for (int kt = wave; kt < nkt; kt += W) {
-    if (kt + W < nkt) load(kt + W, kn, vn);
+  for (int kt0 = 0; kt0 < nkt; kt0 += W) {
     f32x4_t st = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int s1 = 0; s1 < 32; ++s1) st = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[s1 >> 3][s1 & 7], q[s1], st, 0, 0, 0);
     float p[4], mt = -FLT_MAX;
+    if (kt0 + wave < nkt) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int key = 16 * kt + 4 * kk + e;
-      p[e] = (key <= qrow && key < P) ? st[e] * a.scale : -FLT_MAX;
-      mt = fmaxf(mt, p[e]);
+      for (int s1 = 0; s1 < 32; ++s1) st = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[s1 >> 3][s1 & 7], q[s1], st, 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int key = 16 * (kt0 + wave) + 4 * kk + e;
+        p[e] = (key <= qrow && key < P) ? st[e] * a.scale : -FLT_MAX;
+        mt = fmaxf(mt, p[e]);
+      }
+      mt = fmaxf(mt, __builtin_bit_cast(float, lane_xor_u32<16>(__builtin_bit_cast(uint32_t, mt))));
+      mt = fmaxf(mt, __builtin_bit_cast(float, lane_xor_u32<32>(__builtin_bit_cast(uint32_t, mt))));
+      if (kk == 0) mts[wave][li] = mt;
     }
-    mt = fmaxf(mt, __builtin_bit_cast(float, lane_xor_u32<16>(__builtin_bit_cast(uint32_t, mt))));
-    mt = fmaxf(mt, __builtin_bit_cast(float, lane_xor_u32<32>(__builtin_bit_cast(uint32_t, mt))));
-    const float m_new = fmaxf(m_run, mt);
-    const float corr = expf(m_run - m_new);
-    float ps = 0.f;
+    __syncthreads();
+    // the running maximum before and after this wave's tile, and after the round
+    float m_before = m_run, m_new = m_run;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      p[e] = p[e] == -FLT_MAX ? 0.f : expf(p[e] - m_new);
-      ps += p[e];
+    for (int j = 0; j < W; ++j) {
+      if (kt0 + j >= nkt) break;
+      if (j == wave) m_before = m_run;
+      m_run = fmaxf(m_run, mts[j][li]);
+      if (j == wave) m_new = m_run;
     }
-    l = l * corr + ps;
-    m_run = m_new;
+    if (kt0 + wave < nkt) {
+      const float corr = expf(m_before - m_new);
 #pragma unroll
-    for (int t = 0; t < 8; ++t) o[t] *= corr;
+      for (int e = 0; e < 4; ++e) p[e] = p[e] == -FLT_MAX ? 0.f : expf(p[e] - m_new);
+      ps[wave][lane] = f32x4_t{p[0], p[1], p[2], p[3]};
+      if (kk == 0) corrs[wave][li] = corr;
+    }
+    __syncthreads();
+    KvRaw2<KVT> vc[W][4];
 #pragma unroll
-    for (int s2 = 0; s2 < 4; ++s2)
+    for (int j = 0; j < W; ++j)
 #pragma unroll
-      for (int t = 0; t < 8; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[s2][t], p[s2], o[t], 0, 0, 0);
+      for (int s2 = 0; s2 < 4; ++s2) vc[j][s2] = vv[j][s2];
+    if (kt0 + W < nkt) load(kt0 + W);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      kv[c] = kn[c];
-      vv[c] = vn[c];
+    for (int j = 0; j < W; ++j) {
+      if (kt0 + j >= nkt) break;
+      const float corr = corrs[j][li];
+      const f32x4_t pj = ps[j][lane];
+      float sum = 0.f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sum += pj[e];
+      l = l * corr + sum;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) o[t] *= corr;
+#pragma unroll
+      for (int s2 = 0; s2 < 4; ++s2)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) o[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vc[j][s2][t], pj[s2], o[t], 0, 0, 0);
     }
   }
   l = pair32_sum(pair16_sum(l));
-  if (kk == 0) {
-    mm[wave][li] = m_run;
-    ml[wave][li] = l;
-  }
-#pragma unroll
-  for (int t = 0; t < 8; ++t)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) mo[wave][8 * e + t][lane] = o[t][e];
-  __syncthreads();
   if (qrow >= P) return;
-  float m = mm[0][li];
-#pragma unroll
-  for (int w = 1; w < W; ++w) m = fmaxf(m, mm[w][li]);
-  float lsum = 0.f, r[8] = {};
-#pragma unroll
-  for (int w = 0; w < W; ++w) {  // a wave without a tile has m = -FLT_MAX, l = 0: weight 0
-    const float f = expf(mm[w][li] - m);
-    lsum += ml[w][li] * f;
-#pragma unroll
-    for (int t = 0; t < 8; ++t) r[t] += mo[w][8 * wave + t][lane] * f;
-  }
-  const float inv = 1.0f / lsum;
-  float4 *op = reinterpret_cast<float4 *>(a.out + (size_t)(a.row0[sg] + qrow) * a.ldo + hq * D + 32 * kk + 8 * wave);
-  op[0] = make_float4(r[0] * inv, r[1] * inv, r[2] * inv, r[3] * inv);
-  op[1] = make_float4(r[4] * inv, r[5] * inv, r[6] * inv, r[7] * inv);
+  const float inv = 1.0f / l;
+  float4 *op = reinterpret_cast<float4 *>(a.out + (size_t)(a.row0[sg] + qrow) * a.ldo + hq * D + 32 * wave + 8 * kk);
+  op[0] = make_float4(o[0][0] * inv, o[1][0] * inv, o[0][1] * inv, o[1][1] * inv);
+  op[1] = make_float4(o[0][2] * inv, o[1][2] * inv, o[0][3] * inv, o[1][3] * inv);
 }
 
 // ---------------------------------------------------------------------------------------

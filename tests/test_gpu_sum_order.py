@@ -117,6 +117,16 @@ def test_prompt_rows(models, golden, spec):
             assert prompt_digest(eng, n) == golden[f"prompt {spec} {n}"], n
 
 
+@pytest.mark.parametrize("spec,kv_bf16,rows", PREFILLS)
+def test_prefill(models, golden, spec, kv_bf16, rows):
+    model, eng = _engine(models, spec, kv_bf16)
+    with eng:
+        for P in rows:
+            print(f"[gpu] sum order, prefill {spec} kv_bf16={kv_bf16} P={P}", flush=True)
+            got = prefill_digest(eng, model.spec.talker.hidden, P)
+            assert got == golden[f"prefill {spec} {kv_bf16} {P}"], P
+
+
 if __name__ == "__main__":
     from conftest import _ModelCache
 
