@@ -1,5 +1,5 @@
-// Device helpers shared by the kernels: wave sums, the three-term bf16 form of an fp32 value, and the
-// codec's Snake activation.
+// Device helpers shared by the kernels: wave sums, the block order of a tiled grid, the three-term bf16
+// form of an fp32 value, and the codec's Snake activation.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -37,6 +37,20 @@ __device__ __forceinline__ float wave_sum(float v) {
   v += dpp_f<0x142, 0xa>(v, 0.f);
   v += dpp_f<0x143, 0xc>(v, 0.f);
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+}
+
+// Row block mb and column block nb of this workgroup, nbx column blocks a row block, all on grid x (y ends
+// at 65,535 blocks, which a codec decode of 2,185 frames passes).  Few column blocks: each XCD
+// (workgroup id % 8) takes a contiguous range of row-major block tiles, so that its L2 reads only its own
+// rows, once for all column blocks.
+__device__ __forceinline__ void block_tile(int nbx, int &mb, int &nb) {
+  int t = blockIdx.x;
+  if (nbx <= 8) {
+    const int total = gridDim.x, xcd = t % 8, local = t / 8, C = (total + 7) / 8, r = total % 8;
+    t = (r == 0 || xcd < r) ? xcd * C + local : r * C + (xcd - r) * (C - 1) + local;
+  }
+  mb = t / nbx;
+  nb = t % nbx;
 }
 
 // x = hi + mid + lo, each bf16, exactly: hi is the upper half of x (its top 8 significant bits), x -

@@ -47,16 +47,8 @@ __global__ __launch_bounds__(256, 2) void k_codec_conv(CodecConvArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, kb = lane >> 4, wr = wave >> 1, wc = wave & 1;
   const int halo = (TAPS - 1) * a.d, rows = BM + halo, units = rows * 4;
-  // Few column blocks: each XCD (workgroup id % 8) takes a contiguous range of row-major block
-  // tiles, so that its L2 reads only its own X rows, once for all column blocks.
-  int mb = blockIdx.y, nb = blockIdx.x;
-  if (gridDim.x <= 8) {
-    const int total = gridDim.x * gridDim.y, L = blockIdx.y * gridDim.x + blockIdx.x;
-    const int xcd = L % 8, local = L / 8, C = (total + 7) / 8, r = total % 8;
-    const int t = (r == 0 || xcd < r) ? xcd * C + local : r * C + (xcd - r) * (C - 1) + local;
-    mb = t / gridDim.x;
-    nb = t % gridDim.x;
-  }
+  int mb, nb;
+  block_tile(UNIT ? 1 : a.N / BW, mb, nb);
   const int m0 = mb * BM;
   const int nch = a.C / 32, nsplit = gridDim.z, z = blockIdx.z;
   const int c0 = (int)((int64_t)nch * z / nsplit), c1 = (int)((int64_t)nch * (z + 1) / nsplit);
@@ -299,10 +291,10 @@ void conv_launch(const CodecConvArgs &a, dim3 grid, hipStream_t s) {
 
 template <int TAPS, bool SIN, bool SOUT>
 hipError_t conv_shape(const CodecConvArgs &a, hipStream_t s) {
-  const int bw = a.N % 192 == 0 ? 192 : 96, nbx = a.N / bw;
-  dim3 grid(nbx, (a.T + kConvRows - 1) / kConvRows);
+  const int bw = a.N % 192 == 0 ? 192 : 96;
+  dim3 grid(a.N / bw * ((a.T + kConvRows - 1) / kConvRows));
   // channel splits: towards 256 workgroups, at least two chunks each, within the workspace
-  const int blocks = (int)(grid.x * grid.y), nch = a.C / 32;
+  const int blocks = (int)grid.x, nch = a.C / 32;
   int sp = 1;
   if (a.split_ws && blocks < 192) {
     sp = std::max(1, std::min((256 + blocks - 1) / blocks, nch / 2));
@@ -322,7 +314,7 @@ hipError_t conv_shape(const CodecConvArgs &a, hipStream_t s) {
 template <int BM, int BW>
 hipError_t unit_launch(const CodecConvArgs &a, hipStream_t s) {
   const size_t stage = (size_t)2 * 3 * (BM + 6 * a.d) * 64, mid = (size_t)3 * BM * BW * 2;
-  const dim3 grid(1, (a.T + BM - 1) / BM);
+  const dim3 grid((a.T + BM - 1) / BM);
   if (a.ra)
     hipLaunchKernelGGL((k_codec_conv<7, BM, BW, true, true, true, true>), grid, dim3(256), std::max(stage, mid), s, a);
   else

@@ -118,16 +118,8 @@ __global__ __launch_bounds__(256 * KG, 2) void k_gemm_tile(GemmArgs a, int vec) 
   float *rinv = reinterpret_cast<float *>(lds + KG * 2 * BUF);
   f32x4_t *image = reinterpret_cast<f32x4_t *>(rinv + BM) + tid;  // [part - half][RT * CT][256]
 
-  // Few column blocks: each XCD (workgroup id % 8) takes a contiguous range of row-major block
-  // tiles, so that its L2 reads only its own X rows, once for all column blocks.
-  int mb = blockIdx.y, nb = blockIdx.x;
-  if (gridDim.x <= 8) {
-    const int total = gridDim.x * gridDim.y, L = blockIdx.y * gridDim.x + blockIdx.x;
-    const int xcd = L % 8, local = L / 8, C = (total + 7) / 8, r = total % 8;
-    const int t = (r == 0 || xcd < r) ? xcd * C + local : r * C + (xcd - r) * (C - 1) + local;
-    mb = t / gridDim.x;
-    nb = t % gridDim.x;
-  }
+  int mb, nb;
+  block_tile((a.N + (SW ? BW / 2 : BW) - 1) / (SW ? BW / 2 : BW), mb, nb);
   const int m0 = mb * BM;
   const int n0 = nb * (SW ? BW / 2 : BW) + wave * OT * 16;  // this wave's first output column
   // k steps [s0, s1) of 32 for this group, parts [part, ..), worked on in pairs of 64-wide chunks (four
@@ -553,7 +545,7 @@ hipError_t rows_launch(const GemmArgs &a, hipStream_t s) {
 template <int EPI, bool NORM, int KG, int CT, bool TAIL, bool PARTS>
 hipError_t tile_launch(const GemmArgs &a, hipStream_t s) {
   const int out = EPI == EPI_SWIGLU ? 64 : 64 * CT;
-  const dim3 grid((a.N + out - 1) / out, (a.M + 31) / 32);
+  const dim3 grid((unsigned)((a.N + out - 1) / out * (int64_t)((a.M + 31) / 32)));
   const size_t lds = (size_t)KG * 2 * 3 * 2 * 32 * 64 + 32 * 4 + (KG > 1 ? (size_t)(a.k_parts / 2) * CT * 8192 : 0);
   hipLaunchKernelGGL((k_gemm_tile<EPI, NORM, KG, CT, TAIL, PARTS>), grid, dim3(256 * KG), lds, s, a, gemm_vec(a));
   return hipGetLastError();

@@ -56,6 +56,40 @@ def test_decode_at_block_edges(codec_case, frames):
     assert err <= 1.4e-5
 
 
+def test_decode_of_thousands_of_frames(codec_case, monkeypatch):
+    """2,200 frames: the 96-channel units' 64-row blocks pass 65,535 in the 2,185th.  The last 12 frames
+    against the oracle, whose convolutions run over the last 40 only: they and the upsampling stages
+    look back less than 11 frames.  The bound is test_decode_at_block_edges's."""
+    eng, oracle = codec_case
+
+    def attention(q, k, v):  # causal_attention by heads, on BLAS
+        mask = np.triu(np.ones((len(q), len(q)), dtype=bool), 1)
+        out = np.empty_like(q)
+        for h in range(q.shape[1]):
+            s = np.ascontiguousarray(q[:, h]) @ np.ascontiguousarray(k[:, h].T) / np.sqrt(q.shape[2])
+            s[mask] = -np.inf
+            s = np.exp(s - s.max(axis=1, keepdims=True))
+            out[:, h] = s @ np.ascontiguousarray(v[:, h]) / s.sum(axis=1, keepdims=True)
+        return out
+
+    rng = np.random.default_rng(2200)
+    q, k, v = rng.standard_normal((3, 9, 2, 64))
+    np.testing.assert_allclose(attention(q, k, v), C.causal_attention(q, k, v), rtol=1e-12, atol=1e-14)
+    monkeypatch.setattr(C, "causal_attention", attention)
+    codes = rng.integers(0, 2048, (2200, 16)).astype(np.int32)
+    print("[gpu] decode_codes frames=2200", flush=True)
+    got = eng.decode_codes(codes)
+    assert got.shape == (2200 * C.SAMPLES_PER_FRAME,)
+    t = oracle.t
+    x = C.causal_conv(oracle.rvq(codes), t["decoder.pre_conv.conv.weight"], t["decoder.pre_conv.conv.bias"])
+    x = oracle.pre_transformer(x)[-40:]
+    ref = np.clip(oracle.decoder(oracle.upsample(oracle.upsample(x, 0), 1)), -1.0, 1.0)
+    n = 12 * C.SAMPLES_PER_FRAME
+    err = float(np.linalg.norm(got[-n:] - ref[-n:]) / np.linalg.norm(ref[-n:]))
+    print(f"decode 2200 frames, last 12: rel err {err:.2e}")
+    assert err <= 1.4e-5
+
+
 def test_snake_of_large_arguments(models, tmp_path):
     """Snakes whose arguments pass the fast sine's range (alpha = e^12: |x e^12| above 65536)
     in input, output and residual position, beside ones that do not: finite and near float64.
