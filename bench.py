@@ -529,7 +529,7 @@ def main() -> int:
     text_prep = None
     if with_text:
         # Prompt preparation of the same prompt on the device (q3t_prepare_text, host copies
-        # and workspace allocation included), against the package's numpy preparation.
+        # included; its workspace is kept between calls), against the package's numpy preparation.
         ids = w.prompt()
         dev = eng.prepare_text(ids, text_lookahead_tokens=look)
         assert np.abs(dev.prefill - inputs.prefill).max() < 1e-4

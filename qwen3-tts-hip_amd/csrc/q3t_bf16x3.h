@@ -156,11 +156,10 @@ __device__ __forceinline__ float snake_any(float v, float y, float ib) {
 }
 
 // Snake of N values in place (any magnitude): the library sine only where some |y| is past the
-// fast form's range (or not a number).
+// fast form's range.  A NaN goes through either form as a NaN.
 template <int N>
 __device__ __forceinline__ void snake_n(float *v, const float *ea, const float *ib) {
   float big = 0.f;
-  bool bad = false;
   float x[N];
 #pragma unroll
   for (int i = 0; i < N; ++i) {
@@ -168,8 +167,7 @@ __device__ __forceinline__ void snake_n(float *v, const float *ea, const float *
     big = fmaxf(big, fabsf(y));
     x[i] = snake_fast(v[i], y, ib[i]);
   }
-  bad = !(big < kSnakeFast);
-  if (__builtin_expect(bad, 0)) {
+  if (__builtin_expect(!(big < kSnakeFast), 0)) {
 #pragma unroll
     for (int i = 0; i < N; ++i) x[i] = snake_any(v[i], v[i] * ea[i], ib[i]);
   }

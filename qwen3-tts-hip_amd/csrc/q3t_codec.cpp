@@ -30,7 +30,8 @@ namespace {
 
 constexpr int kGroups = 16, kCodebook = 2048, kCodebookDim = 256, kProjected = 512, kPreConv = 1024;
 constexpr int kHidden = 512, kLayers = 8, kHeads = 16, kQ = kHeads * 64, kInter = 1024;
-constexpr int kUp = 1024, kConvNext = 4096, kInit = 1536, kFinal = 96, kPad = 64;
+constexpr int kUp = 1024, kConvNext = 4096, kInit = 1536, kFinal = 96;
+constexpr int kPad = 2;  // zero rows before time 0 of the pre-conv's input (3 taps)
 constexpr float kRmsEps = 1e-5f, kLnEps = 1e-6f;
 struct BlockShape {
   int ci, co, s;
@@ -368,7 +369,7 @@ void codec_decode(Codec &c, const int32_t *codes, int F, int groups, float *samp
   float *Q = Qp + (size_t)kPad * kProjected;
   gemm(EPI_STORE, E, 2 * kCodebookDim, F, c.w_rvq, kProjected, 2 * kCodebookDim, Q, kProjected, nullptr);
   float *PC = take((size_t)F * kPreConv);
-  gemm(EPI_BIAS, Qp + (size_t)(kPad - 2) * kProjected, kProjected, F, c.pre_w, kPreConv, 3 * kProjected, PC, kPreConv,
+  gemm(EPI_BIAS, Qp, kProjected, F, c.pre_w, kPreConv, 3 * kProjected, PC, kPreConv,
        c.pre_b);
 
   // 3. pre-transformer

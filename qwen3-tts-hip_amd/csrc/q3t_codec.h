@@ -44,7 +44,7 @@ struct CodecConvArgs {
   const float *bias;      // [N]
   const float *oa, *ob;   // output Snake tables [N], or null
   float *Y;               // [T][N], not X
-  int32_t N;              // a multiple of 96
+  int32_t N;              // a multiple of 96 (7 taps without w2: of 192)
   float *split_ws;        // channel splits of short inputs: [split][T][N] raw sums, or null
   int64_t split_cap;      // floats in split_ws
   // A whole residual unit (7 taps, both Snakes, C = N, codec_unit_ok): the Snaked output goes on

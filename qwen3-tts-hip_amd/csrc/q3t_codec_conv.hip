@@ -20,7 +20,8 @@
 //     waves of a column half read the same lines.
 //   * Four waves as 2 x 2: BM / 2 rows by BW / 2 columns each.  The weight tile is the A operand,
 //     so a lane ends with four consecutive columns of one row: 16-byte bias loads and stores.
-//   * BW = 192 where N allows it (every layer but N = 96, 288), else 96: all N are exact multiples.
+//   * BW = 192, but 96 for the units of 96 channels and the transposed convolution of N = 288: all N are
+//     exact multiples.
 //   * BM = 64 (45 KB of LDS at dilation 9: up to three blocks a CU).  128-row blocks measured the
 //     same on long inputs and leave CUs idle on short ones; residual units, which nothing splits,
 //     take BM = 32 when short.  A launch of few blocks splits the
@@ -292,6 +293,7 @@ void conv_launch(const CodecConvArgs &a, dim3 grid, hipStream_t s) {
 template <int TAPS, bool SIN, bool SOUT>
 hipError_t conv_shape(const CodecConvArgs &a, hipStream_t s) {
   const int bw = a.N % 192 == 0 ? 192 : 96;
+  if (TAPS > 2 && bw == 96) return hipErrorInvalidValue;
   dim3 grid(a.N / bw * ((a.T + kConvRows - 1) / kConvRows));
   // channel splits: towards 256 workgroups, at least two chunks each, within the workspace
   const int blocks = (int)grid.x, nch = a.C / 32;
@@ -301,8 +303,12 @@ hipError_t conv_shape(const CodecConvArgs &a, hipStream_t s) {
     while (sp > 1 && (int64_t)sp * a.T * a.N > a.split_cap) --sp;
   }
   grid.z = sp;
-  if (bw == 192) conv_launch<TAPS, kConvRows, 192, SIN, SOUT>(a, grid, s);
-  else conv_launch<TAPS, kConvRows, 96, SIN, SOUT>(a, grid, s);
+  if constexpr (TAPS == 2) {
+    if (bw == 192) conv_launch<TAPS, kConvRows, 192, SIN, SOUT>(a, grid, s);
+    else conv_launch<TAPS, kConvRows, 96, SIN, SOUT>(a, grid, s);
+  } else {
+    conv_launch<TAPS, kConvRows, 192, SIN, SOUT>(a, grid, s);
+  }
   if (sp > 1) {
     const size_t n = (size_t)a.T * a.N / 4;
     hipLaunchKernelGGL((k_codec_conv_reduce<SOUT>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a, sp);

@@ -1,8 +1,8 @@
 """Codec decoder on the GPU (q3t_decode_codes, q3t_stream_next_audio) against the float64 CPU
 oracle of the reference's decoder (oracle/codec.py), on the synthetic speech-tokenizer
-checkpoint.  Frame counts 3 and 10 put the decoder stages on both matrix-core GEMM paths
-(fewer and more than 128 rows); 70 frames take the pre-transformer attention past one pass of
-its four waves' 32-key stride and its 64-key softmax loop."""
+checkpoint.  Frame counts 3 and 10 put its linears and 1x1 convolutions on both matrix-core GEMM
+kernels (few and many rows); at 70 frames a query block of the pre-transformer attention has five
+16-key tiles, so that one of its four waves works on two."""
 import numpy as np
 import pytest
 

@@ -68,11 +68,10 @@ def test_epilogues_and_norm(eng):
 
 @pytest.mark.parametrize("N", [96, 192])
 def test_epilogues_96_column_blocks(eng, N):
-    """M >= 128 with N a multiple of 96 but not of 128 (the codec's 96- and 192-channel
-    convolutions) runs the LDS-tiled kernel in 96-column blocks: bias, and residual with the
-    RMSNorm prologue."""
+    """N a multiple of 96 but not of 128, from 128 rows on: the tiled kernel's last block of 128 columns is
+    partial (K parts are counted in blocks of 96 there): bias, and residual with the RMSNorm prologue."""
     M, K = 200, 672
-    print(f"[gpu] gemm 96-column blocks M={M} N={N} K={K}", flush=True)
+    print(f"[gpu] gemm N a multiple of 96 M={M} N={N} K={K}", flush=True)
     rng = np.random.default_rng(N)
     X = (rng.standard_normal((M, K)) * 2).astype(np.float32)
     g = (1 + 0.1 * rng.standard_normal(K)).astype(np.float32)
@@ -132,7 +131,7 @@ def test_rejects_bad_shapes(eng):
 
 @pytest.mark.parametrize("M,K", [(128, 1024), (300, 2048), (521, 1024)])
 def test_prefill_tiles_all_epilogues(eng, M, K):
-    """M >= 128 with K % 64 == 0 runs the LDS-tiled prefill kernel: RMSNorm rows (1/rms and
+    """The tiled prefill kernel over whole pairs of 64-wide chunks: RMSNorm rows (1/rms and
     gain applied on the way into LDS), store / residual / SwiGLU / bias epilogues."""
     print(f"[gpu] gemm tiles M={M} K={K}", flush=True)
     N = 256
@@ -154,9 +153,9 @@ def test_prefill_tiles_all_epilogues(eng, M, K):
 @pytest.mark.parametrize("M", [1, 16, 17, 32, 33, 48, 49, 64, 65, 128, 129, 193])
 @pytest.mark.parametrize("K", [32, 96, 160, 1056])
 def test_row_and_step_remainders(eng, M, K):
-    """Rows around the 16-row tiles of the few-row kernel (up to 64) and the 32-row blocks of the
-    tiled one, k steps that do not fill a wave's share, a chunk or a pair of chunks, and a partial
-    last column tile: residual with RMSNorm, bias, SwiGLU.  The tolerance is the module's."""
+    """Rows around the 16-row tile of the few-row kernel (one tile here, in one K part) and the 32-row
+    blocks of the tiled one, k steps that do not fill a wave's round, a chunk or a pair of chunks, and a
+    partial last column tile: residual with RMSNorm, bias, SwiGLU.  The tolerance is the module's."""
     N = 84
     rng = np.random.default_rng(M * 5 + K)
     X = (rng.standard_normal((M, K)) * 2).astype(np.float32)
@@ -175,8 +174,7 @@ def test_row_and_step_remainders(eng, M, K):
 
 @pytest.mark.parametrize("M,N,K", [(70, 8192, 512), (200, 4100, 512), (520, 2050, 256)])
 def test_wide_tiles(eng, M, N, K):
-    """Enough 128-column blocks for every CU (one K group a block),
-    N not a multiple of 4 among them."""
+    """Many 128-column blocks, N not a multiple of 4 among them."""
     print(f"[gpu] gemm wide M={M} N={N} K={K}", flush=True)
     rng = np.random.default_rng(M)
     X = rng.standard_normal((M, K)).astype(np.float32)

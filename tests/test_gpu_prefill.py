@@ -1,5 +1,5 @@
 """Talker prompt prefill at prompt lengths around the attention's 16-row query blocks and
-16-key tiles (1, 2, 15, 16, 17, 33, and past the 128-row tiles of the prefill GEMM up to
+16-key tiles (1, 2, 15, 16, 17, 33, 130 and
 cap - 1), through the q3t_debug_talker_prefill hook, against the float64 oracle's prefill
 (decode.rs:1077-1298).  Both query-head groupings (two query heads per KV head and one) and
 both KV cache types (the oracle rounds K and V to bf16 where the GPU stores bf16)."""
@@ -44,8 +44,8 @@ def test_prefill_lengths_match_oracle(models, spec, kv_bf16):
 
 @pytest.mark.parametrize("kv_bf16", [False, True])
 def test_prefill_tiles_per_wave(models, kv_bf16):
-    """Lengths at which the attention's four waves (every fourth 16-key tile each) gain a tile, or
-    one of them does: 48 / 49 and 63 .. 65 rows (three, four and five tiles), 80 / 81 and 128 / 129."""
+    """Lengths around the attention's rounds of four 16-key tiles, one scored by each of its waves: 48 / 49
+    and 63 .. 65 rows (three, four and five tiles), 80 / 81 and 128 / 129."""
     model, d = models.get("tiny", 0)
     rng = np.random.default_rng(12)
     print(f"[gpu] prefill tiles per wave kv_bf16={kv_bf16}", flush=True)
@@ -62,9 +62,8 @@ def test_prefill_tiles_per_wave(models, kv_bf16):
 
 
 def test_prefill_split_sums_leave_no_trace(models):
-    """Prompts of few rows accumulate the O and down projections into buffers that each GEMM leaves
-    zeroed for the next: the same prompt before and after others, on both sides of the 64 rows from
-    which the tiled kernel does it, gives the same bits."""
+    """The O and down projections add onto the rows that they read as the residual, in K parts: the same
+    prompt before and after others, through either GEMM kernel, gives the same bits."""
     model, d = models.get("tiny", 0)
     rng = np.random.default_rng(13)
     xs = [(rng.standard_normal((P, model.spec.talker.hidden)) * 0.5).astype(np.float32) for P in (41, 64, 65, 3, 130)]
@@ -80,8 +79,8 @@ def test_prefill_split_sums_leave_no_trace(models):
 
 @pytest.mark.parametrize("P", [65, 96, 97, 1023, 1024, 1025])
 def test_prefill_tiled_split_sums(models, P):
-    """O and down of 65 rows on in 32-row tiles: K halves up to 1,024 rows at hidden 512, whole sums
-    beyond; whole and partial last tiles, the same bits when run again."""
+    """O and down in 32-row tiles at hidden 512: K parts in two groups of waves a block, of 64 and of 128
+    columns; whole and partial last tiles, the same bits when run again."""
     model, d = models.get("tiny", 0)
     x = (np.random.default_rng(P).standard_normal((P, model.spec.talker.hidden)) * 0.5).astype(np.float32)
     print(f"[gpu] prefill tiled split sums P={P}", flush=True)

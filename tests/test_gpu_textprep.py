@@ -1,7 +1,7 @@
 """Device prompt preparation (q3t_prepare_text / q3t_stream_start_text) against the CPU
 oracle of text.rs:340-382 / 516-603 (oracle/textprep.py), on the tiny model written with its
-full text-embedding table.  Prompts of 4..150 content ids cover both GEMM paths of the text
-projection (fewer and more than 128 rows)."""
+full text-embedding table.  Prompts of 4..150 content ids cover both GEMM kernels of the text
+projection (few and many rows)."""
 import numpy as np
 import pytest
 
@@ -48,7 +48,7 @@ def test_prepare_text_matches_oracle(tiny_text, n, look, speaker, language):
 
 def test_prepare_text_sizes_in_turn(tiny_text):
     """One engine over prompts that grow, shrink and pass the kept memory's limit: 64 and 65 rows (11
-    more than the ids; the two sides of the few-row GEMM) and 3011, with nothing left of the call
+    more than the ids) and 3011, with nothing left of the call
     before.  The bound is the other tests'; results handed out earlier stay as they were."""
     model, oracle, eng = tiny_text
     kept = []
